@@ -37,6 +37,7 @@ void ensure_runtime() {
         if (status == hipSuccess) status = init_f32z_attributes();
         if (status == hipSuccess) status = init_f64_attributes();
         if (status == hipSuccess) status = init_appr_attributes();
+        if (status == hipSuccess) status = init_live_attributes();
     });
     BNMF_HIP(status);
 }
@@ -226,18 +227,28 @@ BldInst make_desc(const InstLayout& L, void* base, double eps, double a, double 
     return d;
 }
 
-PassKey pass_key(int dtype, int mode, const InstLayout& L, bool nonneg) {
-    // BNMF_PASS_GENERIC=1 routes the FP32 steps through the generic z-bucket
-    // kernel, for comparisons. Its update is the same formula evaluated in
-    // another order (the exact-z kernel folds X_reciprocal and X / S_ij+
-    // into per-fiber constants), so the two agree to FP32 rounding, not
-    // bit for bit.
+// BNMF_PASS_GENERIC=1 routes the FP32 steps through the generic z-bucket
+// kernel, for comparisons. Its update is the same formula evaluated in
+// another order (the exact-z kernel folds X_reciprocal and X / S_ij+
+// into per-fiber constants), so the two agree to FP32 rounding, not
+// bit for bit.
+static bool generic_steps() {
     static const bool generic = [] {
         const char* e = std::getenv("BNMF_PASS_GENERIC");
         return e != nullptr && e[0] == '1';
     }();
+    return generic;
+}
+
+PassKey pass_key(int dtype, int mode, const InstLayout& L, bool nonneg, bool live) {
+    const bool generic = generic_steps();
     PassKey k;
     if (L.z > kFusedZ) return k;  // the wide pass (zexact = zb = 0)
+    if (live && (mode == MODE_UPDATE || mode == MODE_ADD)) {
+        k.live = dtype == BNMF_F32 ? (int)(L.z + 3) / 4 : (int)(kTileCols / L.tile_cols * 4u + L.rw);
+        k.f64 = dtype == BNMF_F64;
+        return k;
+    }
     if (dtype == BNMF_F64 && (mode == MODE_UPDATE || mode == MODE_ADD)) {
         k.f64 = 1;
         k.zb = (int)L.zb;
@@ -266,6 +277,23 @@ hipError_t launch_pass_key(const PassKey& k, int dtype, int psi, int mode, dim3 
         return launch_pass_f32z(k.zexact, mode, grid, st, insts, items, n_items);
     }
     return launch_pass(dtype, psi, mode, k.zb, k.rw, grid, st, insts, items, n_items, zmax);
+}
+
+// *nonneg: every S0 element is >= 0; *packable also: none above 1e30, and
+// zero throughout the fibers with X = 0.
+template <typename T>
+static void scan_S0(const T* S0, const T* X, size_t xy, size_t z, bool* nonneg, bool* packable) {
+    bool nn = true, pk = *packable;
+    for (size_t f = 0; f < xy && nn; ++f) {
+        const T most = X[f] == T(0) ? T(0) : T(1e30);
+        for (size_t k = 0; k < z; ++k) {
+            const T v = S0[f * z + k];
+            nn = nn && v >= T(0);
+            pk = pk && v <= most;
+        }
+    }
+    *nonneg = nn;
+    *packable = nn && pk;
 }
 
 // ------------------------------------------------------------------ batch
@@ -302,13 +330,18 @@ Batch::Batch(int dtype, int psi_mode, double eps, const std::vector<InstSpec>& s
         base_off[n] = total;
         total += layouts_.back().bytes;
     }
+    const size_t off_scratch = total;
+    total += LivePlan::scratch_bytes(layouts_);
     arena_ = DeviceBuffer(std::max<size_t>(total, kAlign));
     device_bytes_ = arena_.bytes;
 
     // uploads (X, alpha, beta, S0 or its device draw). nonneg[n]: S0 >= 0
     // and every beta_k >= 1, so grad_plus >= 0 and S stays nonnegative (the
     // kernels then skip the psi(S+1) guard for S < 0).
-    std::vector<bool> nonneg(specs.size(), false);
+    // packable[n]: besides, every S0 element is finite and zero where X is
+    // zero, every alpha_i is positive and eps leaves 1 / eps finite, so a
+    // fiber with X_ij = 0 stays exactly zero (LivePlan).
+    std::vector<bool> nonneg(specs.size(), false), packable(specs.size(), false);
     for (size_t n = 0; n < specs.size(); ++n) {
         const InstSpec& s = specs[n];
         const InstLayout& L = layouts_[n];
@@ -321,16 +354,18 @@ Batch::Batch(int dtype, int psi_mode, double eps, const std::vector<InstSpec>& s
         const void* S0 = s.S0;
         bool nn = true;
         for (uint32_t k = 0; k < s.z; ++k) nn = nn && s.beta[k] >= 1.0;
+        bool pk = nn && s.z <= kFusedZ && !(dtype == BNMF_F32 && generic_steps()) && eps >= 1e-200 && eps <= 1.0 &&
+                  LivePlan::worth(dtype, s.X, xy);
+        for (uint32_t i = 0; i < s.x; ++i) pk = pk && s.alpha[i] >= 1e-6 && s.alpha[i] <= 1e30;
+        for (uint32_t k = 0; k < s.z; ++k) pk = pk && s.beta[k] <= 1e30;
         if (nn && s.S0) {
-            if (dtype == BNMF_F32) {
-                const float* p = static_cast<const float*>(S0);
-                for (size_t t = 0; t < xyz && nn; ++t) nn = p[t] >= 0.0f;
-            } else {
-                const double* p = static_cast<const double*>(S0);
-                for (size_t t = 0; t < xyz && nn; ++t) nn = p[t] >= 0.0;
-            }
+            if (dtype == BNMF_F32)
+                scan_S0(static_cast<const float*>(S0), static_cast<const float*>(s.X), xy, s.z, &nn, &pk);
+            else
+                scan_S0(static_cast<const double*>(S0), static_cast<const double*>(s.X), xy, s.z, &nn, &pk);
         }
         nonneg[n] = nn;
+        packable[n] = nn && pk;
         if (S0) {
             BNMF_HIP(hipMemcpy(b + L.off_S0, S0, xyz * es_, hipMemcpyHostToDevice));
         } else {
@@ -345,12 +380,18 @@ Batch::Batch(int dtype, int psi_mode, double eps, const std::vector<InstSpec>& s
     // descriptors and work lists of the whole batch (the sums-only and
     // scoring passes, bld_fact, tensor_sums)
     std::vector<BldInst> d_first, d_main;
-    std::vector<PrepItem> prep;
     for (size_t n = 0; n < specs.size(); ++n) {
         const InstLayout& L = layouts_[n];
         char* b = arena_.as<char>(base_off[n]);
         d_first.push_back(make_desc(L, b, eps, specs[n].a, specs[n].b, true, nonneg[n]));
         d_main.push_back(make_desc(L, b, eps, specs[n].a, specs[n].b, false, nonneg[n]));
+    }
+    // the instances whose nonempty fibers are kept packed
+    live_ = LivePlan(dtype, d_main, layouts_, packable, arena_.as<char>(off_scratch));
+    device_bytes_ += live_.bytes();
+    std::vector<PrepItem> prep;
+    for (size_t n = 0; n < specs.size(); ++n) {
+        const InstLayout& L = layouts_[n];
         if (L.elements() == 0) continue;
         for (uint32_t c = 0; c < L.n_cj; ++c) prep.push_back(PrepItem{(uint32_t)n, 0, c, 0});
         for (uint32_t c = 0; c < L.nA; ++c) prep.push_back(PrepItem{(uint32_t)n, 1, c, 0});
@@ -365,7 +406,7 @@ Batch::Batch(int dtype, int psi_mode, double eps, const std::vector<InstSpec>& s
         auto& v = sum_items[pass_key(dtype, MODE_SUMS, L, nonneg[n])];
         for (uint32_t ti = 0; ti < L.n_ti; ++ti)
             for (uint32_t tj = 0; tj < L.n_tj; ++tj) v.push_back(PassItem{(uint32_t)n, ti, tj, 0});
-        members[pass_key(dtype, step_mode_, L, nonneg[n])].push_back((uint32_t)n);
+        members[pass_key(dtype, step_mode_, L, nonneg[n], live_.live(n))].push_back((uint32_t)n);
     }
     auto tile_work = [&](const InstLayout& L, uint32_t ti, uint32_t tj) {
         const uint32_t rows = std::min(L.ti_rows, L.x - ti * L.ti_rows);
@@ -394,6 +435,10 @@ Batch::Batch(int dtype, int psi_mode, double eps, const std::vector<InstSpec>& s
         for (uint32_t n : kv.second) {
             bk.work += layouts_[n].elements();
             bk.zmax = std::max(bk.zmax, layouts_[n].z);
+            if (bk.key.live) {
+                bk.lds = std::max(bk.lds, live_.lds(n));
+                bk.most = std::max(bk.most, live_.most(n));
+            }
         }
         bk.lane = 0;
         groups_[0].push_back(bk);
@@ -436,10 +481,12 @@ Batch::Batch(int dtype, int psi_mode, double eps, const std::vector<InstSpec>& s
                 lm.push_back(n);
                 const InstLayout& L = layouts_[n];
                 for (uint32_t ti = 0; ti < L.n_ti; ++ti)
-                    for (uint32_t tj = 0; tj < L.n_tj; ++tj) upd_items[gi].push_back(PassItem{local, ti, tj, 0});
+                    for (uint32_t tj = 0; tj < L.n_tj; ++tj)
+                        upd_items[gi].push_back(PassItem{bk.key.live ? n : local, ti, tj, 0});
             }
             bk.n_items = (uint32_t)upd_items[gi].size();
             xcd_order(upd_items[gi]);
+            if (bk.key.live) bk.tile0 = live_.add_launch(upd_items[gi], d_main);
             ++gi;
         }
     }
@@ -520,6 +567,7 @@ Batch::Batch(int dtype, int psi_mode, double eps, const std::vector<InstSpec>& s
         BNMF_HIP(hipMemcpy(m + ln.off_prep_count, &ln.n_prep, sizeof(uint32_t), hipMemcpyHostToDevice));
     }
     BNMF_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
+    live_.build(d_main, reinterpret_cast<const BldInst*>(m + off_desc_), stream_);
     if (ns > 1) {
         side_.resize(ns);
         fork_ev_.resize(ns);
@@ -571,6 +619,12 @@ void Batch::enqueue_pass(int mode, bool first) {
     }
 }
 
+void Batch::pack_S(bool first) {
+    live_.gather(reinterpret_cast<const BldInst*>(meta_.as<char>() + (first ? off_desc_first_ : off_desc_)), stream_);
+}
+
+void Batch::unpack_S() { live_.scatter(reinterpret_cast<const BldInst*>(meta_.as<char>() + off_desc_), stream_); }
+
 void Batch::enqueue_iterations(int iters, bool first, bool with_prep) {
     if (n_prep_items_ == 0 || iters <= 0) return;
     char* m = meta_.as<char>();
@@ -597,6 +651,11 @@ void Batch::enqueue_iterations(int iters, bool first, bool with_prep) {
                 reinterpret_cast<const BldInst*>(m + ((first && t == 0) ? ln.off_desc_first : ln.off_desc));
             for (const Bucket& bk : groups_[0]) {
                 if ((size_t)bk.lane != l) continue;
+                if (bk.key.live) {
+                    BNMF_HIP(launch_pass_live(dtype_, psi_, step_mode_, bk.key.live, bk.n_items, st,
+                                              live_.tiles() + bk.tile0, bk.most, bk.lds));
+                    continue;
+                }
                 BNMF_HIP(launch_pass_key(bk.key, dtype_, psi_, step_mode_, dim3(bk.n_items), st, dp,
                                          reinterpret_cast<const PassItem*>(m + bk.off_items),
                                          reinterpret_cast<const uint32_t*>(m + bk.off_count), bk.zmax));
@@ -645,6 +704,7 @@ void Batch::solve_async(size_t iters) {
     }
     start_solve();
     replay_iterations(iters - 1);
+    unpack_S();
     partials_valid_ = true;
 }
 
@@ -655,6 +715,7 @@ void Batch::start_solve() {
         BNMF_HIP(hipMemsetAsync(meta_.as<char>() + off_iter_, 0, specs_.size() * sizeof(uint32_t), stream_));
     // partial axis sums of S0, then the first iteration reading S0
     enqueue_pass(MODE_SUMS, true);
+    pack_S(true);
     enqueue_iteration(true);
 }
 
@@ -697,6 +758,7 @@ size_t Batch::solve_tol(size_t max_iter, double tol, size_t check_every, double*
             enqueue_pass(MODE_SUMS, false);
             replay_iterations(chunk);
         }
+        unpack_S();
         done += chunk;
         scored = false;
         if (done >= max_iter) break;
@@ -794,6 +856,8 @@ void Batch::time_pass(int reps, double* pass_ms, double* iter_ms) {
         BNMF_HIP(hipEventCreate(&e0));
         BNMF_HIP(hipEventCreate(&e1));
         BNMF_HIP(hipEventCreate(&e2));
+        enqueue_pass(MODE_SUMS, false);
+        pack_S(false);
         BNMF_HIP(hipGraphLaunch(gp, stream_));
         BNMF_HIP(hipGraphLaunch(gi, stream_));
         BNMF_HIP(hipEventRecord(e0, stream_));
@@ -801,6 +865,7 @@ void Batch::time_pass(int reps, double* pass_ms, double* iter_ms) {
         BNMF_HIP(hipEventRecord(e1, stream_));
         BNMF_HIP(hipGraphLaunch(gi, stream_));
         BNMF_HIP(hipEventRecord(e2, stream_));
+        unpack_S();
         BNMF_HIP(hipEventSynchronize(e2));
         float tp = 0.f, ti = 0.f;
         BNMF_HIP(hipEventElapsedTime(&tp, e0, e1));

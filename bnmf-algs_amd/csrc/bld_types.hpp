@@ -72,6 +72,59 @@ struct BldInst {
     uint32_t nonneg;      // 1: S0 >= 0 and beta >= 1, so S stays >= 0 (fast psi(S+1))
 };
 
+// Live fibers. A fiber whose X_ij is 0 holds zeros from S0 on (S_ijk = X_ij
+// w_k with w on the simplex) and every step writes zeros back: it adds nothing
+// to an axis sum and can be left out of the iteration. An instance with few
+// nonempty fibers keeps those packed, tile by tile, and its step passes run
+// over the packed copy (bld_live.hip). Fibers of a tile are numbered q =
+// 0..n-1 by (column, row mod 4, row): the order in which the dense pass's four
+// wavefronts add them to S_+jk.
+//
+// A nonempty row: its first four fibers in the order in which the dense pass
+// meets them (the zero fiber n past its count), and the shape of their sum:
+// 0 ((a+b)+c)+d, 1 (a+(b+c))+d, 2 (a+b)+(c+d), 3 a+((b+c)+d), 4 a+(b+(c+d)).
+struct LiveRow {
+    uint16_t row, shape;
+    uint16_t q[4];
+    uint32_t pad;
+};
+// A nonempty column: its first fiber, and where its rows of classes 0 to 3
+// (mod 4) end, counted from there.
+struct LiveCol {
+    uint16_t q0, col;
+    uint16_t end[4];
+    uint32_t pad;
+};
+static_assert(sizeof(LiveRow) == 16 && sizeof(LiveCol) == 16, "16-byte table entries");
+// All a block needs to know of its tile, in one read: every further level of
+// indirection costs it a memory latency.
+struct LiveTile {
+    void* Sc;              // packed S of the tile (bld_live.hip: live_index)
+    const uint16_t* fib;   // [q] row in tile << 6 | column in tile
+    const void* xv;        // [q] X_ij
+    const LiveRow* rdesc;  // nonempty rows: those with at most four fibers first
+    const LiveCol* cdesc;  // nonempty columns
+    const uint16_t* map;   // [row * tile_cols + column] fiber number, n where empty
+    const uint16_t* smap;  // its rows with more than four fibers, in rdesc's order
+    const void* psib;      // the workspace of the instance, at the tile's rows or columns
+    const void* psia;
+    const void* psiA;
+    void* part_ipk;
+    void* part_pjk;
+    const uint32_t* iter;
+    double eps;
+    uint32_t inst;           // descriptor of the instance
+    uint32_t ti, tj;
+    uint32_t z, n;           // depth, nonempty fibers
+    uint16_t trows, tcols;   // rows and columns of the tile (x and y may end within it)
+    uint16_t rows4, rows;    // nonempty rows with at most four fibers, all nonempty rows
+    uint16_t cols;           // nonempty columns
+    uint8_t xs, xm;          // FP32 visit order: chunk m is stored at m ^ ((column >> xs) & xm)
+    uint32_t zq_log2;
+    float inv_z;
+};
+constexpr uint32_t kLiveRows = 512;  // tallest tile the packed form takes
+
 struct PassItem {
     uint32_t inst, ti, tj, pad;
 };

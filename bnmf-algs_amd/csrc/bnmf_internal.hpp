@@ -70,6 +70,20 @@ hipError_t launch_pass_wide(int dtype, int psi, int mode, dim3 grid, hipStream_t
 hipError_t launch_pass_f32z(int z, int mode, dim3 grid, hipStream_t st, const BldInst* insts,
                             const PassItem* items, const uint32_t* n_items);
 hipError_t init_f32z_attributes();
+// step passes over the packed nonempty fibers of n tiles (bld_live.hip): ng =
+// ceil(z / 4) (FP32) or 4 * the dense pass's lanes per fiber + its read width
+// (FP64); most: fibers of the fullest tile; lds: dynamic LDS bytes
+hipError_t launch_pass_live(int dtype, int psi, int mode, int ng, uint32_t n, hipStream_t st, const LiveTile* tiles,
+                            uint32_t most, uint32_t lds);
+hipError_t init_live_attributes();
+// LDS of a block whose tile has n fibers, with kc elements of k at once
+size_t live_lds_need(int dtype, uint32_t z, uint32_t tile_cols, uint32_t rows, uint32_t n, uint32_t kc);
+void live_group(int dtype, uint32_t z, uint32_t* elems, uint32_t* fibers);
+hipError_t launch_live_count(int dtype, const BldInst* insts, const PassItem* items, uint32_t n, uint32_t* counts,
+                             hipStream_t st);
+hipError_t launch_live_build(int dtype, const BldInst* insts, LiveTile* tiles, uint32_t n, hipStream_t st);
+hipError_t launch_live_gather(int dtype, const BldInst* insts, const LiveTile* tiles, uint32_t n, hipStream_t st);
+hipError_t launch_live_scatter(int dtype, const BldInst* insts, const LiveTile* tiles, uint32_t n, hipStream_t st);
 // approximate solver (bld_appr.hip): mode 0 sums, 1 nu step, 2 mu step
 hipError_t launch_appr_pass(int dtype, int mode, int zb, dim3 grid, hipStream_t st, const ApprInst* insts,
                             const PassItem* items, const uint32_t* n_items, uint32_t zmax);
@@ -172,19 +186,62 @@ BldInst make_desc(const InstLayout& L, void* base, double eps, double a, double 
 // shape only, so an instance runs the same kernel alone, batched or served.
 struct PassKey {
     int zexact = 0, zb = 0, rw = 0, f64 = 0;
+    int live = 0;  // step over packed nonempty fibers: ceil(z / 4) (FP32), 4 lanes per fiber + read width (FP64)
     bool operator<(const PassKey& o) const {
-        return std::tie(zexact, zb, rw, f64) < std::tie(o.zexact, o.zb, o.rw, o.f64);
+        return std::tie(zexact, zb, rw, f64, live) < std::tie(o.zexact, o.zb, o.rw, o.f64, o.live);
     }
     bool wide() const { return zexact == 0 && zb == 0; }
 };
 // fibers per tile row of an instance: kWideCols for z > kFusedZ, else
 // kTileColsF64 (FP64, z <= 32), half that (FP64, z <= 64) or kTileCols (FP32)
 uint32_t tile_cols_of(int dtype, uint32_t z);
-// nonneg: the instance's S stays >= 0 (S0 >= 0 and beta >= 1)
-PassKey pass_key(int dtype, int mode, const InstLayout& L, bool nonneg);
+// nonneg: the instance's S stays >= 0 (S0 >= 0 and beta >= 1); live: its
+// nonempty fibers are packed (LivePlan)
+PassKey pass_key(int dtype, int mode, const InstLayout& L, bool nonneg, bool live = false);
 hipError_t launch_pass_key(const PassKey& k, int dtype, int psi, int mode, dim3 grid,
                            hipStream_t st, const BldInst* insts, const PassItem* items,
                            const uint32_t* n_items, uint32_t zmax);
+
+// Which instances of a batch keep their nonempty fibers packed, and where
+// (live.cpp). Results do not depend on it.
+class LivePlan {
+   public:
+    // Counts the nonempty fibers of the candidates' tiles (X and the tile
+    // plan from the descriptors) and lays the packed buffers out.
+    // scratch: device memory of scratch_bytes, used until the call returns.
+    LivePlan(int dtype, const std::vector<BldInst>& descs, const std::vector<InstLayout>& lay,
+             const std::vector<bool>& candidate, char* scratch);
+    LivePlan() = default;
+    static size_t scratch_bytes(const std::vector<InstLayout>& lay);
+    // false where X (host, n entries) is plainly too full to be packed
+    static bool worth(int dtype, const void* X, size_t n);
+    bool any() const { return !tiles_.empty(); }
+    bool live(size_t n) const { return n < lds_.size() && lds_[n] > 0; }
+    uint32_t lds(size_t n) const { return lds_[n]; }
+    uint32_t most(size_t n) const { return most_[n]; }  // fibers of its fullest tile
+    size_t bytes() const { return buf_.bytes; }
+    // Appends the tiles of one launch (items: batch instance numbers) to the
+    // tile table and returns the first one's index.
+    uint32_t add_launch(const std::vector<PassItem>& items, const std::vector<BldInst>& descs);
+    // Uploads the tile table and builds the lists; insts: the descriptors on
+    // the device
+    void build(const std::vector<BldInst>& descs, const BldInst* insts, hipStream_t st);
+    const LiveTile* tiles() const { return tab_.as<LiveTile>(); }
+    // packed S from S_src, and S from its packed form
+    void gather(const BldInst* insts, hipStream_t st) const;
+    void scatter(const BldInst* insts, hipStream_t st) const;
+
+   private:
+    struct Off {
+        size_t Sc, fib, xv, rdesc, cdesc, map, smap, tile0;
+    };
+    int dtype_ = 0;
+    DeviceBuffer buf_, tab_;
+    std::vector<Off> offs_;
+    std::vector<uint32_t> lds_, most_;  // lds_ 0: the instance runs the dense passes
+    std::vector<uint32_t> slot_, count_;  // per tile of the live instances: first slot, fibers
+    std::vector<LiveTile> tiles_;
+};
 
 // A fixed set of instances sharing one arena, one stream and one set of
 // captured per-iteration graphs.
@@ -220,7 +277,12 @@ class Batch {
         uint32_t n_items;
         size_t off_items;  // in meta_
         size_t off_count;
+        // live groups: first tile, dynamic LDS, fibers of the fullest tile
+        uint32_t tile0 = 0, lds = 0, most = 0;
     };
+    // S of the packed instances from their packed form, and back
+    void unpack_S();
+    void pack_S(bool first);
     void enqueue_iteration(bool first) { enqueue_iterations(1, first); }
     // first iteration of a solve (step counters reset, S0's partials, the
     // step reading S0), then `rem` more iterations from the captured graphs
@@ -248,6 +310,7 @@ class Batch {
     std::vector<InstSpec> specs_;
     DeviceBuffer arena_;
     DeviceBuffer meta_;  // descriptors, work lists, counts
+    LivePlan live_;
     size_t off_desc_first_ = 0, off_desc_ = 0, off_prep_items_ = 0, off_prep_count_ = 0;
     size_t off_iter_ = 0;  // additive solver: uint32 iteration counters, one per instance
     uint32_t n_prep_items_ = 0;

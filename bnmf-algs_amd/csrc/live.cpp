@@ -1,0 +1,196 @@
+// live.cpp — host side of the packed nonempty fibers (bld_live.hip): which
+// instances take them, and the layout of their lists and packed S.
+
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <vector>
+
+#include "bnmf_internal.hpp"
+
+namespace bnmf {
+
+namespace {
+constexpr size_t kAlign = 256;
+size_t align_up(size_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
+
+// Largest share of nonempty fibers at which an instance is packed. The packed
+// step's cost grows with the share, the dense step's does not; at 28 % (100 x
+// 100 x 17 in double) it takes half the dense step's time.
+constexpr double kLiveMax = 0.5;
+// LDS a block takes when its tile needs it, so that two share a CU; a tile
+// with more fibers does its partial sums over k in parts, and may take up to
+// kLdsMost.
+constexpr size_t kLdsWant = 80 * 1024;
+constexpr size_t kLdsMost = 150 * 1024;
+}  // namespace
+
+size_t LivePlan::scratch_bytes(const std::vector<InstLayout>& lay) {
+    size_t tiles = 0;
+    for (const InstLayout& L : lay) tiles += (size_t)L.n_ti * L.n_tj;
+    return align_up(lay.size() * sizeof(BldInst)) + align_up(tiles * sizeof(PassItem)) + align_up(tiles * 4);
+}
+
+// A matrix whose sampled entries (4096 at most, evenly spaced) are mostly
+// nonzero is not worth the count on the device.
+template <typename T>
+static bool mostly_full(const T* X, size_t n) {
+    const size_t step = std::max<size_t>(1, n / 4096);
+    size_t seen = 0, full = 0;
+    for (size_t t = 0; t < n; t += step) {
+        ++seen;
+        full += X[t] != T(0);
+    }
+    return (double)full > 1.2 * kLiveMax * (double)seen;
+}
+
+bool LivePlan::worth(int dtype, const void* X, size_t n) {
+    return !(dtype == BNMF_F32 ? mostly_full(static_cast<const float*>(X), n)
+                               : mostly_full(static_cast<const double*>(X), n));
+}
+
+LivePlan::LivePlan(int dtype, const std::vector<BldInst>& descs, const std::vector<InstLayout>& lay,
+                   const std::vector<bool>& candidate, char* scratch)
+    : dtype_(dtype), offs_(descs.size()), lds_(descs.size(), 0), most_(descs.size(), 0) {
+    const size_t es = dtype == BNMF_F32 ? 4 : 8;
+    // nonempty fibers of every candidate's tiles
+    std::vector<PassItem> items;
+    for (size_t n = 0; n < descs.size(); ++n) {
+        const InstLayout& L = lay[n];
+        if (!candidate[n] || L.elements() == 0 || L.z > kFusedZ || L.ti_rows > kLiveRows) continue;
+        for (uint32_t ti = 0; ti < L.n_ti; ++ti)
+            for (uint32_t tj = 0; tj < L.n_tj; ++tj) items.push_back(PassItem{(uint32_t)n, ti, tj, 0});
+    }
+    if (items.empty() || items.size() > 0x7fffffffu) return;
+    std::vector<uint32_t> counts(items.size());
+    {
+        char* const it = scratch + align_up(descs.size() * sizeof(BldInst));
+        char* const ct = it + align_up(items.size() * sizeof(PassItem));
+        BNMF_HIP(hipMemcpy(scratch, descs.data(), descs.size() * sizeof(BldInst), hipMemcpyHostToDevice));
+        BNMF_HIP(hipMemcpy(it, items.data(), items.size() * sizeof(PassItem), hipMemcpyHostToDevice));
+        BNMF_HIP(launch_live_count(dtype, reinterpret_cast<const BldInst*>(scratch), reinterpret_cast<const PassItem*>(it),
+                                   (uint32_t)items.size(), reinterpret_cast<uint32_t*>(ct), nullptr));
+        BNMF_HIP(hipMemcpy(counts.data(), ct, items.size() * 4, hipMemcpyDeviceToHost));
+    }
+
+    size_t off = 0;
+    auto take = [&](size_t n) {
+        const size_t o = off;
+        off = align_up(off + n);
+        return o;
+    };
+    for (size_t at = 0; at < items.size();) {
+        const size_t n = items[at].inst;
+        const InstLayout& L = lay[n];
+        const size_t nt = (size_t)L.n_ti * L.n_tj;
+        uint32_t ge = 0, gf = 0;
+        live_group(dtype, L.z, &ge, &gf);
+        uint64_t total = 0, slots = 0;
+        uint32_t most = 0;
+        bool ok = true;
+        std::vector<uint32_t> slot(nt);
+        for (size_t t = 0; t < nt && ok; ++t) {
+            const uint32_t c = counts[at + t];
+            ok = c < 65536u;
+            slot[t] = (uint32_t)slots;
+            total += c;
+            slots += (c + gf - 1) / gf * gf;
+            most = std::max(most, c);
+        }
+        ok = ok && total > 0 && (double)total <= kLiveMax * (double)L.x * (double)L.y && slots < (1ull << 31);
+        if (ok) {
+            const size_t least = live_lds_need(dtype, L.z, L.tile_cols, L.ti_rows, most, 4);
+            const size_t all = live_lds_need(dtype, L.z, L.tile_cols, L.ti_rows, most, (L.z + 3) / 4 * 4);
+            ok = least <= kLdsMost;
+            if (ok) lds_[n] = (uint32_t)std::max(least, std::min(all, kLdsWant));
+        }
+        if (ok) {
+            most_[n] = most;
+            Off& o = offs_[n];
+            o.Sc = take((size_t)(slots / gf) * ge * es);
+            o.fib = take((size_t)slots * 2);
+            o.xv = take((size_t)slots * es);
+            o.rdesc = take(nt * L.ti_rows * sizeof(LiveRow));
+            o.cdesc = take(nt * L.tile_cols * sizeof(LiveCol));
+            o.map = take(nt * L.ti_rows * L.tile_cols * 2);
+            o.smap = take(nt * L.ti_rows * L.tile_cols * 2);
+            o.tile0 = slot_.size();
+            slot_.insert(slot_.end(), slot.begin(), slot.end());
+            count_.insert(count_.end(), counts.begin() + at, counts.begin() + at + nt);
+        }
+        at += nt;
+    }
+    if (slot_.empty()) return;
+    // the packed form is extra memory: without room for it every instance
+    // runs the dense passes, with the same results
+    {
+        void* p = nullptr;
+        if (hipMalloc(&p, off) != hipSuccess) {
+            (void)hipGetLastError();
+            std::fill(lds_.begin(), lds_.end(), 0u);
+            return;
+        }
+        buf_.ptr = p;
+        buf_.bytes = off;
+    }
+    // slots past a tile's fibers are read as zeros
+    BNMF_HIP(hipMemset(buf_.ptr, 0, off));
+}
+
+uint32_t LivePlan::add_launch(const std::vector<PassItem>& items, const std::vector<BldInst>& descs) {
+    const uint32_t first = (uint32_t)tiles_.size();
+    const size_t es = dtype_ == BNMF_F32 ? 4 : 8;
+    for (const PassItem& it : items) {
+        const BldInst& d = descs[it.inst];
+        const Off& o = offs_[it.inst];
+        const size_t tile = (size_t)it.ti * d.n_tj + it.tj, slot = slot_[o.tile0 + tile];
+        const size_t i0 = (size_t)it.ti * d.ti_rows, j0 = (size_t)it.tj * d.tile_cols, z = d.z;
+        uint32_t ge = 0, gf = 0;
+        live_group(dtype_, d.z, &ge, &gf);
+        LiveTile t{};
+        t.Sc = buf_.as<char>(o.Sc + slot / gf * ge * es);
+        t.fib = buf_.as<uint16_t>(o.fib) + slot;
+        t.xv = buf_.as<char>(o.xv + slot * es);
+        t.rdesc = buf_.as<LiveRow>(o.rdesc) + tile * d.ti_rows;
+        t.cdesc = buf_.as<LiveCol>(o.cdesc) + tile * d.tile_cols;
+        t.map = buf_.as<uint16_t>(o.map) + tile * d.ti_rows * d.tile_cols;
+        t.smap = buf_.as<uint16_t>(o.smap) + tile * d.ti_rows * d.tile_cols;
+        t.psib = static_cast<const char*>(d.psib) + j0 * z * es;
+        t.psia = static_cast<const char*>(d.psia) + i0 * z * es;
+        t.psiA = d.psiA;
+        t.part_ipk = static_cast<char*>(d.part_ipk) + ((size_t)it.tj * d.x + i0) * z * es;
+        t.part_pjk = static_cast<char*>(d.part_pjk) + ((size_t)it.ti * d.y + j0) * z * es;
+        t.eps = d.eps;
+        t.inst = it.inst;
+        t.ti = it.ti;
+        t.tj = it.tj;
+        t.z = d.z;
+        t.n = count_[o.tile0 + tile];
+        t.trows = (uint16_t)std::min<size_t>(d.ti_rows, d.x - i0);
+        t.tcols = (uint16_t)std::min<size_t>(d.tile_cols, d.y - j0);
+        t.xs = (uint8_t)(d.rw == 4 ? d.hs : 0);
+        t.xm = (uint8_t)(d.rw == 4 ? d.hm : 0);
+        t.zq_log2 = d.zq_log2;
+        t.inv_z = d.inv_z;
+        tiles_.push_back(t);
+    }
+    return first;
+}
+
+void LivePlan::build(const std::vector<BldInst>& descs, const BldInst* insts, hipStream_t st) {
+    if (!any()) return;
+    for (LiveTile& t : tiles_) t.iter = descs[t.inst].iter;
+    tab_ = DeviceBuffer(tiles_.size() * sizeof(LiveTile));
+    BNMF_HIP(hipMemcpy(tab_.ptr, tiles_.data(), tab_.bytes, hipMemcpyHostToDevice));
+    BNMF_HIP(launch_live_build(dtype_, insts, tab_.as<LiveTile>(), (uint32_t)tiles_.size(), st));
+}
+
+void LivePlan::gather(const BldInst* insts, hipStream_t st) const {
+    if (any()) BNMF_HIP(launch_live_gather(dtype_, insts, tiles(), (uint32_t)tiles_.size(), st));
+}
+
+void LivePlan::scatter(const BldInst* insts, hipStream_t st) const {
+    if (any()) BNMF_HIP(launch_live_scatter(dtype_, insts, tiles(), (uint32_t)tiles_.size(), st));
+}
+
+}  // namespace bnmf

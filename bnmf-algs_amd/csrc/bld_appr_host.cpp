@@ -335,7 +335,7 @@ void ApprBatch::get(size_t idx, void* S, void* nu, void* mu) {
         BNMF_HIP(launch_appr_S(dtype_ == BNMF_F32 ? 0 : 1, ai, xy, stream_));
     }
     BNMF_HIP(hipStreamSynchronize(stream_));
-    if (S && xy) BNMF_HIP(hipMemcpy(S, b + l.off_S, xy * l.z * es_, hipMemcpyDeviceToHost));
+    if (S && xy) stage_.copy(S, b + l.off_S, xy * l.z * es_, stream_);
     if (nu && l.x) BNMF_HIP(hipMemcpy(nu, b + l.off_nu, (size_t)l.x * l.z * es_, hipMemcpyDeviceToHost));
     if (mu && l.y) BNMF_HIP(hipMemcpy(mu, b + l.off_mu, (size_t)l.z * l.y * es_, hipMemcpyDeviceToHost));
 }

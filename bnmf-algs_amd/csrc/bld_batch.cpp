@@ -788,8 +788,7 @@ void Batch::get_S(size_t idx, void* host) const {
     for (size_t n = 0; n < idx; ++n) base += layouts_[n].bytes;
     const InstLayout& L = layouts_[idx];
     if (L.elements() == 0) return;
-    BNMF_HIP(hipStreamSynchronize(stream_));
-    BNMF_HIP(hipMemcpy(host, arena_.as<char>(base) + L.off_S, L.elements() * es_, hipMemcpyDeviceToHost));
+    stage_.copy(host, arena_.as<char>(base) + L.off_S, L.elements() * es_, stream_);
 }
 
 void Batch::log_marginal(double* out) {

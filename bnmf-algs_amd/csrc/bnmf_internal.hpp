@@ -5,6 +5,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <tuple>
@@ -151,6 +152,20 @@ struct DeviceBuffer {
     T* as(size_t byte_off = 0) const {
         return reinterpret_cast<T*>(static_cast<char*>(ptr) + byte_off);
     }
+};
+
+// Results to (pageable) host memory through a pinned buffer of its own
+// (hostcopy.cpp). Safe with several threads: one copy at a time.
+struct HostStage {
+    void* pinned = nullptr;
+    size_t size = 0;
+    std::mutex mu;
+    HostStage() = default;
+    HostStage(const HostStage&) = delete;
+    HostStage& operator=(const HostStage&) = delete;
+    ~HostStage();
+    // bytes from device memory, after the work on st; returns when they are there
+    void copy(void* dst, const void* src, size_t bytes, hipStream_t st);
 };
 
 // ----------------------------------------------------------------- batches
@@ -311,6 +326,7 @@ class Batch {
     DeviceBuffer arena_;
     DeviceBuffer meta_;  // descriptors, work lists, counts
     LivePlan live_;
+    mutable HostStage stage_;
     size_t off_desc_first_ = 0, off_desc_ = 0, off_prep_items_ = 0, off_prep_count_ = 0;
     size_t off_iter_ = 0;  // additive solver: uint32 iteration counters, one per instance
     uint32_t n_prep_items_ = 0;
@@ -390,6 +406,7 @@ class ApprBatch {
     uint32_t n_prep_ = 0, n_fnu_ = 0, n_fmu_ = 0;
     hipStream_t stream_ = nullptr;
     hipGraphExec_t graph_ = nullptr;
+    HostStage stage_;
 };
 
 }  // namespace bnmf

@@ -195,8 +195,7 @@ class Server {
         }
         if (r->state == RS_DONE && S_out && r->L.elements()) {
             BNMF_HIP(hipSetDevice(dev_));
-            BNMF_HIP(hipMemcpy(S_out, dev_buf_.as<char>(r->off) + r->L.off_S, r->L.elements() * es_,
-                               hipMemcpyDeviceToHost));
+            stage_.copy(S_out, dev_buf_.as<char>(r->off) + r->L.off_S, r->L.elements() * es_, nullptr);
         }
         if (lm) *lm = r->log_marginal;
         if (st) {
@@ -576,6 +575,7 @@ class Server {
     int dev_ = 0;
     Arena arena_;
     DeviceBuffer dev_buf_, meta_;
+    HostStage stage_;
     hipStream_t stream_ = nullptr;
     std::vector<hipStream_t> side_;
     std::vector<hipEvent_t> fork_, join_;

@@ -245,7 +245,7 @@ PassKey pass_key(int dtype, int mode, const InstLayout& L, bool nonneg, bool liv
     PassKey k;
     if (L.z > kFusedZ) return k;  // the wide pass (zexact = zb = 0)
     if (live && (mode == MODE_UPDATE || mode == MODE_ADD)) {
-        k.live = dtype == BNMF_F32 ? (int)(L.z + 3) / 4 : (int)(kTileCols / L.tile_cols * 4u + L.rw);
+        k.live = L.z <= 32 ? 1 : 2;
         k.f64 = dtype == BNMF_F64;
         return k;
     }
@@ -433,12 +433,10 @@ Batch::Batch(int dtype, int psi_mode, double eps, const std::vector<InstSpec>& s
         bk.zmax = 1;
         bk.work = 0;
         for (uint32_t n : kv.second) {
-            bk.work += layouts_[n].elements();
+            // a packed element costs about three streamed ones
+            bk.work += bk.key.live ? 3 * live_.fibers(n) * layouts_[n].z : layouts_[n].elements();
             bk.zmax = std::max(bk.zmax, layouts_[n].z);
-            if (bk.key.live) {
-                bk.lds = std::max(bk.lds, live_.lds(n));
-                bk.most = std::max(bk.most, live_.most(n));
-            }
+            if (bk.key.live) bk.lds = std::max(bk.lds, live_.lds(n));
         }
         bk.lane = 0;
         groups_[0].push_back(bk);
@@ -652,8 +650,8 @@ void Batch::enqueue_iterations(int iters, bool first, bool with_prep) {
             for (const Bucket& bk : groups_[0]) {
                 if ((size_t)bk.lane != l) continue;
                 if (bk.key.live) {
-                    BNMF_HIP(launch_pass_live(dtype_, psi_, step_mode_, bk.key.live, bk.n_items, st,
-                                              live_.tiles() + bk.tile0, bk.most, bk.lds));
+                    BNMF_HIP(launch_pass_live(dtype_, psi_, step_mode_, bk.key.live == 2, bk.n_items, st,
+                                              live_.tiles() + bk.tile0, bk.lds));
                     continue;
                 }
                 BNMF_HIP(launch_pass_key(bk.key, dtype_, psi_, step_mode_, dim3(bk.n_items), st, dp,

@@ -312,14 +312,11 @@ __device__ __forceinline__ bool live_psi(const double (&s)[U], double (&ps)[U]) 
 // products the compiler contracts there (nom and den scaled by X_reciprocal,
 // the exp-row norm) are written as the FMAs they become.
 template <int NG, int MODE>
-__global__ void __launch_bounds__(64 * kWaves32) __attribute__((amdgpu_waves_per_eu(NG <= 5 ? 4 : NG <= 8 ? 3 : 2)))
-    bld_live_f32_kernel(const LiveTile* __restrict__ tiles, uint32_t lds_bytes) {
-    extern __shared__ __align__(16) unsigned char lds_raw[];
+__device__ __forceinline__ void live_step_f32(const LiveTile& t, unsigned char* lds_raw, uint32_t lds_bytes) {
     typedef float V4 __attribute__((ext_vector_type(4)));
     typedef float V4u __attribute__((ext_vector_type(4), aligned(4)));
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const LiveTile t = tiles[blockIdx.x];
     const uint32_t z = t.z, n = t.n, xs = t.xs, xmask = t.xm;
     const float epsf = static_cast<float>(t.eps);
     LiveRow* const rt = reinterpret_cast<LiveRow*>(lds_raw);
@@ -457,22 +454,42 @@ __global__ void __launch_bounds__(64 * kWaves32) __attribute__((amdgpu_waves_per
     }
 }
 
+// One launch for every depth up to 32 (LAST = 8) or from 33 to 64 (LAST = 16):
+// a batch's instances of a dozen depths, a few hundred blocks each, fill the
+// GPU together and finish with one tail instead of one per depth (60 instances
+// of z 4 to 32: iteration 80 us against 145 us with a launch per ceil(z / 4),
+// part of it from fullest tiles first and from weighing the streams by packed
+// elements). The registers are those of the deepest case.
+template <int LAST, int MODE>
+__global__ void __launch_bounds__(64 * kWaves32) __attribute__((amdgpu_waves_per_eu(LAST <= 8 ? 3 : 2)))
+    bld_live_f32_kernel(const LiveTile* __restrict__ tiles, uint32_t lds_bytes) {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    const LiveTile t = tiles[blockIdx.x];
+    switch (LAST - (t.z + 3u) / 4u) {
+        case 7: live_step_f32<LAST - 7, MODE>(t, lds_raw, lds_bytes); break;
+        case 6: live_step_f32<LAST - 6, MODE>(t, lds_raw, lds_bytes); break;
+        case 5: live_step_f32<LAST - 5, MODE>(t, lds_raw, lds_bytes); break;
+        case 4: live_step_f32<LAST - 4, MODE>(t, lds_raw, lds_bytes); break;
+        case 3: live_step_f32<LAST - 3, MODE>(t, lds_raw, lds_bytes); break;
+        case 2: live_step_f32<LAST - 2, MODE>(t, lds_raw, lds_bytes); break;
+        case 1: live_step_f32<LAST - 1, MODE>(t, lds_raw, lds_bytes); break;
+        default: live_step_f32<LAST, MODE>(t, lds_raw, lds_bytes); break;
+    }
+}
+
 // FP64, LPF lanes per fiber in the dense pass: a thread evaluates kElems64
 // elements at a time of a set of whole fibers; the gradients meet the fiber
 // sums through LDS.
 template <int LPF, int RW, int MODE, int PSI>
-__global__ void __launch_bounds__(64 * kWaves64) __attribute__((amdgpu_waves_per_eu(4)))
-    bld_live_f64_kernel(const LiveTile* __restrict__ tiles, uint32_t most, uint32_t lds_bytes) {
-    extern __shared__ __align__(16) unsigned char lds_raw[];
+__device__ __forceinline__ void live_step_f64(const LiveTile& t, unsigned char* lds_raw, uint32_t lds_bytes) {
     constexpr uint32_t NT = 64u * kWaves64;
     constexpr uint32_t TW = 64u / LPF;  // tile columns
     constexpr uint32_t U = kElems64;
     const uint32_t tid = threadIdx.x;
-    const LiveTile t = tiles[blockIdx.x];
     const uint32_t z = t.z, n = t.n;
     const double eps = t.eps;
     const float inv_z = t.inv_z;
-    const uint32_t fb = live_fibers64(z, most), ws = odd(z);
+    const uint32_t fb = live_fibers64(z, n), ws = odd(z);
     LiveRow* const rt = reinterpret_cast<LiveRow*>(lds_raw);
     double* const pa_l = reinterpret_cast<double*>(lds_raw + live_table_bytes<TW>(t));  // psi(alpha_eph) of the rows
     double* const pA_l = pa_l + t.trows * z;                                            // psi(A)
@@ -695,6 +712,17 @@ __global__ void __launch_bounds__(64 * kWaves64) __attribute__((amdgpu_waves_per
     }
 }
 
+template <int LPF, int MODE, int PSI>
+__global__ void __launch_bounds__(64 * kWaves64) __attribute__((amdgpu_waves_per_eu(4)))
+    bld_live_f64_kernel(const LiveTile* __restrict__ tiles, uint32_t lds_bytes) {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    const LiveTile t = tiles[blockIdx.x];
+    if (t.z % 2u == 0u)
+        live_step_f64<LPF, 2, MODE, PSI>(t, lds_raw, lds_bytes);
+    else
+        live_step_f64<LPF, 1, MODE, PSI>(t, lds_raw, lds_bytes);
+}
+
 // ------------------------------------------------------- packing, unpacking
 // Nonempty fibers of each tile, one wavefront per tile; ~0u marks an
 // instance the packed form is not for: an X_ij above `most` (near the type's
@@ -907,73 +935,53 @@ void live_group(int dtype, uint32_t z, uint32_t* elems, uint32_t* fibers) {
     *fibers = dtype == 0 ? 64u : 1u;
 }
 
-template <int NG, int MODE>
-static hipError_t live32_one(uint32_t n, hipStream_t st, const LiveTile* tiles, uint32_t lds) {
+template <int LAST, int MODE>
+static hipError_t live32(uint32_t n, hipStream_t st, const LiveTile* tiles, uint32_t lds) {
     if (n == 0)  // set-up
-        return hipFuncSetAttribute(reinterpret_cast<const void*>(bld_live_f32_kernel<NG, MODE>),
+        return hipFuncSetAttribute(reinterpret_cast<const void*>(bld_live_f32_kernel<LAST, MODE>),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes);
-    hipLaunchKernelGGL((bld_live_f32_kernel<NG, MODE>), dim3(n), dim3(64 * kWaves32), lds, st, tiles, lds);
+    hipLaunchKernelGGL((bld_live_f32_kernel<LAST, MODE>), dim3(n), dim3(64 * kWaves32), lds, st, tiles, lds);
     return hipGetLastError();
 }
 
-template <int MODE, int... NGs>
-struct Live32 {
-    static hipError_t launch(int ng, uint32_t n, hipStream_t st, const LiveTile* tiles, uint32_t lds) {
-        hipError_t e = hipErrorInvalidValue;
-        (void)((NGs == ng ? (e = live32_one<NGs, MODE>(n, st, tiles, lds), true) : false) || ...);
-        return e;
-    }
-    static hipError_t attrs() {
-        hipError_t e = hipSuccess;
-        (void)((e = live32_one<NGs, MODE>(0, nullptr, nullptr, 0), e != hipSuccess) || ...);
-        return e;
-    }
-};
-template <int MODE>
-using Live32All = Live32<MODE, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16>;
-
-template <int LPF, int RW, int MODE, int PSI>
-static hipError_t live64_one(uint32_t n, hipStream_t st, const LiveTile* tiles, uint32_t most, uint32_t lds) {
+template <int LPF, int MODE, int PSI>
+static hipError_t live64(uint32_t n, hipStream_t st, const LiveTile* tiles, uint32_t lds) {
     if (n == 0)  // set-up
-        return hipFuncSetAttribute(reinterpret_cast<const void*>(bld_live_f64_kernel<LPF, RW, MODE, PSI>),
+        return hipFuncSetAttribute(reinterpret_cast<const void*>(bld_live_f64_kernel<LPF, MODE, PSI>),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes);
-    hipLaunchKernelGGL((bld_live_f64_kernel<LPF, RW, MODE, PSI>), dim3(n), dim3(64 * kWaves64), lds, st, tiles, most, lds);
+    hipLaunchKernelGGL((bld_live_f64_kernel<LPF, MODE, PSI>), dim3(n), dim3(64 * kWaves64), lds, st, tiles, lds);
     return hipGetLastError();
 }
 
-template <int MODE, int PSI>
-static hipError_t live64(int lpf, int rw, uint32_t n, hipStream_t st, const LiveTile* tiles, uint32_t most, uint32_t lds) {
-    if (lpf == 2)
-        return rw == 2 ? live64_one<2, 2, MODE, PSI>(n, st, tiles, most, lds)
-                       : live64_one<2, 1, MODE, PSI>(n, st, tiles, most, lds);
-    return rw == 2 ? live64_one<4, 2, MODE, PSI>(n, st, tiles, most, lds)
-                   : live64_one<4, 1, MODE, PSI>(n, st, tiles, most, lds);
-}
-
-// Step pass (PASS_UPDATE or PASS_ADD) over the packed fibers of n tiles: ng =
-// ceil(z / 4) of every instance of the launch in FP32; 4 * (the dense pass's
-// lanes per fiber) + (its read width) in FP64.
-hipError_t launch_pass_live(int dtype, int psi, int mode, int ng, uint32_t n, hipStream_t st, const LiveTile* tiles,
-                            uint32_t most, uint32_t lds) {
-    if (n == 0 || (mode != PASS_UPDATE && mode != PASS_ADD)) return hipErrorInvalidValue;
+// Step pass (PASS_UPDATE or PASS_ADD) over the packed fibers of n tiles; big:
+// the instances' depths are 33 to 64, else at most 32.
+hipError_t launch_pass_live(int dtype, int psi, int mode, bool big, uint32_t n, hipStream_t st, const LiveTile* tiles,
+                            uint32_t lds) {
+    if (mode == PASS_ADD) {
+        if (dtype == 0)
+            return big ? live32<16, PASS_ADD>(n, st, tiles, lds) : live32<8, PASS_ADD>(n, st, tiles, lds);
+        return big ? live64<4, PASS_ADD, PSI_F64_APPR>(n, st, tiles, lds)
+                   : live64<2, PASS_ADD, PSI_F64_APPR>(n, st, tiles, lds);
+    }
+    if (mode != PASS_UPDATE) return hipErrorInvalidValue;
     if (dtype == 0)
-        return mode == PASS_UPDATE ? Live32All<PASS_UPDATE>::launch(ng, n, st, tiles, lds)
-                                   : Live32All<PASS_ADD>::launch(ng, n, st, tiles, lds);
-    const int lpf = ng / 4, rw = ng % 4;
-    if (mode == PASS_ADD) return live64<PASS_ADD, PSI_F64_APPR>(lpf, rw, n, st, tiles, most, lds);
-    if (psi == PSI_F64_APPR) return live64<PASS_UPDATE, PSI_F64_APPR>(lpf, rw, n, st, tiles, most, lds);
-    return live64<PASS_UPDATE, PSI_F64_EXACT>(lpf, rw, n, st, tiles, most, lds);
+        return big ? live32<16, PASS_UPDATE>(n, st, tiles, lds) : live32<8, PASS_UPDATE>(n, st, tiles, lds);
+    if (psi == PSI_F64_APPR)
+        return big ? live64<4, PASS_UPDATE, PSI_F64_APPR>(n, st, tiles, lds)
+                   : live64<2, PASS_UPDATE, PSI_F64_APPR>(n, st, tiles, lds);
+    return big ? live64<4, PASS_UPDATE, PSI_F64_EXACT>(n, st, tiles, lds)
+               : live64<2, PASS_UPDATE, PSI_F64_EXACT>(n, st, tiles, lds);
 }
 
 hipError_t init_live_attributes() {
-    hipError_t e = Live32All<PASS_UPDATE>::attrs();
-    if (e == hipSuccess) e = Live32All<PASS_ADD>::attrs();
-    for (int lpf = 2; lpf <= 4; lpf += 2)
-        for (int rw = 1; rw <= 2; ++rw) {
-            if (e == hipSuccess) e = live64<PASS_UPDATE, PSI_F64_EXACT>(lpf, rw, 0, nullptr, nullptr, 0, 0);
-            if (e == hipSuccess) e = live64<PASS_UPDATE, PSI_F64_APPR>(lpf, rw, 0, nullptr, nullptr, 0, 0);
-            if (e == hipSuccess) e = live64<PASS_ADD, PSI_F64_APPR>(lpf, rw, 0, nullptr, nullptr, 0, 0);
-        }
+    hipError_t e = hipSuccess;
+    for (int big = 0; big < 2 && e == hipSuccess; ++big) {
+        e = launch_pass_live(0, PSI_F32, PASS_UPDATE, big, 0, nullptr, nullptr, 0);
+        if (e == hipSuccess) e = launch_pass_live(0, PSI_F32, PASS_ADD, big, 0, nullptr, nullptr, 0);
+        if (e == hipSuccess) e = launch_pass_live(1, PSI_F64_EXACT, PASS_UPDATE, big, 0, nullptr, nullptr, 0);
+        if (e == hipSuccess) e = launch_pass_live(1, PSI_F64_APPR, PASS_UPDATE, big, 0, nullptr, nullptr, 0);
+        if (e == hipSuccess) e = launch_pass_live(1, PSI_F64_APPR, PASS_ADD, big, 0, nullptr, nullptr, 0);
+    }
     return e;
 }
 

@@ -71,11 +71,10 @@ hipError_t launch_pass_wide(int dtype, int psi, int mode, dim3 grid, hipStream_t
 hipError_t launch_pass_f32z(int z, int mode, dim3 grid, hipStream_t st, const BldInst* insts,
                             const PassItem* items, const uint32_t* n_items);
 hipError_t init_f32z_attributes();
-// step passes over the packed nonempty fibers of n tiles (bld_live.hip): ng =
-// ceil(z / 4) (FP32) or 4 * the dense pass's lanes per fiber + its read width
-// (FP64); most: fibers of the fullest tile; lds: dynamic LDS bytes
-hipError_t launch_pass_live(int dtype, int psi, int mode, int ng, uint32_t n, hipStream_t st, const LiveTile* tiles,
-                            uint32_t most, uint32_t lds);
+// step passes over the packed nonempty fibers of n tiles (bld_live.hip) of
+// instances with z <= 32 or (big) 33 <= z <= 64; lds: dynamic LDS bytes
+hipError_t launch_pass_live(int dtype, int psi, int mode, bool big, uint32_t n, hipStream_t st, const LiveTile* tiles,
+                            uint32_t lds);
 hipError_t init_live_attributes();
 // LDS of a block whose tile has n fibers, with kc elements of k at once
 size_t live_lds_need(int dtype, uint32_t z, uint32_t tile_cols, uint32_t rows, uint32_t n, uint32_t kc);
@@ -201,7 +200,7 @@ BldInst make_desc(const InstLayout& L, void* base, double eps, double a, double 
 // shape only, so an instance runs the same kernel alone, batched or served.
 struct PassKey {
     int zexact = 0, zb = 0, rw = 0, f64 = 0;
-    int live = 0;  // step over packed nonempty fibers: ceil(z / 4) (FP32), 4 lanes per fiber + read width (FP64)
+    int live = 0;  // step over packed nonempty fibers: 1 for z <= 32, 2 for 33 <= z <= 64
     bool operator<(const PassKey& o) const {
         return std::tie(zexact, zb, rw, f64, live) < std::tie(o.zexact, o.zb, o.rw, o.f64, o.live);
     }
@@ -233,11 +232,11 @@ class LivePlan {
     bool any() const { return !tiles_.empty(); }
     bool live(size_t n) const { return n < lds_.size() && lds_[n] > 0; }
     uint32_t lds(size_t n) const { return lds_[n]; }
-    uint32_t most(size_t n) const { return most_[n]; }  // fibers of its fullest tile
+    size_t fibers(size_t n) const { return fibers_[n]; }  // its nonempty fibers
     size_t bytes() const { return buf_.bytes; }
     // Appends the tiles of one launch (items: batch instance numbers) to the
     // tile table and returns the first one's index.
-    uint32_t add_launch(const std::vector<PassItem>& items, const std::vector<BldInst>& descs);
+    uint32_t add_launch(std::vector<PassItem>& items, const std::vector<BldInst>& descs);
     // Uploads the tile table and builds the lists; insts: the descriptors on
     // the device
     void build(const std::vector<BldInst>& descs, const BldInst* insts, hipStream_t st);
@@ -253,7 +252,8 @@ class LivePlan {
     int dtype_ = 0;
     DeviceBuffer buf_, tab_;
     std::vector<Off> offs_;
-    std::vector<uint32_t> lds_, most_;  // lds_ 0: the instance runs the dense passes
+    std::vector<size_t> fibers_;
+    std::vector<uint32_t> lds_;  // 0: the instance runs the dense passes
     std::vector<uint32_t> slot_, count_;  // per tile of the live instances: first slot, fibers
     std::vector<LiveTile> tiles_;
 };
@@ -292,8 +292,7 @@ class Batch {
         uint32_t n_items;
         size_t off_items;  // in meta_
         size_t off_count;
-        // live groups: first tile, dynamic LDS, fibers of the fullest tile
-        uint32_t tile0 = 0, lds = 0, most = 0;
+        uint32_t tile0 = 0, lds = 0;  // live groups: first tile, dynamic LDS
     };
     // S of the packed instances from their packed form, and back
     void unpack_S();

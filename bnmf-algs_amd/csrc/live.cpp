@@ -51,7 +51,7 @@ bool LivePlan::worth(int dtype, const void* X, size_t n) {
 
 LivePlan::LivePlan(int dtype, const std::vector<BldInst>& descs, const std::vector<InstLayout>& lay,
                    const std::vector<bool>& candidate, char* scratch)
-    : dtype_(dtype), offs_(descs.size()), lds_(descs.size(), 0), most_(descs.size(), 0) {
+    : dtype_(dtype), offs_(descs.size()), fibers_(descs.size(), 0), lds_(descs.size(), 0) {
     const size_t es = dtype == BNMF_F32 ? 4 : 8;
     // nonempty fibers of every candidate's tiles
     std::vector<PassItem> items;
@@ -105,7 +105,7 @@ LivePlan::LivePlan(int dtype, const std::vector<BldInst>& descs, const std::vect
             if (ok) lds_[n] = (uint32_t)std::max(least, std::min(all, kLdsWant));
         }
         if (ok) {
-            most_[n] = most;
+            fibers_[n] = (size_t)total;
             Off& o = offs_[n];
             o.Sc = take((size_t)(slots / gf) * ge * es);
             o.fib = take((size_t)slots * 2);
@@ -137,7 +137,15 @@ LivePlan::LivePlan(int dtype, const std::vector<BldInst>& descs, const std::vect
     BNMF_HIP(hipMemset(buf_.ptr, 0, off));
 }
 
-uint32_t LivePlan::add_launch(const std::vector<PassItem>& items, const std::vector<BldInst>& descs) {
+uint32_t LivePlan::add_launch(std::vector<PassItem>& items, const std::vector<BldInst>& descs) {
+    // fullest tiles first: the launch's tail is then made of its short blocks
+    std::stable_sort(items.begin(), items.end(), [&](const PassItem& a, const PassItem& b) {
+        auto cost = [&](const PassItem& it) {
+            const BldInst& d = descs[it.inst];
+            return (uint64_t)count_[offs_[it.inst].tile0 + (size_t)it.ti * d.n_tj + it.tj] * d.z;
+        };
+        return cost(a) > cost(b);
+    });
     const uint32_t first = (uint32_t)tiles_.size();
     const size_t es = dtype_ == BNMF_F32 ? 4 : 8;
     for (const PassItem& it : items) {

@@ -51,7 +51,141 @@ uint32_t appr_ti_rows(uint32_t x, uint32_t y, uint32_t n_tj) {
     ti = (ti + 3) / 4 * 4;
     return std::min<uint32_t>(std::max<uint32_t>(ti, 4), 64);
 }
+
+uint32_t zq_of(uint32_t z) {
+    uint32_t q = 1;
+    while (q < z) q <<= 1;
+    return q;
+}
+// Wavefronts per list: four once the mean list keeps one busy for more than a
+// dozen entries per group.
+uint32_t list_waves(size_t entries, uint32_t lists, uint32_t z) {
+    return (double)entries * zq_of(z) > 768.0 * lists ? 4u : 1u;
+}
+// Largest share of nonempty entries at which an FP64 instance runs over them
+// (bld_appr_live.hip), where lanes past z count as work too. Measured per
+// iteration, lists against dense passes: 1024x1024x32 131 us against 975 at a
+// share of 0.1 and 856 against 1000 full; 64 of 200x200x17 (17 of 32 lanes in
+// use) 1072 against 1520 at 0.5 and 1865 against 1529 full; 64 of 400x40x10, 282
+// against 405 and 459 against 419. An instance so small that its launches are
+// all latency takes the lists always (8x10x3: 24 against 40).
+double live_share(size_t x, size_t y, uint32_t z) { return x * y * zq_of(z) <= 8192 ? 1.0 : 0.9 * z / zq_of(z); }
+// Longest list (entries times lanes per entry) that one block may be left to
+// walk where the dense passes would spread it over the chip: 20000x100x20, 633 us
+// against 1725 at lists of 2000; at 6000 both would take about 1750.
+double list_budget(size_t elements) { return std::max(65536.0, (double)elements / 256.0); }
+
+bool within(const double* p, size_t n, double lo, double hi) {
+    for (size_t t = 0; t < n; ++t)
+        if (!(p[t] >= lo && p[t] <= hi)) return false;
+    return true;
+}
 }  // namespace
+
+// May the instance run over its nonempty entries only? An empty one then has
+// to contribute exactly 0, so the gradients it multiplies must be finite:
+// parameters, eps and starting factors of ordinary size. Whatever else the
+// caller gives takes the dense passes, and so does FP32: its solves carry
+// rounding errors of up to 1e-5 after 200 iterations, which sums taken in
+// another order would replace by others as large.
+bool ApprBatch::live_candidate(const ApprSpec& s, double eps) const {
+    const size_t x = s.x, y = s.y, z = s.z;
+    if (dtype_ == BNMF_F32 || z > kFusedZ || x * y == 0 || x * y > 0xffffffffull) return false;
+    if (!(eps >= 1e-200 && eps <= 1.0)) return false;
+    if (!within(s.alpha, x, 1e-6, 1e30) || !within(s.beta, z, 1e-6, 1e30)) return false;
+    auto tame = [](const void* p, size_t n) { return !p || within(static_cast<const double*>(p), n, 0.0, 1e100); };
+    return tame(s.nu0, x * z) && tame(s.mu0, z * y) && LivePlan::worth(dtype_, s.X, x * y, live_share(x, y, s.z));
+}
+
+// The lists of the instances that are sparse enough, in one allocation; none
+// if it cannot be had. counts: (x + y) words per candidate, in order.
+void ApprBatch::plan_live(uint32_t* counts, std::vector<ApprInst>& ai, std::vector<BldInst>& bi) {
+    char* const base = arena_.as<char>();
+    size_t total = 0;
+    for (const L_& l : lay_)
+        if (l.live) {
+            BNMF_HIP(launch_appr_count(arena_.as<double>(l.off_X), l.x, l.y, counts + total, nullptr));
+            total += (size_t)l.x + l.y;
+        }
+    if (total == 0) return;
+    std::vector<uint32_t> cnt(total);
+    BNMF_HIP(hipMemcpy(cnt.data(), counts, total * 4, hipMemcpyDeviceToHost));
+
+    std::vector<uint32_t> ptr;  // per instance: x + 1 row offsets, y + 1 column offsets
+    std::vector<size_t> off_ptr(lay_.size()), off_ent(lay_.size());
+    size_t at = 0, ent_bytes = 0;
+    for (size_t n = 0; n < lay_.size(); ++n) {
+        L_& l = lay_[n];
+        if (!l.live) continue;
+        const uint32_t* const c = cnt.data() + at;
+        at += (size_t)l.x + l.y;
+        size_t entries = 0;
+        uint32_t longest = 0;
+        bool bad = false;
+        for (size_t i = 0; i < (size_t)l.x + l.y; ++i) {
+            bad = bad || c[i] == ~0u;
+            longest = std::max(longest, c[i]);
+            if (i < l.x) entries += c[i];
+        }
+        l.live = !bad && (double)entries <= live_share(l.x, l.y, l.z) * (double)l.x * (double)l.y && (double)longest * zq_of(l.z) <= list_budget((size_t)l.x * l.y * l.z);
+        if (!l.live) continue;
+        l.entries = entries;
+        off_ptr[n] = ptr.size();
+        uint32_t sum = 0;
+        for (size_t i = 0; i < l.x; ++i) {
+            ptr.push_back(sum);
+            sum += c[i];
+        }
+        ptr.push_back(sum);
+        sum = 0;
+        for (size_t j = 0; j < l.y; ++j) {
+            ptr.push_back(sum);
+            sum += c[l.x + j];
+        }
+        ptr.push_back(sum);
+        off_ent[n] = ent_bytes;
+        ent_bytes += 2 * (align_up(entries * 4 + 4) + align_up(entries * 8 + 8));
+    }
+    if (ptr.empty()) return;
+    const size_t ptr_bytes = align_up(ptr.size() * 4);
+    void* p = nullptr;
+    if (hipMalloc(&p, ptr_bytes + ent_bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        for (L_& l : lay_) l.live = false;
+        return;
+    }
+    lists_.ptr = p;
+    lists_.bytes = ptr_bytes + ent_bytes;
+    BNMF_HIP(hipMemcpy(p, ptr.data(), ptr.size() * 4, hipMemcpyHostToDevice));
+    for (size_t n = 0; n < lay_.size(); ++n) {
+        const L_& l = lay_[n];
+        if (!l.live) continue;
+        const size_t oi = align_up(l.entries * 4 + 4), ox = align_up(l.entries * 8 + 8);
+        const uint32_t* const rptr = lists_.as<uint32_t>(off_ptr[n] * 4);
+        const uint32_t* const cptr = rptr + l.x + 1;
+        char* const e = lists_.as<char>(ptr_bytes + off_ent[n]);
+        uint32_t* const ridx = reinterpret_cast<uint32_t*>(e);
+        uint32_t* const cidx = reinterpret_cast<uint32_t*>(e + oi);
+        double* const rxv = reinterpret_cast<double*>(e + 2 * oi);
+        double* const cxv = reinterpret_cast<double*>(e + 2 * oi + ox);
+        BNMF_HIP(launch_appr_fill(arena_.as<double>(l.off_X), l.x, l.y, rptr, ridx, rxv, cptr, cidx, cxv, nullptr));
+        ApprInst& a = ai[n];
+        a.rptr = rptr;
+        a.ridx = ridx;
+        a.rxv = rxv;
+        a.cptr = cptr;
+        a.cidx = cidx;
+        a.cxv = cxv;
+        // the dense passes' second partials are free: y*z and x*z at least
+        a.muT = base + l.off_pjk2;
+        a.partA = base + l.off_ipk2;
+        a.nA = ceil_div(l.x, 4u / list_waves(l.entries, l.x, l.z));
+        zmax_live_ = std::max(zmax_live_, l.z);
+        // left out of the dense instances' psi(A)
+        bi[n].x = 0;
+    }
+    BNMF_HIP(hipStreamSynchronize(nullptr));
+}
 
 ApprBatch::ApprBatch(int dtype, double eps, const std::vector<ApprSpec>& specs)
     : dtype_(dtype), es_(dtype == BNMF_F32 ? 4 : 8) {
@@ -59,7 +193,7 @@ ApprBatch::ApprBatch(int dtype, double eps, const std::vector<ApprSpec>& specs)
     const int psi = dtype == BNMF_F32 ? PSIM_F32 : PSIM_F64_APPR;
     psi_ = psi;
     // layouts
-    size_t total = 0;
+    size_t total = 0, n_counts = 0;
     for (const ApprSpec& s : specs) {
         BNMF_REQUIRE(s.z >= 1, "bld_appr needs z >= 1");
         L_ l{};
@@ -97,10 +231,12 @@ ApprBatch::ApprBatch(int dtype, double eps, const std::vector<ApprSpec>& specs)
         l.off_ipk = take((size_t)l.n_tj * x * z * es_);
         l.off_ipk2 = take((size_t)l.n_tj * x * z * es_);
         l.off_S = take(x * y * z * es_);
+        l.live = live_candidate(s, eps);
+        if (l.live) n_counts += x + y;
         total = off;
         lay_.push_back(l);
     }
-    arena_ = DeviceBuffer(std::max<size_t>(total, kAlign));
+    arena_ = DeviceBuffer(std::max<size_t>(total + n_counts * 4, kAlign));
 
     // uploads; nu0 / mu0 drawn when not given: rows of nu and columns of mu
     // are Dirichlet(1_z) (bld_appr.hpp:302-318), from the init_S stream of
@@ -170,6 +306,8 @@ ApprBatch::ApprBatch(int dtype, double eps, const std::vector<ApprSpec>& specs)
         }
         a.zq = zq;
         a.zq_log2 = lg;
+        a.alpha = reinterpret_cast<const double*>(b + l.off_alpha);
+        a.beta = reinterpret_cast<const double*>(b + l.off_beta);
         ai.push_back(a);
 
         // the prep view of the same buffers
@@ -195,15 +333,22 @@ ApprBatch::ApprBatch(int dtype, double eps, const std::vector<ApprSpec>& specs)
         d.zq_log2 = lg;
         bi.push_back(d);
     }
+    plan_live(arena_.as<uint32_t>(total), ai, bi);
 
     // work lists: pass items by z bucket, prep items, factor items
     std::map<uint32_t, std::vector<PassItem>> by_zb;
     std::map<uint32_t, uint32_t> zmax;
     std::vector<PrepItem> prep;
-    std::vector<PassItem> fnu, fmu;
+    std::vector<PassItem> fnu, fmu, lrow, lcol, lall;
     for (size_t n = 0; n < specs.size(); ++n) {
         const L_& l = lay_[n];
         if ((size_t)l.x * l.y == 0) continue;
+        if (l.live) {
+            const uint32_t wr = list_waves(l.entries, l.x, l.z), wc = list_waves(l.entries, l.y, l.z);
+            for (uint32_t i = 0; i < l.x; i += 4u / wr) lrow.push_back(PassItem{(uint32_t)n, i, 0, wr});
+            for (uint32_t j = 0; j < l.y; j += 4u / wc) lcol.push_back(PassItem{(uint32_t)n, j, 1, wc});
+            continue;
+        }
         const uint32_t zb = z_bucket(l.z);
         auto& v = by_zb[zb];
         for (uint32_t ti = 0; ti < l.n_ti; ++ti)
@@ -215,12 +360,20 @@ ApprBatch::ApprBatch(int dtype, double eps, const std::vector<ApprSpec>& specs)
         for (uint32_t c = 0; c < ceil_div(l.x, 4); ++c) fnu.push_back(PassItem{(uint32_t)n, c, 0, 0});
         for (uint32_t c = 0; c < ceil_div(l.y, 4); ++c) fmu.push_back(PassItem{(uint32_t)n, c, 0, 0});
     }
+    lall = lrow;
+    lall.insert(lall.end(), lcol.begin(), lcol.end());
+    n_live_ = (uint32_t)lall.size();
+    n_lrow_ = (uint32_t)lrow.size();
+    n_lcol_ = (uint32_t)lcol.size();
     size_t moff = 0;
     auto mtake = [&](size_t nbytes) {
         const size_t o = moff;
         moff = align_up(moff + std::max<size_t>(nbytes, 4));
         return o;
     };
+    off_live_ = mtake(lall.size() * sizeof(PassItem));
+    off_lrow_ = mtake(lrow.size() * sizeof(PassItem));
+    off_lcol_ = mtake(lcol.size() * sizeof(PassItem));
     off_ai_ = mtake(ai.size() * sizeof(ApprInst));
     off_bi_ = mtake(bi.size() * sizeof(BldInst));
     for (auto& kv : by_zb) {
@@ -256,6 +409,9 @@ ApprBatch::ApprBatch(int dtype, double eps, const std::vector<ApprSpec>& specs)
             put(g.off_count, &g.n_items, 4);
         }
     }
+    put(off_live_, lall.data(), lall.size() * sizeof(PassItem));
+    put(off_lrow_, lrow.data(), lrow.size() * sizeof(PassItem));
+    put(off_lcol_, lcol.data(), lcol.size() * sizeof(PassItem));
     put(off_prep_, prep.data(), prep.size() * sizeof(PrepItem));
     put(off_prep_count_, &n_prep_, 4);
     put(off_fnu_, fnu.data(), fnu.size() * sizeof(PassItem));
@@ -267,7 +423,8 @@ ApprBatch::ApprBatch(int dtype, double eps, const std::vector<ApprSpec>& specs)
 
 ApprBatch::~ApprBatch() {
     if (stream_) (void)hipStreamSynchronize(stream_);
-    if (graph_) (void)hipGraphExecDestroy(graph_);
+    for (hipGraphExec_t g : graphs_)
+        if (g) (void)hipGraphExecDestroy(g);
     if (stream_) (void)hipStreamDestroy(stream_);
 }
 
@@ -281,34 +438,49 @@ void ApprBatch::enqueue_iteration() {
                                       reinterpret_cast<const PassItem*>(m + g.off_items),
                                       reinterpret_cast<const uint32_t*>(m + g.off_count), g.zmax));
     };
+    const int dt = dtype_ == BNMF_F32 ? 0 : 1;
+    const PassItem* live = reinterpret_cast<const PassItem*>(m + off_live_);
     for (int half = 0; half < 2; ++half) {
         passes(0);
-        BNMF_HIP(launch_prep(dtype_, psi_, false, dim3(n_prep_), stream_, bi,
-                             reinterpret_cast<const PrepItem*>(m + off_prep_),
-                             reinterpret_cast<const uint32_t*>(m + off_prep_count_), (uint32_t)lay_.size()));
+        BNMF_HIP(launch_appr_live(0, n_live_, stream_, ai, live));
+        if (n_prep_ > 0)
+            BNMF_HIP(launch_prep(dtype_, psi_, false, dim3(n_prep_), stream_, bi,
+                                 reinterpret_cast<const PrepItem*>(m + off_prep_),
+                                 reinterpret_cast<const uint32_t*>(m + off_prep_count_), (uint32_t)lay_.size()));
+        if (n_live_ > 0) BNMF_HIP(launch_appr_psiA((uint32_t)lay_.size(), zmax_live_, stream_, ai));
         passes(1 + half);
+        BNMF_HIP(launch_appr_live(1, half == 0 ? n_lrow_ : n_lcol_, stream_, ai,
+                                  reinterpret_cast<const PassItem*>(m + (half == 0 ? off_lrow_ : off_lcol_))));
         const uint32_t nf = half == 0 ? n_fnu_ : n_fmu_;
-        BNMF_HIP(launch_appr_factor(dtype_ == BNMF_F32 ? 0 : 1, half, dim3(nf), stream_, ai,
-                                    reinterpret_cast<const PassItem*>(m + (half == 0 ? off_fnu_ : off_fmu_)),
-                                    reinterpret_cast<const uint32_t*>(m + (half == 0 ? off_fnu_count_ : off_fmu_count_))));
+        if (nf > 0)
+            BNMF_HIP(launch_appr_factor(dt, half, dim3(nf), stream_, ai,
+                                        reinterpret_cast<const PassItem*>(m + (half == 0 ? off_fnu_ : off_fmu_)),
+                                        reinterpret_cast<const uint32_t*>(m + (half == 0 ? off_fnu_count_ : off_fmu_count_))));
     }
 }
 
-void ApprBatch::capture() {
-    if (graph_) return;
+hipGraphExec_t ApprBatch::graph_of(int level) {
+    if (graphs_[level]) return graphs_[level];
     hipGraph_t g = nullptr;
     BNMF_HIP(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
     try {
-        enqueue_iteration();
+        for (int t = 0; t < 1 << level; ++t) enqueue_iteration();
     } catch (...) {
         (void)hipStreamEndCapture(stream_, &g);
         if (g) (void)hipGraphDestroy(g);
         throw;
     }
     BNMF_HIP(hipStreamEndCapture(stream_, &g));
-    hipError_t e = hipGraphInstantiate(&graph_, g, nullptr, nullptr, 0);
+    hipError_t e = hipGraphInstantiate(&graphs_[level], g, nullptr, nullptr, 0);
     (void)hipGraphDestroy(g);
     BNMF_HIP(e);
+    return graphs_[level];
+}
+
+// iterations from the largest graphs down
+void ApprBatch::replay(size_t iters) {
+    for (int l = kGraphLevels - 1; l >= 0; --l)
+        for (; iters >= (size_t)1 << l; iters -= (size_t)1 << l) BNMF_HIP(hipGraphLaunch(graph_of(l), stream_));
 }
 
 void ApprBatch::solve_async(size_t iters) {
@@ -317,10 +489,19 @@ void ApprBatch::solve_async(size_t iters) {
         const size_t xz = (size_t)l.x * l.z, zy = (size_t)l.z * l.y;
         if (xz) BNMF_HIP(hipMemcpyAsync(b + l.off_nu, b + l.off_nu0, xz * es_, hipMemcpyDeviceToDevice, stream_));
         if (zy) BNMF_HIP(hipMemcpyAsync(b + l.off_mu, b + l.off_mu0, zy * es_, hipMemcpyDeviceToDevice, stream_));
+        if (l.live)
+            BNMF_HIP(launch_appr_transpose(arena_.as<double>(l.off_pjk2), arena_.as<double>(l.off_mu0), l.y, l.z, stream_));
     }
-    if (n_prep_ == 0 || iters == 0) return;
-    capture();
-    for (size_t t = 0; t < iters; ++t) BNMF_HIP(hipGraphLaunch(graph_, stream_));
+    if (n_prep_ + n_live_ == 0 || iters == 0) return;
+    replay(iters);
+    mu_back();
+}
+
+// mu of the instances that hold it transposed during a solve
+void ApprBatch::mu_back() {
+    for (const L_& l : lay_)
+        if (l.live)
+            BNMF_HIP(launch_appr_transpose(arena_.as<double>(l.off_mu), arena_.as<double>(l.off_pjk2), l.z, l.y, stream_));
 }
 
 void ApprBatch::synchronize() { BNMF_HIP(hipStreamSynchronize(stream_)); }
@@ -342,8 +523,11 @@ void ApprBatch::get(size_t idx, void* S, void* nu, void* mu) {
 
 double ApprBatch::time_iteration(int reps) {
     BNMF_REQUIRE(reps > 0, "reps must be positive");
-    if (n_prep_ == 0) return 0.0;
-    capture();
+    if (n_prep_ + n_live_ == 0) return 0.0;
+    for (const L_& l : lay_)
+        if (l.live)
+            BNMF_HIP(launch_appr_transpose(arena_.as<double>(l.off_pjk2), arena_.as<double>(l.off_mu), l.y, l.z, stream_));
+    hipGraphExec_t graph = graph_of(0);
     hipEvent_t e0 = nullptr, e1 = nullptr;
     BNMF_HIP(hipEventCreate(&e0));
     hipError_t err = hipEventCreate(&e1);
@@ -352,18 +536,19 @@ double ApprBatch::time_iteration(int reps) {
         BNMF_HIP(err);
     }
     float ms = 0.f;
-    err = hipGraphLaunch(graph_, stream_);
+    err = hipGraphLaunch(graph, stream_);
     if (err == hipSuccess) err = hipEventRecord(e0, stream_);
-    for (int r = 0; r < reps && err == hipSuccess; ++r) err = hipGraphLaunch(graph_, stream_);
+    for (int r = 0; r < reps && err == hipSuccess; ++r) err = hipGraphLaunch(graph, stream_);
     if (err == hipSuccess) err = hipEventRecord(e1, stream_);
     if (err == hipSuccess) err = hipEventSynchronize(e1);
     if (err == hipSuccess) err = hipEventElapsedTime(&ms, e0, e1);
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     BNMF_HIP(err);
+    mu_back();
     return (double)ms / reps;
 }
 
-size_t ApprBatch::device_bytes() const { return arena_.bytes + meta_.bytes; }
+size_t ApprBatch::device_bytes() const { return arena_.bytes + meta_.bytes + lists_.bytes; }
 
 }  // namespace bnmf

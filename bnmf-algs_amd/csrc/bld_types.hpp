@@ -145,7 +145,20 @@ struct ApprInst {
     void* part_pjk2;      // n_ti*y*z: mu's denominator partials
     void* part_ipk2;      // n_tj*x*z: nu's denominator partials
     void* S;              // x*y*z output (final materialisation only)
+    // nonempty entries of X by row and by column (bld_appr_live.hip); null
+    // rptr: dense
+    const uint32_t* rptr; // x + 1: first entry of a row
+    const uint32_t* ridx; // columns of the entries
+    const double* rxv;    // their X_ij
+    const uint32_t* cptr; // y + 1
+    const uint32_t* cidx;
+    const double* cxv;
+    void* muT;            // mu transposed (y*z) during a solve
+    void* partA;          // column sums of alpha_eph per row block
+    const double* alpha;
+    const double* beta;
     double eps;
+    uint32_t nA;          // rows of partA
     uint32_t x, y, z;
     uint32_t ti_rows, n_ti, n_tj;
     uint32_t zq, zq_log2;

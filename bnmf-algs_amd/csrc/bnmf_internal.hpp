@@ -89,6 +89,14 @@ hipError_t launch_appr_pass(int dtype, int mode, int zb, dim3 grid, hipStream_t 
                             const PassItem* items, const uint32_t* n_items, uint32_t zmax);
 hipError_t launch_appr_factor(int dtype, int half, dim3 grid, hipStream_t st, const ApprInst* insts,
                               const PassItem* items, const uint32_t* n_items);
+// the FP64 iteration over the nonempty entries of X (bld_appr_live.hip): step
+// 0 sums (row and column items), 1 step
+hipError_t launch_appr_live(int step, uint32_t n, hipStream_t st, const ApprInst* insts, const PassItem* items);
+hipError_t launch_appr_psiA(uint32_t n_inst, uint32_t zmax, hipStream_t st, const ApprInst* insts);
+hipError_t launch_appr_count(const double* X, uint32_t x, uint32_t y, uint32_t* counts, hipStream_t st);
+hipError_t launch_appr_fill(const double* X, uint32_t x, uint32_t y, const uint32_t* rptr, uint32_t* ridx, double* rxv,
+                            const uint32_t* cptr, uint32_t* cidx, double* cxv, hipStream_t st);
+hipError_t launch_appr_transpose(double* dst, const double* src, uint32_t n, uint32_t m, hipStream_t st);
 hipError_t launch_appr_S(int dtype, const ApprInst* inst, size_t n_fibers, hipStream_t st);
 hipError_t init_appr_attributes();
 void ensure_runtime();  // per-process kernel attributes, once
@@ -227,8 +235,12 @@ class LivePlan {
              const std::vector<bool>& candidate, char* scratch);
     LivePlan() = default;
     static size_t scratch_bytes(const std::vector<InstLayout>& lay);
-    // false where X (host, n entries) is plainly too full to be packed
-    static bool worth(int dtype, const void* X, size_t n);
+    // Largest share of nonempty fibers at which an instance is packed. The packed
+    // step's cost grows with the share, the dense step's does not; at 28 % (100 x
+    // 100 x 17 in double) it takes half the dense step's time.
+    static constexpr double kLiveMax = 0.5;
+    // false where X (host, n entries) is plainly fuller than `most`
+    static bool worth(int dtype, const void* X, size_t n, double most = kLiveMax);
     bool any() const { return !tiles_.empty(); }
     bool live(size_t n) const { return n < lds_.size() && lds_[n] > 0; }
     uint32_t lds(size_t n) const { return lds_[n]; }
@@ -387,13 +399,19 @@ class ApprBatch {
         uint32_t x, y, z, ti_rows, n_ti, n_tj, nA, n_cj;
         size_t off_X, off_nu, off_mu, off_nu0, off_mu0, off_alpha, off_beta, off_psib, off_psia, off_partA,
             off_psiA, off_pjk, off_pjk2, off_ipk, off_ipk2, off_S;
+        bool live = false;  // over the nonempty entries of X
+        size_t entries = 0;
     };
     struct Group {
         uint32_t zb, zmax, n_items;
         size_t off_items, off_count;
     };
     void enqueue_iteration();
-    void capture();
+    hipGraphExec_t graph_of(int level);
+    void replay(size_t iters);
+    void mu_back();
+    bool live_candidate(const ApprSpec& s, double eps) const;
+    void plan_live(uint32_t* counts, std::vector<ApprInst>& ai, std::vector<BldInst>& bi);
 
     int dtype_, psi_ = 0;
     size_t es_;
@@ -403,8 +421,14 @@ class ApprBatch {
     size_t off_ai_ = 0, off_bi_ = 0, off_prep_ = 0, off_prep_count_ = 0, off_fnu_ = 0, off_fnu_count_ = 0,
            off_fmu_ = 0, off_fmu_count_ = 0;
     uint32_t n_prep_ = 0, n_fnu_ = 0, n_fmu_ = 0;
+    // work lists over the nonempty entries: both sides (sums), rows, columns
+    DeviceBuffer lists_;
+    size_t off_live_ = 0, off_lrow_ = 0, off_lcol_ = 0;
+    uint32_t zmax_live_ = 0, n_live_ = 0, n_lrow_ = 0, n_lcol_ = 0;
     hipStream_t stream_ = nullptr;
-    hipGraphExec_t graph_ = nullptr;
+    // captured graphs of 1, 2, 4, ... iterations, each instantiated on first use
+    static constexpr int kGraphLevels = 5;
+    hipGraphExec_t graphs_[kGraphLevels] = {};
     HostStage stage_;
 };
 

@@ -14,10 +14,6 @@ namespace {
 constexpr size_t kAlign = 256;
 size_t align_up(size_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 
-// Largest share of nonempty fibers at which an instance is packed. The packed
-// step's cost grows with the share, the dense step's does not; at 28 % (100 x
-// 100 x 17 in double) it takes half the dense step's time.
-constexpr double kLiveMax = 0.5;
 // LDS a block takes when its tile needs it, so that two share a CU; a tile
 // with more fibers does its partial sums over k in parts, and may take up to
 // kLdsMost.
@@ -34,19 +30,19 @@ size_t LivePlan::scratch_bytes(const std::vector<InstLayout>& lay) {
 // A matrix whose sampled entries (4096 at most, evenly spaced) are mostly
 // nonzero is not worth the count on the device.
 template <typename T>
-static bool mostly_full(const T* X, size_t n) {
+static bool mostly_full(const T* X, size_t n, double most) {
     const size_t step = std::max<size_t>(1, n / 4096);
     size_t seen = 0, full = 0;
     for (size_t t = 0; t < n; t += step) {
         ++seen;
         full += X[t] != T(0);
     }
-    return (double)full > 1.2 * kLiveMax * (double)seen;
+    return (double)full > 1.2 * most * (double)seen;
 }
 
-bool LivePlan::worth(int dtype, const void* X, size_t n) {
-    return !(dtype == BNMF_F32 ? mostly_full(static_cast<const float*>(X), n)
-                               : mostly_full(static_cast<const double*>(X), n));
+bool LivePlan::worth(int dtype, const void* X, size_t n, double most) {
+    return !(dtype == BNMF_F32 ? mostly_full(static_cast<const float*>(X), n, most)
+                               : mostly_full(static_cast<const double*>(X), n, most));
 }
 
 LivePlan::LivePlan(int dtype, const std::vector<BldInst>& descs, const std::vector<InstLayout>& lay,

@@ -243,7 +243,10 @@ static bool generic_steps() {
 PassKey pass_key(int dtype, int mode, const InstLayout& L, bool nonneg, bool live) {
     const bool generic = generic_steps();
     PassKey k;
-    if (L.z > kFusedZ) return k;  // the wide pass (zexact = zb = 0)
+    if (L.z > kFusedZ) {  // the wide pass (zexact = zb = 0)
+        k.rw = wide_regs_nk(L.z);
+        return k;
+    }
     if (live && (mode == MODE_UPDATE || mode == MODE_ADD)) {
         k.live = L.z <= 32 ? 1 : 2;
         k.f64 = dtype == BNMF_F64;
@@ -267,7 +270,7 @@ PassKey pass_key(int dtype, int mode, const InstLayout& L, bool nonneg, bool liv
 hipError_t launch_pass_key(const PassKey& k, int dtype, int psi, int mode, dim3 grid,
                            hipStream_t st, const BldInst* insts, const PassItem* items,
                            const uint32_t* n_items, uint32_t zmax) {
-    if (k.wide()) return launch_pass_wide(dtype, psi, mode, grid, st, insts, items, n_items);
+    if (k.wide()) return launch_pass_wide(dtype, psi, mode, k.rw, grid, st, insts, items, n_items);
     if (k.f64) {
         if (dtype != BNMF_F64 || (mode != MODE_UPDATE && mode != MODE_ADD)) return hipErrorInvalidValue;
         return launch_pass_f64(psi, mode, k.zb, k.rw, grid, st, insts, items, n_items);

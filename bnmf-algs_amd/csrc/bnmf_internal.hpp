@@ -64,7 +64,8 @@ hipError_t launch_pass_f64(int psi, int mode, int zb, int rw, dim3 grid, hipStre
                            const PassItem* items, const uint32_t* n_items);
 hipError_t init_f64_attributes();
 // any mode and dtype for instances deeper than kFusedZ (bld_wide.hip)
-hipError_t launch_pass_wide(int dtype, int psi, int mode, dim3 grid, hipStream_t st, const BldInst* insts,
+int wide_regs_nk(uint32_t z);  // wavefront-lengths of a fiber the wide pass holds in registers; 0: too deep
+hipError_t launch_pass_wide(int dtype, int psi, int mode, int nk, dim3 grid, hipStream_t st, const BldInst* insts,
                             const PassItem* items, const uint32_t* n_items);
 // FP32 step pass (MODE_UPDATE or MODE_ADD) specialised on the exact fiber
 // depth z (bld_pass_f32z.hip)
@@ -207,7 +208,7 @@ BldInst make_desc(const InstLayout& L, void* base, double eps, double a, double 
 // Instances with equal keys share a launch. The key depends on the instance
 // shape only, so an instance runs the same kernel alone, batched or served.
 struct PassKey {
-    int zexact = 0, zb = 0, rw = 0, f64 = 0;
+    int zexact = 0, zb = 0, rw = 0, f64 = 0;  // wide: rw as wide_regs_nk
     int live = 0;  // step over packed nonempty fibers: 1 for z <= 32, 2 for 33 <= z <= 64
     bool operator<(const PassKey& o) const {
         return std::tie(zexact, zb, rw, f64, live) < std::tie(o.zexact, o.zb, o.rw, o.f64, o.live);

@@ -74,7 +74,7 @@ uint32_t tile_cols_of(int dtype, uint32_t z) {
     return kTileCols;
 }
 
-uint32_t choose_ti_rows(int dtype, uint32_t x, uint32_t y, uint32_t z) {
+uint32_t choose_ti_rows(int dtype, uint32_t x, uint32_t y, uint32_t z, bool tall) {
     // an empty instance has no tiles (and x = 0 would divide by zero below)
     if (x == 0 || y == 0) return 4;
     // deep fibers: the wide pass's fixed tiles
@@ -100,6 +100,20 @@ uint32_t choose_ti_rows(int dtype, uint32_t x, uint32_t y, uint32_t z) {
     const uint32_t cap = env_cap > 0 ? (uint32_t)std::min<long>(std::max<long>(env_cap, 4), 1024)
                                      : tuned ? tuned : (large ? 128u : 64u);
     uint32_t nt = (x + cap - 1) / cap;
+    // A small FP64 instance without a table entry takes tiles of about 5120
+    // elements, of 8 rows at least, up to 1024 tiles: its step is bound by the
+    // arithmetic of each tile's block, and 64-row tiles leave most CUs idle.
+    // Iteration of a lone dense instance at 64 rows and by this rule: 100x100x17
+    // 127 -> 74 us, 384x300x32 180 -> 54, 256x128x64 193 -> 167; with mostly zero
+    // counts 225 -> 49, 98 -> 34 and 136 -> 35. Sixteen at once: 128 -> 75,
+    // 200x200x17 187 -> 163, 256x128x64 279 -> 293 dense and 182 -> 43. FP32 keeps
+    // its heights: its sums in another order move results by up to 1e-5.
+    if (dtype == BNMF_F64 && !large && !tall && env_cap <= 0 && tuned == 0) {
+        const uint64_t row = (uint64_t)std::min(y, tile_cols_of(dtype, z)) * z;
+        const uint32_t rows = (uint32_t)std::max<uint64_t>(5120u / row / 4u * 4u, 8u);
+        const uint32_t fill = (1024u + n_tj - 1) / n_tj;
+        nt = std::max(nt, std::min((x + rows - 1) / rows, fill));
+    }
     if (large) {
         const uint32_t target = dtype == BNMF_F64 ? 1024u : 512u;
         const uint32_t fill = (target + n_tj - 1) / n_tj;
@@ -142,7 +156,7 @@ void xcd_order(std::vector<PassItem>& v) {
     v.swap(out);
 }
 
-InstLayout plan_instance(int dtype, uint32_t x, uint32_t y, uint32_t z, bool with_S0) {
+InstLayout plan_instance(int dtype, uint32_t x, uint32_t y, uint32_t z, bool with_S0, bool tall) {
     InstLayout L{};
     const size_t es = dtype == BNMF_F32 ? 4 : 8;
     L.x = x;
@@ -150,7 +164,7 @@ InstLayout plan_instance(int dtype, uint32_t x, uint32_t y, uint32_t z, bool wit
     L.z = z;
     L.zb = z_bucket(z);
     read_layout(dtype, z, &L.rw, &L.hs, &L.hm);
-    L.ti_rows = choose_ti_rows(dtype, x, y, z);
+    L.ti_rows = choose_ti_rows(dtype, x, y, z, tall);
     L.tile_cols = tile_cols_of(dtype, z);
     L.n_ti = ceil_div(x, L.ti_rows);
     L.n_tj = ceil_div(y, L.tile_cols);
@@ -322,20 +336,32 @@ Batch::Batch(int dtype, int psi_mode, double eps, const std::vector<InstSpec>& s
     dev_ = dev;
     BNMF_HIP(hipDeviceGetAttribute(&cus_, hipDeviceAttributeMultiprocessorCount, dev));
 
-    // layouts and arena
+    // layouts and arena; tall tiles where the memory for short ones' partial
+    // sums cannot be had
     std::vector<size_t> base_off(specs.size());
-    size_t total = 0;
-    for (size_t n = 0; n < specs.size(); ++n) {
-        const InstSpec& s = specs[n];
+    size_t off_scratch = 0;
+    for (const InstSpec& s : specs)
         BNMF_REQUIRE(s.x < (1u << 31) && s.y < (1u << 31) && s.z < (1u << 31),
                      "x, y and z must be below 2^31");
-        layouts_.push_back(plan_instance(dtype, s.x, s.y, s.z));
-        base_off[n] = total;
-        total += layouts_.back().bytes;
+    auto plan = [&](bool tall) {
+        layouts_.clear();
+        size_t total = 0;
+        for (size_t n = 0; n < specs.size(); ++n) {
+            layouts_.push_back(plan_instance(dtype, specs[n].x, specs[n].y, specs[n].z, true, tall));
+            base_off[n] = total;
+            total += layouts_.back().bytes;
+        }
+        off_scratch = total;
+        return std::max<size_t>(total + LivePlan::scratch_bytes(layouts_), kAlign);
+    };
+    const size_t bytes = plan(false);
+    if (hipMalloc(&arena_.ptr, bytes) == hipSuccess) {
+        arena_.bytes = bytes;
+    } else {
+        (void)hipGetLastError();
+        arena_.ptr = nullptr;
+        arena_ = DeviceBuffer(plan(true));
     }
-    const size_t off_scratch = total;
-    total += LivePlan::scratch_bytes(layouts_);
-    arena_ = DeviceBuffer(std::max<size_t>(total, kAlign));
     device_bytes_ = arena_.bytes;
 
     // uploads (X, alpha, beta, S0 or its device draw). nonneg[n]: S0 >= 0

@@ -120,7 +120,8 @@ hipError_t launch_sample(double* out, const double* W, const double* H, const do
 // ----------------------------------------------------------- tile planner
 // z bucket of the fused generic pass (z <= kFusedZ); 0 for the wide pass
 uint32_t z_bucket(uint32_t z);
-uint32_t choose_ti_rows(int dtype, uint32_t x, uint32_t y, uint32_t z);
+// tall: without the short tiles of small FP64 instances
+uint32_t choose_ti_rows(int dtype, uint32_t x, uint32_t y, uint32_t z, bool tall = false);
 // Lays the items of one pass launch out XCD by XCD (L2 sharing of the
 // per-column psi staging); results do not depend on item order.
 void xcd_order(std::vector<PassItem>& items);
@@ -198,7 +199,7 @@ struct InstLayout {
 };
 // with_S0: reserve a separate buffer for the initial tensor (batches keep S0
 // to restart solves; the server solves in place).
-InstLayout plan_instance(int dtype, uint32_t x, uint32_t y, uint32_t z, bool with_S0 = true);
+InstLayout plan_instance(int dtype, uint32_t x, uint32_t y, uint32_t z, bool with_S0 = true, bool tall = false);
 BldInst make_desc(const InstLayout& L, void* base, double eps, double a, double b, bool first,
                   bool nonneg = false);
 

@@ -143,6 +143,8 @@ class Server {
         r->want_lm = want_lm != 0;
         r->max_iter = max_iter;
         r->L = plan_instance(dtype_, r->x, r->y, r->z, false);
+        // tall tiles (a last-digits change) rather than no answer
+        if (r->L.bytes > arena_.capacity()) r->L = plan_instance(dtype_, r->x, r->y, r->z, false, true);
         r->t_submit = now_s();
         std::lock_guard<std::mutex> lk(mu_);
         if (failed_) throw Error(BNMF_ERR_DEVICE, "server failed: " + fail_msg_);

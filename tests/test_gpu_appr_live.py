@@ -1,6 +1,5 @@
-"""The approximate solver over the nonempty entries of X (bld_appr_live.hip, FP64;
-FP32 stays on the dense passes) against the oracle, on both sides of the rule that chooses it: shares of
-nonempty entries from almost none to all, empty rows and columns, lists for one
+"""The approximate solver over the nonempty entries of X (bld_appr_live.hip)
+against the oracle, on both sides of the rule that chooses it: shares of nonempty entries from almost none to all, empty rows and columns, lists for one
 and for four wavefronts, z at and around powers of two.
 
 FP64 bounds are those of tests/test_gpu_bld_appr.py (1e-12 relative normwise
@@ -79,3 +78,17 @@ def test_appr_over_nonempty_entries(hip, oracle, dtype, share):
                 for g, a in zip(got, alone):
                     assert np.array_equal(g, a, equal_nan=True), (SHAPES[n], share, iters)
     assert compared >= len(SHAPES)
+
+
+@pytest.mark.parametrize("n", range(len(SHAPES) - 1))
+def test_appr_f32_iterates_in_double(hip, oracle, n):
+    """An FP32 instance over lists is solved in double from its FP32 start: nu and
+    mu carry one rounding (2^-24 = 6e-8; 1e-7 with the FP64 bound), S the roundings
+    of an FP32 sum of z products and five more operations, (z + 5) 2^-24 at most."""
+    i = _problem(hip, SHAPES[n], 0.03, 11 * n + 1, np.float32)
+    ref, moves = _oracle(oracle, i, 12, np.float64)
+    S, nu, mu = hip.bld_appr(i.X, i.z, i.params, 12, nu0=i.nu0, mu0=i.mu0, dtype=np.float32)
+    if not moves < 1e-13:
+        return  # no trajectory to compare, see above
+    assert _rel(nu, ref[1]) < 1e-7 and _rel(mu, ref[2]) < 1e-7
+    assert _rel(S, ref[0]) < (i.z + 5) * 2.0 ** -24 + 1e-10

@@ -38,6 +38,7 @@ void ensure_runtime() {
         if (status == hipSuccess) status = init_f64_attributes();
         if (status == hipSuccess) status = init_appr_attributes();
         if (status == hipSuccess) status = init_live_attributes();
+        if (status == hipSuccess) status = init_tiny_attributes();
     });
     BNMF_HIP(status);
 }
@@ -415,6 +416,22 @@ Batch::Batch(int dtype, int psi_mode, double eps, const std::vector<InstSpec>& s
         d_first.push_back(make_desc(L, b, eps, specs[n].a, specs[n].b, true, nonneg[n]));
         d_main.push_back(make_desc(L, b, eps, specs[n].a, specs[n].b, false, nonneg[n]));
     }
+    // A batch of nothing but tiny instances is solved by bld_tiny.hip. One that
+    // also holds others runs the passes for all (equal bits): its iteration is
+    // theirs, and the tiny ones cost it next to nothing.
+    if (dtype == BNMF_F64 && algo_ == BNMF_ALGO_MULT) {
+        bool all = true;
+        for (const InstLayout& L : layouts_) {
+            if (L.elements() == 0) continue;
+            all = all && L.n_ti == 1 && L.n_tj == 1 && L.z <= kFusedZ && L.x <= 64 && L.elements() <= kTinyElems &&
+                  tiny_lds(L.x, L.y, L.z) <= kTinyLds;
+            if (!all) break;
+            tiny_threads_ = std::max(tiny_threads_, tiny_threads(L.x, L.y, L.z));
+            tiny_lds_ = std::max(tiny_lds_, tiny_lds(L.x, L.y, L.z));
+        }
+        if (!all) tiny_threads_ = 0;
+        if (tiny_threads_) packable.assign(specs.size(), false);
+    }
     // the instances whose nonempty fibers are kept packed
     live_ = LivePlan(dtype, d_main, layouts_, packable, arena_.as<char>(off_scratch));
     device_bytes_ += live_.bytes();
@@ -729,10 +746,25 @@ void Batch::solve_async(size_t iters) {
         }
         return;
     }
-    start_solve();
-    replay_iterations(iters - 1);
-    unpack_S();
+    if (tiny_threads_) {
+        run_tiny(iters, true);
+    } else {
+        start_solve();
+        replay_iterations(iters - 1);
+        unpack_S();
+    }
     partials_valid_ = true;
+}
+
+// launches of 4096 iterations (some 20 ms) at most
+void Batch::run_tiny(size_t iters, bool first) {
+    while (iters > 0) {
+        const uint32_t n = (uint32_t)std::min<size_t>(iters, 4096);
+        BNMF_HIP(launch_tiny(psi_, (uint32_t)layouts_.size(), tiny_threads_, tiny_lds_, stream_,
+                             reinterpret_cast<const BldInst*>(meta_.as<char>() + (first ? off_desc_first_ : off_desc_)), n));
+        iters -= n;
+        first = false;
+    }
 }
 
 void Batch::start_solve() {
@@ -775,7 +807,9 @@ size_t Batch::solve_tol(size_t max_iter, double tol, size_t check_every, double*
     bool scored = false;
     while (done < max_iter) {
         const size_t chunk = std::min(check_every, max_iter - done);
-        if (done == 0) {
+        if (tiny_threads_) {
+            run_tiny(chunk, done == 0);
+        } else if (done == 0) {
             start_solve();
             replay_iterations(chunk - 1);
         } else {

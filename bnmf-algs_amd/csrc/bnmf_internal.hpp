@@ -85,6 +85,16 @@ hipError_t launch_live_count(int dtype, const BldInst* insts, const PassItem* it
 hipError_t launch_live_build(int dtype, const BldInst* insts, LiveTile* tiles, uint32_t n, hipStream_t st);
 hipError_t launch_live_gather(int dtype, const BldInst* insts, const LiveTile* tiles, uint32_t n, hipStream_t st);
 hipError_t launch_live_scatter(int dtype, const BldInst* insts, const LiveTile* tiles, uint32_t n, hipStream_t st);
+// iters iterations of n_inst FP64 instances of one tile each, a block per
+// instance with everything in LDS (bld_tiny.hip): S from S_src, S and its
+// partial sums out
+constexpr uint32_t kTinyElems = 4096;
+constexpr size_t kTinyLds = 156 * 1024;
+size_t tiny_lds(uint32_t x, uint32_t y, uint32_t z);
+uint32_t tiny_threads(uint32_t x, uint32_t y, uint32_t z);
+hipError_t launch_tiny(int psi, uint32_t n_inst, uint32_t threads, size_t lds, hipStream_t st, const BldInst* insts,
+                       uint32_t iters);
+hipError_t init_tiny_attributes();
 // approximate solver (bld_appr.hip): mode 0 sums, 1 nu step, 2 mu step
 hipError_t launch_appr_pass(int dtype, int mode, int zb, dim3 grid, hipStream_t st, const ApprInst* insts,
                             const PassItem* items, const uint32_t* n_items, uint32_t zmax);
@@ -311,6 +321,8 @@ class Batch {
         size_t off_count;
         uint32_t tile0 = 0, lds = 0;  // live groups: first tile, dynamic LDS
     };
+    // iterations of a batch of tiny instances; first: from S0
+    void run_tiny(size_t iters, bool first);
     // S of the packed instances from their packed form, and back
     void unpack_S();
     void pack_S(bool first);
@@ -342,6 +354,9 @@ class Batch {
     DeviceBuffer arena_;
     DeviceBuffer meta_;  // descriptors, work lists, counts
     LivePlan live_;
+    // every instance is tiny: threads and LDS of a block (0: run the passes)
+    uint32_t tiny_threads_ = 0;
+    size_t tiny_lds_ = 0;
     mutable HostStage stage_;
     size_t off_desc_first_ = 0, off_desc_ = 0, off_prep_items_ = 0, off_prep_count_ = 0;
     size_t off_iter_ = 0;  // additive solver: uint32 iteration counters, one per instance

@@ -401,6 +401,7 @@ ApprBatch::ApprBatch(int dtype, double eps, const std::vector<ApprSpec>& specs)
         for (uint32_t ti = 0; ti < l.n_ti; ++ti)
             for (uint32_t tj = 0; tj < l.n_tj; ++tj) v.push_back(PassItem{(uint32_t)n, ti, tj, 0});
         zmax[zb] = std::max(zmax[zb], l.z);
+        zmax_dense_ = std::max(zmax_dense_, l.z);
         for (uint32_t c = 0; c < l.n_cj; ++c) prep.push_back(PrepItem{(uint32_t)n, 0, c, 0});
         for (uint32_t c = 0; c < l.nA; ++c) prep.push_back(PrepItem{(uint32_t)n, 1, c, 0});
         // factor updates: four rows (columns) per item, one per wavefront
@@ -494,7 +495,7 @@ void ApprBatch::enqueue_dense() {
         passes(0);
         BNMF_HIP(launch_prep(dtype_, psi_, false, dim3(n_prep_), stream_, reinterpret_cast<const BldInst*>(m + off_bi_),
                              reinterpret_cast<const PrepItem*>(m + off_prep_),
-                             reinterpret_cast<const uint32_t*>(m + off_prep_count_), (uint32_t)lay_.size()));
+                             reinterpret_cast<const uint32_t*>(m + off_prep_count_), (uint32_t)lay_.size(), zmax_dense_));
         passes(1 + half);
         BNMF_HIP(launch_appr_factor(dt, half, dim3(half == 0 ? n_fnu_ : n_fmu_), stream_, ai,
                                     reinterpret_cast<const PassItem*>(m + (half == 0 ? off_fnu_ : off_fmu_)),

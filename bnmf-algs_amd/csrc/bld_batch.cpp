@@ -554,7 +554,11 @@ Batch::Batch(int dtype, int psi_mode, double eps, const std::vector<InstSpec>& s
     for (size_t l = 0; l < lanes_.size(); ++l) {
         Lane& ln = lanes_[l];
         ln.n_inst = (uint32_t)lane_members[l].size();
-        for (uint32_t n : lane_members[l]) ln.n_prep += layouts_[n].n_cj + layouts_[n].nA;
+        for (uint32_t n : lane_members[l]) {
+            ln.n_prep += layouts_[n].n_cj + layouts_[n].nA;
+            ln.zmax = std::max(ln.zmax, layouts_[n].z);
+        }
+        zmax_ = std::max(zmax_, ln.zmax);
         ln.off_desc = mtake(ln.n_inst * sizeof(BldInst));
         ln.off_desc_first = mtake(ln.n_inst * sizeof(BldInst));
         ln.off_prep = mtake((size_t)ln.n_prep * sizeof(PrepItem));
@@ -690,7 +694,7 @@ void Batch::enqueue_iterations(int iters, bool first, bool with_prep) {
                 BNMF_HIP(launch_prep(dtype_, psi_, false, dim3(ln.n_prep), st,
                                      reinterpret_cast<const BldInst*>(m + ln.off_desc),
                                      reinterpret_cast<const PrepItem*>(m + ln.off_prep),
-                                     reinterpret_cast<const uint32_t*>(m + ln.off_prep_count), ln.n_inst));
+                                     reinterpret_cast<const uint32_t*>(m + ln.off_prep_count), ln.n_inst, ln.zmax));
             const BldInst* dp =
                 reinterpret_cast<const BldInst*>(m + ((first && t == 0) ? ln.off_desc_first : ln.off_desc));
             for (const Bucket& bk : groups_[0]) {
@@ -957,7 +961,7 @@ void Batch::tensor_sums(void* S_pjk, void* S_ipk, void* S_ijp) {
                              reinterpret_cast<const uint32_t*>(m + bk.off_count), bk.zmax));
     BNMF_HIP(launch_prep(dtype_, psi_, true, dim3(n_prep_items_), stream_, dd.as<BldInst>(),
                          reinterpret_cast<const PrepItem*>(m + off_prep_items_),
-                         reinterpret_cast<const uint32_t*>(m + off_prep_count_), (uint32_t)layouts_.size()));
+                         reinterpret_cast<const uint32_t*>(m + off_prep_count_), (uint32_t)layouts_.size(), L.z));
     BNMF_HIP(hipStreamSynchronize(stream_));
     if (S_pjk) BNMF_HIP(hipMemcpy(S_pjk, arena_.as<char>(L.off_psib), (size_t)L.y * L.z * es_, hipMemcpyDeviceToHost));
     if (S_ipk) BNMF_HIP(hipMemcpy(S_ipk, arena_.as<char>(L.off_psia), (size_t)L.x * L.z * es_, hipMemcpyDeviceToHost));
@@ -979,7 +983,7 @@ void Batch::fact(size_t idx, double eps, double* W, double* H, double* L) {
     BNMF_HIP(launch_prep(dtype_, psi_, true, dim3(n_prep_items_), stream_,
                          reinterpret_cast<const BldInst*>(m + off_desc_),
                          reinterpret_cast<const PrepItem*>(m + off_prep_items_),
-                         reinterpret_cast<const uint32_t*>(m + off_prep_count_), (uint32_t)layouts_.size()));
+                         reinterpret_cast<const uint32_t*>(m + off_prep_count_), (uint32_t)layouts_.size(), zmax_));
     const size_t nW = (size_t)Li.x * Li.z, nH = (size_t)Li.z * Li.y, nL = Li.y;
     DeviceBuffer out((nW + nH + nL) * 8);
     const BldInst* d = reinterpret_cast<const BldInst*>(m + off_desc_) + idx;

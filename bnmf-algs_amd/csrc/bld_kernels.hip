@@ -501,6 +501,13 @@ __device__ __forceinline__ void add_strided(SumAcc<T>& s, const T* __restrict__ 
     for (; t < n; ++t) s.add(base[(size_t)t * stride]);
 }
 
+// Deep fibers (z > kFusedZ): elements of k a block takes at a time; up to
+// kPrepDeepParts blocks share an item (grid.y). An instance has x / 16 + y / 16
+// items, too few for the chip when one block walks all of k: 320x448x100 45 us
+// with a thread per k and a block per item, 9 us so.
+constexpr uint32_t kPrepDeep = 32;
+constexpr uint32_t kPrepDeepParts = 8;
+
 template <typename T, int PSI, bool RAW>
 __global__ void __launch_bounds__(256)
     bld_prep_kernel(const BldInst* __restrict__ insts, const PrepItem* __restrict__ items,
@@ -513,13 +520,15 @@ __global__ void __launch_bounds__(256)
         const BldInst* __restrict__ I = insts + item.inst;
         const uint32_t x = I->x, y = I->y, z = I->z;
         const float inv_z = I->inv_z;
+        if (blockIdx.y > 0 && z <= kFusedZ) continue;  // one block an item
         if (item.kind == 0) {
             const uint32_t c0 = item.chunk * kPrepCols;
             const uint32_t nc = min(kPrepCols, y - c0);
             const T* __restrict__ pp = static_cast<const T*>(I->part_pjk);
             T* __restrict__ psib = static_cast<T*>(I->psib);
             const size_t stride = (size_t)y * z;
-            for (uint32_t e = tid; e < nc * z; e += 256) {
+            const uint32_t step = 256u * (z > kFusedZ ? gridDim.y : 1u);
+            for (uint32_t e = blockIdx.y * 256u + tid; e < nc * z; e += step) {
                 const size_t idx = (size_t)c0 * z + e;
                 const uint32_t k = z <= kFusedZ ? e - fiber_of(e, inv_z) * z : e % z;
                 SumAcc<T> s;
@@ -532,16 +541,18 @@ __global__ void __launch_bounds__(256)
                 }
             }
         } else if (z > kFusedZ) {
-            // deep fibers: one thread per k walks the chunk's rows in order,
-            // so the alpha_eph column sums need no LDS staging
+            // deep fibers: kPrepDeep elements of k at a time, dealt over the
+            // blocks of grid.y, a thread per (row, k); then the alpha_eph
+            // column sums in row order
             const uint32_t r0 = item.chunk * kPrepRows;
             const uint32_t nr = min(kPrepRows, x - r0);
             const T* __restrict__ pp = static_cast<const T*>(I->part_ipk);
             T* __restrict__ psia = static_cast<T*>(I->psia);
             const size_t stride = (size_t)x * z;
-            for (uint32_t k = tid; k < z; k += 256) {
-                SumAcc<T> A;
-                for (uint32_t r = 0; r < nr; ++r) {
+            for (uint32_t k0 = blockIdx.y * kPrepDeep; k0 < z; k0 += gridDim.y * kPrepDeep) {
+                for (uint32_t e = tid; e < nr * kPrepDeep; e += 256) {
+                    const uint32_t r = e / kPrepDeep, k = k0 + e % kPrepDeep;
+                    if (k >= z) continue;
                     const size_t idx = (size_t)(r0 + r) * z + k;
                     SumAcc<T> s;
                     add_strided(s, pp + idx, stride, I->n_tj);
@@ -550,10 +561,16 @@ __global__ void __launch_bounds__(256)
                     } else {
                         const T alpha_eph = s.get() + static_cast<T>(I->alpha[r0 + r]);
                         psia[idx] = psi_sel<PSI, T>(alpha_eph);
-                        A.add(alpha_eph);
+                        aeph[e] = alpha_eph;
                     }
                 }
-                if constexpr (!RAW) static_cast<T*>(I->partA)[(size_t)item.chunk * z + k] = A.get();
+                __syncthreads();
+                if (!RAW && tid < kPrepDeep && k0 + tid < z) {
+                    SumAcc<T> A;
+                    for (uint32_t r = 0; r < nr; ++r) A.add(aeph[r * kPrepDeep + tid]);
+                    static_cast<T*>(I->partA)[(size_t)item.chunk * z + k0 + tid] = A.get();
+                }
+                __syncthreads();
             }
         } else {
             const uint32_t r0 = item.chunk * kPrepRows;
@@ -893,7 +910,8 @@ void read_layout(int dtype, uint32_t z, uint32_t* rw, uint32_t* hs, uint32_t* hm
 
 hipError_t launch_prep(int dtype, int psi, bool raw, dim3 grid, hipStream_t st,
                        const BldInst* insts, const PrepItem* items, const uint32_t* n_items,
-                       uint32_t n_inst) {
+                       uint32_t n_inst, uint32_t zmax) {
+    if (zmax > kFusedZ) grid.y = zmax >= kPrepDeep * kPrepDeepParts ? kPrepDeepParts : (zmax + kPrepDeep - 1) / kPrepDeep;
     const dim3 gA(n_inst < 65535u ? (n_inst ? n_inst : 1u) : 65535u);
     if (dtype == 0) {
         if (raw) {

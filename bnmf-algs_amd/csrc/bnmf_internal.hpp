@@ -49,7 +49,7 @@ void read_layout(int dtype, uint32_t z, uint32_t* rw, uint32_t* hs, uint32_t* hm
 // descriptors
 hipError_t launch_prep(int dtype, int psi, bool raw, dim3 grid, hipStream_t st,
                        const BldInst* insts, const PrepItem* items, const uint32_t* n_items,
-                       uint32_t n_inst);
+                       uint32_t n_inst, uint32_t zmax);
 hipError_t launch_score(dim3 grid, hipStream_t st, const BldInst* insts, const PrepItem* items,
                         const uint32_t* n_items, uint32_t n_inst);
 hipError_t launch_psi_eval(int kind, const double* xin, double* out, size_t n, hipStream_t st);
@@ -360,13 +360,13 @@ class Batch {
     mutable HostStage stage_;
     size_t off_desc_first_ = 0, off_desc_ = 0, off_prep_items_ = 0, off_prep_count_ = 0;
     size_t off_iter_ = 0;  // additive solver: uint32 iteration counters, one per instance
-    uint32_t n_prep_items_ = 0;
+    uint32_t n_prep_items_ = 0, zmax_ = 0;
     std::vector<Bucket> groups_[2];
     // per stream: descriptor arrays of the instances of its update groups
     // (the groups' pass items index them), its prep work list
     struct Lane {
         size_t off_desc = 0, off_desc_first = 0, off_prep = 0, off_prep_count = 0;
-        uint32_t n_prep = 0, n_inst = 0;
+        uint32_t n_prep = 0, n_inst = 0, zmax = 0;
     };
     std::vector<Lane> lanes_;
     hipStream_t stream_ = nullptr;
@@ -447,7 +447,7 @@ class ApprBatch {
     // work lists over the nonempty entries: both sides (sums), rows, columns
     DeviceBuffer lists_;
     size_t off_live_ = 0, off_lrow_ = 0, off_lcol_ = 0, off_al_ = 0;
-    uint32_t zmax_live_ = 0, n_live_ = 0, n_lrow_ = 0, n_lcol_ = 0;
+    uint32_t zmax_dense_ = 0, zmax_live_ = 0, n_live_ = 0, n_lrow_ = 0, n_lcol_ = 0;
     hipStream_t stream_ = nullptr;
     hipStream_t side_ = nullptr;  // the listed instances' branch of a graph
     hipEvent_t fork_ = nullptr, join_ = nullptr;

@@ -214,7 +214,7 @@ void bld_mult_f32_noalloc(const float* X, uint32_t x, uint32_t y, uint32_t z, co
     BNMF_HIP(launch_pass_key(k_sums, BNMF_F32, PSIM_F32, MODE_SUMS, dim3(n_items), st, dfirst_dev, items,
                              counts + CNT_ITEMS, z));
     for (size_t t = 0; t < max_iter; ++t) {
-        BNMF_HIP(launch_prep(BNMF_F32, PSIM_F32, false, dim3(n_prep), st, dmain_dev, prep, counts + CNT_PREP, 1));
+        BNMF_HIP(launch_prep(BNMF_F32, PSIM_F32, false, dim3(n_prep), st, dmain_dev, prep, counts + CNT_PREP, 1, z));
         const BldInst* dp = t == 0 ? dfirst_dev : dmain_dev;
         if (split) {
             BNMF_HIP(launch_pass_key(k_exact, BNMF_F32, PSIM_F32, MODE_UPDATE, dim3(n_items), st, dp, items,

@@ -244,7 +244,7 @@ class Server {
     // index it), so each stream can iterate on its own.
     struct LaneWS {
         size_t off_desc = 0, off_prep = 0, off_prep_count = 0;
-        uint32_t n_prep = 0, n_inst = 0;
+        uint32_t n_prep = 0, n_inst = 0, zmax = 0;
     };
     struct WorkSet {
         std::vector<Launch> launches;
@@ -397,6 +397,7 @@ class Server {
                 for (uint32_t loc = 0; loc < (uint32_t)lane_members[ln].size(); ++loc) {
                     const uint32_t n = lane_members[ln][loc];
                     ld.push_back(desc[n]);
+                    lw.zmax = std::max(lw.zmax, set[n]->L.z);
                     const InstLayout& L = set[n]->L;
                     for (uint32_t c = 0; c < L.n_cj; ++c) lp.push_back(PrepItem{loc, 0, c, 0});
                     for (uint32_t c = 0; c < L.nA; ++c) lp.push_back(PrepItem{loc, 1, c, 0});
@@ -462,7 +463,7 @@ class Server {
                 const BldInst* d = reinterpret_cast<const BldInst*>(m + lw.off_desc);
                 BNMF_HIP(launch_prep(dtype_, psi_, false, dim3(lw.n_prep), st, d,
                                      reinterpret_cast<const PrepItem*>(m + lw.off_prep),
-                                     reinterpret_cast<const uint32_t*>(m + lw.off_prep_count), lw.n_inst));
+                                     reinterpret_cast<const uint32_t*>(m + lw.off_prep_count), lw.n_inst, lw.zmax));
                 for (const Launch& ln : ws.launches) {
                     if (ln.lane != l) continue;
                     BNMF_HIP(launch_pass_key(ln.key, dtype_, psi_, MODE_UPDATE, dim3(ln.n), st, d,

@@ -314,6 +314,24 @@ static void scan_S0(const T* S0, const T* X, size_t xy, size_t z, bool* nonneg, 
     *packable = nn && pk;
 }
 
+void classify(int dtype, const InstSpec& s, double eps, bool* nonneg, bool* packable) {
+    const size_t xy = (size_t)s.x * s.y;
+    bool nn = true;
+    for (uint32_t k = 0; k < s.z; ++k) nn = nn && s.beta[k] >= 1.0;
+    bool pk = nn && xy > 0 && s.z <= kFusedZ && !(dtype == BNMF_F32 && generic_steps()) && eps >= 1e-200 && eps <= 1.0 &&
+              LivePlan::worth(dtype, s.X, xy);
+    for (uint32_t i = 0; i < s.x; ++i) pk = pk && s.alpha[i] >= 1e-6 && s.alpha[i] <= 1e30;
+    for (uint32_t k = 0; k < s.z; ++k) pk = pk && s.beta[k] <= 1e30;
+    if (nn && s.S0) {
+        if (dtype == BNMF_F32)
+            scan_S0(static_cast<const float*>(s.S0), static_cast<const float*>(s.X), xy, s.z, &nn, &pk);
+        else
+            scan_S0(static_cast<const double*>(s.S0), static_cast<const double*>(s.X), xy, s.z, &nn, &pk);
+    }
+    *nonneg = nn;
+    *packable = nn && pk;
+}
+
 // ------------------------------------------------------------------ batch
 Batch::Batch(int dtype, int psi_mode, double eps, const std::vector<InstSpec>& specs, int algo)
     : dtype_(dtype), psi_(psi_mode), algo_(algo), eps_(eps), es_(dtype == BNMF_F32 ? 4 : 8), specs_(specs) {
@@ -382,20 +400,10 @@ Batch::Batch(int dtype, int psi_mode, double eps, const std::vector<InstSpec>& s
         BNMF_HIP(hipMemcpy(b + L.off_alpha, s.alpha, (size_t)s.x * 8, hipMemcpyHostToDevice));
         BNMF_HIP(hipMemcpy(b + L.off_beta, s.beta, (size_t)s.z * 8, hipMemcpyHostToDevice));
         const void* S0 = s.S0;
-        bool nn = true;
-        for (uint32_t k = 0; k < s.z; ++k) nn = nn && s.beta[k] >= 1.0;
-        bool pk = nn && s.z <= kFusedZ && !(dtype == BNMF_F32 && generic_steps()) && eps >= 1e-200 && eps <= 1.0 &&
-                  LivePlan::worth(dtype, s.X, xy);
-        for (uint32_t i = 0; i < s.x; ++i) pk = pk && s.alpha[i] >= 1e-6 && s.alpha[i] <= 1e30;
-        for (uint32_t k = 0; k < s.z; ++k) pk = pk && s.beta[k] <= 1e30;
-        if (nn && s.S0) {
-            if (dtype == BNMF_F32)
-                scan_S0(static_cast<const float*>(S0), static_cast<const float*>(s.X), xy, s.z, &nn, &pk);
-            else
-                scan_S0(static_cast<const double*>(S0), static_cast<const double*>(s.X), xy, s.z, &nn, &pk);
-        }
+        bool nn = true, pk = true;
+        classify(dtype, s, eps, &nn, &pk);
         nonneg[n] = nn;
-        packable[n] = nn && pk;
+        packable[n] = pk;
         if (S0) {
             BNMF_HIP(hipMemcpy(b + L.off_S0, S0, xyz * es_, hipMemcpyHostToDevice));
         } else {

@@ -5,6 +5,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <functional>
 #include <mutex>
 #include <stdexcept>
 #include <string>
@@ -239,15 +240,22 @@ hipError_t launch_pass_key(const PassKey& k, int dtype, int psi, int mode, dim3 
                            hipStream_t st, const BldInst* insts, const PassItem* items,
                            const uint32_t* n_items, uint32_t zmax);
 
+// nonneg: S stays >= 0 (S0 >= 0 and beta >= 1). packable: additionally every
+// gradient of its solve is finite, so that a fiber with X_ij = 0 stays exactly
+// zero, and X looks sparse enough (LivePlan).
+void classify(int dtype, const InstSpec& s, double eps, bool* nonneg, bool* packable);
+
 // Which instances of a batch keep their nonempty fibers packed, and where
 // (live.cpp). Results do not depend on it.
 class LivePlan {
    public:
     // Counts the nonempty fibers of the candidates' tiles (X and the tile
     // plan from the descriptors) and lays the packed buffers out.
-    // scratch: device memory of scratch_bytes, used until the call returns.
+    // scratch: device memory of scratch_bytes, used until the call returns; it
+    // starts with the descriptors. mem: where the packed buffers come from and
+    // are given back to (null for none left); without it they are the plan's own.
     LivePlan(int dtype, const std::vector<BldInst>& descs, const std::vector<InstLayout>& lay,
-             const std::vector<bool>& candidate, char* scratch);
+             const std::vector<bool>& candidate, char* scratch, const std::function<void*(size_t)>& mem = nullptr);
     LivePlan() = default;
     static size_t scratch_bytes(const std::vector<InstLayout>& lay);
     // Largest share of nonempty fibers at which an instance is packed. The packed
@@ -260,7 +268,8 @@ class LivePlan {
     bool live(size_t n) const { return n < lds_.size() && lds_[n] > 0; }
     uint32_t lds(size_t n) const { return lds_[n]; }
     size_t fibers(size_t n) const { return fibers_[n]; }  // its nonempty fibers
-    size_t bytes() const { return buf_.bytes; }
+    size_t bytes() const { return bytes_; }
+    uint32_t n_tiles() const { return (uint32_t)tiles_.size(); }
     // Appends the tiles of one launch (items: batch instance numbers) to the
     // tile table and returns the first one's index.
     uint32_t add_launch(std::vector<PassItem>& items, const std::vector<BldInst>& descs);
@@ -276,7 +285,13 @@ class LivePlan {
     struct Off {
         size_t Sc, fib, xv, rdesc, cdesc, map, smap, tile0;
     };
+    template <typename T>
+    T* at(size_t off) const {
+        return reinterpret_cast<T*>(base_ + off);
+    }
     int dtype_ = 0;
+    char* base_ = nullptr;
+    size_t bytes_ = 0;
     DeviceBuffer buf_, tab_;
     std::vector<Off> offs_;
     std::vector<size_t> fibers_;

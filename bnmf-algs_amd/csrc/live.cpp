@@ -46,7 +46,7 @@ bool LivePlan::worth(int dtype, const void* X, size_t n, double most) {
 }
 
 LivePlan::LivePlan(int dtype, const std::vector<BldInst>& descs, const std::vector<InstLayout>& lay,
-                   const std::vector<bool>& candidate, char* scratch)
+                   const std::vector<bool>& candidate, char* scratch, const std::function<void*(size_t)>& mem)
     : dtype_(dtype), offs_(descs.size()), fibers_(descs.size(), 0), lds_(descs.size(), 0) {
     const size_t es = dtype == BNMF_F32 ? 4 : 8;
     // nonempty fibers of every candidate's tiles
@@ -120,17 +120,24 @@ LivePlan::LivePlan(int dtype, const std::vector<BldInst>& descs, const std::vect
     // the packed form is extra memory: without room for it every instance
     // runs the dense passes, with the same results
     {
-        void* p = nullptr;
-        if (hipMalloc(&p, off) != hipSuccess) {
+        void* p = mem ? mem(off) : nullptr;
+        if (!mem && hipMalloc(&p, off) != hipSuccess) {
             (void)hipGetLastError();
+            p = nullptr;
+        }
+        if (!p) {
             std::fill(lds_.begin(), lds_.end(), 0u);
             return;
         }
-        buf_.ptr = p;
-        buf_.bytes = off;
+        base_ = static_cast<char*>(p);
+        bytes_ = off;
+        if (!mem) {
+            buf_.ptr = p;
+            buf_.bytes = off;
+        }
     }
     // slots past a tile's fibers are read as zeros
-    BNMF_HIP(hipMemset(buf_.ptr, 0, off));
+    BNMF_HIP(hipMemset(base_, 0, off));
 }
 
 uint32_t LivePlan::add_launch(std::vector<PassItem>& items, const std::vector<BldInst>& descs) {
@@ -152,13 +159,13 @@ uint32_t LivePlan::add_launch(std::vector<PassItem>& items, const std::vector<Bl
         uint32_t ge = 0, gf = 0;
         live_group(dtype_, d.z, &ge, &gf);
         LiveTile t{};
-        t.Sc = buf_.as<char>(o.Sc + slot / gf * ge * es);
-        t.fib = buf_.as<uint16_t>(o.fib) + slot;
-        t.xv = buf_.as<char>(o.xv + slot * es);
-        t.rdesc = buf_.as<LiveRow>(o.rdesc) + tile * d.ti_rows;
-        t.cdesc = buf_.as<LiveCol>(o.cdesc) + tile * d.tile_cols;
-        t.map = buf_.as<uint16_t>(o.map) + tile * d.ti_rows * d.tile_cols;
-        t.smap = buf_.as<uint16_t>(o.smap) + tile * d.ti_rows * d.tile_cols;
+        t.Sc = at<char>(o.Sc + slot / gf * ge * es);
+        t.fib = at<uint16_t>(o.fib) + slot;
+        t.xv = at<char>(o.xv + slot * es);
+        t.rdesc = at<LiveRow>(o.rdesc) + tile * d.ti_rows;
+        t.cdesc = at<LiveCol>(o.cdesc) + tile * d.tile_cols;
+        t.map = at<uint16_t>(o.map) + tile * d.ti_rows * d.tile_cols;
+        t.smap = at<uint16_t>(o.smap) + tile * d.ti_rows * d.tile_cols;
         t.psib = static_cast<const char*>(d.psib) + j0 * z * es;
         t.psia = static_cast<const char*>(d.psia) + i0 * z * es;
         t.psiA = d.psiA;

@@ -55,7 +55,10 @@ struct Request {
     double a = 1, b = 1;
     uint64_t seed = 0;
     bool has_S0 = false, want_lm = false;
-    bool nonneg = false;  // S0 >= 0 and beta >= 1: S stays >= 0
+    bool nonneg = false, packable = false;  // classify
+    // its packed nonempty fibers while it is active, in arena bytes of their own
+    LivePlan live;
+    size_t live_off = 0, live_bytes = 0;
     size_t max_iter = 0, done_iter = 0;
     InstLayout L{};
     size_t off = 0;
@@ -130,16 +133,19 @@ class Server {
         r->a = d.a;
         r->b = d.b;
         r->seed = d.seed;
-        bool nn = true;
-        for (size_t k = 0; k < d.z; ++k) nn = nn && d.beta[k] >= 1.0;
         if (d.S0) {
             r->has_S0 = true;
             r->S0.assign(static_cast<const char*>(d.S0), static_cast<const char*>(d.S0) + xyz * es_);
-            for (size_t t = 0; t < xyz && nn; ++t)
-                nn = dtype_ == BNMF_F32 ? static_cast<const float*>(d.S0)[t] >= 0.0f
-                                        : static_cast<const double*>(d.S0)[t] >= 0.0;
         }
-        r->nonneg = nn;
+        InstSpec s;
+        s.x = r->x;
+        s.y = r->y;
+        s.z = r->z;
+        s.X = r->X.data();
+        s.S0 = d.S0 ? r->S0.data() : nullptr;
+        s.alpha = d.alpha;
+        s.beta = d.beta;
+        classify(dtype_, s, eps_, &r->nonneg, &r->packable);
         r->want_lm = want_lm != 0;
         r->max_iter = max_iter;
         r->L = plan_instance(dtype_, r->x, r->y, r->z, false);
@@ -237,6 +243,7 @@ class Server {
         int lane;
         uint32_t zmax, n;
         size_t off_items, off_count, work;
+        uint32_t lds = 0;  // packed fibers: dynamic LDS; items are LiveTile
     };
     // Device-side work lists for a set of instances.
     // Update work sets also keep, per stream, a descriptor array and prep
@@ -251,6 +258,8 @@ class Server {
         size_t off_desc = 0, off_prep = 0, off_prep_count = 0;
         uint32_t n_prep = 0, n_inst = 0;
         LaneWS lanes[4];
+        // the packed requests' tiles within the work lists
+        std::vector<std::pair<size_t, const Request*>> tiles;
     };
 
     void loop() {
@@ -317,6 +326,34 @@ class Server {
         r.X.shrink_to_fit();
         r.S0.clear();
         r.S0.shrink_to_fit();
+        if (r.packable) pack(r);
+    }
+
+    // The nonempty fibers' lists, in arena memory that no queued request waits for
+    // (only the tile table, some 150 bytes a tile, lies outside);
+    // without it the request runs the dense passes, with the same results.
+    void pack(Request& r) {
+        const std::vector<InstLayout> lay{r.L};
+        const std::vector<BldInst> desc{make_desc(r.L, dev_buf_.as<char>(r.off), eps_, r.a, r.b, false, r.nonneg)};
+        const size_t need = LivePlan::scratch_bytes(lay);
+        if (scratch_.bytes < need) scratch_ = DeviceBuffer(need);
+        r.live = LivePlan(dtype_, desc, lay, {true}, scratch_.as<char>(), [&](size_t n) -> void* {
+            std::lock_guard<std::mutex> lk(mu_);
+            size_t waiting = 0;
+            for (const auto& q : queue_) waiting += align_up(q->L.bytes);
+            if (arena_.used() + waiting + align_up(n) > arena_.capacity() || !arena_.alloc(align_up(n), &r.live_off))
+                return nullptr;
+            r.live_bytes = align_up(n);
+            peak_bytes_ = std::max(peak_bytes_, arena_.used());
+            return dev_buf_.as<char>(r.live_off);
+        });
+        if (!r.live.live(0)) return;
+        std::vector<PassItem> items;
+        for (uint32_t ti = 0; ti < r.L.n_ti; ++ti)
+            for (uint32_t tj = 0; tj < r.L.n_tj; ++tj) items.push_back(PassItem{0, ti, tj, 0});
+        r.live.add_launch(items, desc);
+        r.live.build(desc, scratch_.as<BldInst>(), stream_);
+        BNMF_HIP(hipStreamSynchronize(stream_));
     }
 
 
@@ -341,10 +378,11 @@ class Server {
             BldInst d = make_desc(L, dev_buf_.as<char>(r.off), eps_, r.a, r.b, false, r.nonneg);
             desc.push_back(d);
             if (L.elements() == 0) continue;
-            const PassKey key = pass_key(dtype_, mode, L, r.nonneg);
+            const PassKey key = pass_key(dtype_, mode, L, r.nonneg, r.live.live(0));
             zmax[key] = std::max(zmax[key], L.z);
             members[key].push_back((uint32_t)n);
-            work[key] += L.elements();
+            // a packed element costs about three streamed ones
+            work[key] += key.live ? 3 * r.live.fibers(0) * L.z : L.elements();
             for (uint32_t c = 0; c < L.n_cj; ++c) prep.push_back(PrepItem{(uint32_t)n, 0, c, 0});
             for (uint32_t c = 0; c < L.nA; ++c) prep.push_back(PrepItem{(uint32_t)n, 1, c, 0});
         }
@@ -372,6 +410,7 @@ class Server {
             l.lane = (int)(std::min_element(load.begin(), load.end()) - load.begin());
             load[l.lane] += l.work;
             std::vector<PassItem> items;
+            uint32_t tiles = 0;
             for (uint32_t n : members[o.second]) {
                 uint32_t idx = n;
                 if (per_lane) {
@@ -379,8 +418,26 @@ class Server {
                     lane_members[l.lane].push_back(n);
                 }
                 const InstLayout& L = set[n]->L;
+                if (l.key.live) {
+                    tiles += set[n]->live.n_tiles();
+                    l.lds = std::max(l.lds, set[n]->live.lds(0));
+                    continue;
+                }
                 for (uint32_t ti = 0; ti < L.n_ti; ++ti)
                     for (uint32_t tj = 0; tj < L.n_tj; ++tj) items.push_back(PassItem{idx, ti, tj, 0});
+            }
+            if (l.key.live) {
+                // one launch for the packed requests, whose tiles are gathered
+                // on the device
+                l.n = tiles;
+                l.off_items = take(tiles * sizeof(LiveTile));
+                size_t at = l.off_items;
+                for (uint32_t n : members[o.second]) {
+                    ws.tiles.push_back({at, set[n]});
+                    at += set[n]->live.n_tiles() * sizeof(LiveTile);
+                }
+                ws.launches.push_back(l);
+                continue;
             }
             l.n = (uint32_t)items.size();
             l.off_items = take(items.size() * sizeof(PassItem));
@@ -466,6 +523,11 @@ class Server {
                                      reinterpret_cast<const uint32_t*>(m + lw.off_prep_count), lw.n_inst, lw.zmax));
                 for (const Launch& ln : ws.launches) {
                     if (ln.lane != l) continue;
+                    if (ln.key.live) {
+                        BNMF_HIP(launch_pass_live(dtype_, psi_, MODE_UPDATE, ln.key.live == 2, ln.n, st,
+                                                  reinterpret_cast<const LiveTile*>(m + ln.off_items), ln.lds));
+                        continue;
+                    }
                     BNMF_HIP(launch_pass_key(ln.key, dtype_, psi_, MODE_UPDATE, dim3(ln.n), st, d,
                                              reinterpret_cast<const PassItem*>(m + ln.off_items),
                                              reinterpret_cast<const uint32_t*>(m + ln.off_count), ln.zmax));
@@ -496,8 +558,16 @@ class Server {
         ensure_meta(end);
         BNMF_HIP(hipMemcpyAsync(meta_.ptr, host.data(), end, hipMemcpyHostToDevice, stream_));
         char* m = meta_.as<char>();
+        for (const auto& t : ws_all.tiles)
+            BNMF_HIP(hipMemcpyAsync(m + t.first, t.second->live.tiles(), t.second->live.n_tiles() * sizeof(LiveTile),
+                                    hipMemcpyDeviceToDevice, stream_));
+        const BldInst* desc = reinterpret_cast<const BldInst*>(m + ws_all.off_desc);
         if (!fresh.empty()) passes(ws_fresh, MODE_SUMS);
+        for (size_t n = 0; n < all.size(); ++n)
+            if (all[n]->fresh) all[n]->live.gather(desc + n, stream_);
         iterate(ws_all, k_iters);
+        for (size_t n = 0; n < all.size(); ++n)
+            if (all[n]->done_iter + k_iters >= all[n]->max_iter) all[n]->live.scatter(desc + n, stream_);
         // requests that finish in this step, scored if asked
         std::vector<Request*> fin, score;
         for (Request* r : all) {
@@ -535,6 +605,7 @@ class Server {
         }
         BNMF_HIP(hipStreamSynchronize(stream_));
         const double t1 = now_s();
+        for (Request* r : fin) r->live = LivePlan();
         std::lock_guard<std::mutex> lk(mu_);
         busy_s_ += t1 - t0;
         ++steps_;
@@ -543,6 +614,8 @@ class Server {
             for (Request* r : fin) {
                 r->state = RS_DONE;
                 r->t_done = t1;
+                if (r->live_bytes) arena_.release(r->live_off, r->live_bytes);
+                r->live_bytes = 0;
                 ++completed_;
             }
             active_.erase(std::remove_if(active_.begin(), active_.end(),
@@ -577,7 +650,7 @@ class Server {
     size_t max_chunk_ = 8;  // iterations per scheduling step
     int dev_ = 0;
     Arena arena_;
-    DeviceBuffer dev_buf_, meta_;
+    DeviceBuffer dev_buf_, meta_, scratch_;
     HostStage stage_;
     hipStream_t stream_ = nullptr;
     std::vector<hipStream_t> side_;

@@ -62,38 +62,20 @@ uint32_t zq_of(uint32_t z) {
 uint32_t list_waves(size_t entries, uint32_t lists, uint32_t z) {
     return (double)entries * zq_of(z) > 768.0 * lists ? 4u : 1u;
 }
-// Largest share of nonempty entries at which an instance runs over them
+// Largest share of nonempty entries at which an FP64 instance runs over them
 // (bld_appr_live.hip), where lanes past z count as work too. Measured per
 // iteration, lists against dense passes: 1024x1024x32 131 us against 975 at a
 // share of 0.1 and 856 against 1000 full; 64 of 200x200x17 (17 of 32 lanes in
 // use) 1072 against 1520 at 0.5 and 1865 against 1529 full; 64 of 400x40x10, 282
 // against 405 and 459 against 419. An instance so small that its launches are
 // all latency takes the lists always (8x10x3: 24 against 40).
-// FP32 compares with dense passes three times as fast, and is for short fibers
-// soon at their launches' latency: per iteration, 384x384x32 80 us against 284 at
-// 0.3, sixteen of them 538 against 575; 64 of 200x200x17, 219 against 396 at 0.08
-// and 376 at 0.15; of 400x40x10, 103 against 149 at 0.08 and 178 at 0.3; of 64x64x8,
-// 90 against 59 at 0.27; 8 of 512x512x64, 864 against 2045 at 0.3, of 512x512x36
-// 861 against 852. A batch of both kinds pays both launches' latency, side by side.
-double live_share(int dtype, size_t x, size_t y, uint32_t z) {
-    if (x * y * zq_of(z) <= 8192) return 1.0;
-    return (dtype == BNMF_F64 ? 0.9 : z <= 16 ? 0.1 : z <= 32 ? 0.28 : 0.4) * z / zq_of(z);
-}
-// Is the longest list (rows, then columns) short enough for the block that is
-// left to walk it, where the dense passes would spread it over the chip? FP64,
-// entries times lanes per entry: 20000x100x20, 633 us against 1725 at lists of
-// 2000; at 6000 both would take about 1750. FP32, with dense passes that
-// take 628 us there, per wavefront of the list, whose step of 64 elements costs
-// 2.2 us an iteration: 384x384x32 with a full row and column 473 us against 284,
-// 1024x1024x32 so 1105 against 311.
-bool lists_fit(int dtype, const uint32_t longest[2], size_t entries, uint32_t x, uint32_t y, uint32_t z) {
-    const double elements = (double)x * y * z, r = (double)longest[0] * zq_of(z), c = (double)longest[1] * zq_of(z);
-    if (dtype == BNMF_F64) return std::max(r, c) <= std::max(65536.0, elements / 256.0);
-    return std::max(r / list_waves(entries, x, z), c / list_waves(entries, y, z)) <= std::max(4096.0, elements / 4096.0);
-}
+double live_share(size_t x, size_t y, uint32_t z) { return x * y * zq_of(z) <= 8192 ? 1.0 : 0.9 * z / zq_of(z); }
+// Longest list (entries times lanes per entry) that one block may be left to
+// walk where the dense passes would spread it over the chip: 20000x100x20, 633 us
+// against 1725 at lists of 2000; at 6000 both would take about 1750.
+double list_budget(double elements) { return std::max(65536.0, elements / 256.0); }
 
-template <typename T>
-bool within(const T* p, size_t n, double lo, double hi) {
+bool within(const double* p, size_t n, double lo, double hi) {
     for (size_t t = 0; t < n; ++t)
         if (!(p[t] >= lo && p[t] <= hi)) return false;
     return true;
@@ -103,33 +85,26 @@ bool within(const T* p, size_t n, double lo, double hi) {
 // May the instance run over its nonempty entries only? An empty one then has
 // to contribute exactly 0, so the gradients it multiplies must be finite:
 // parameters, eps and starting factors of ordinary size. Whatever else the
-// caller gives takes the dense passes. An FP32 instance is iterated in double:
-// in FP32 a solve carries rounding errors of up to 1e-5 after 200 iterations,
-// which sums taken in another order would replace by others as large.
+// caller gives takes the dense passes, and so does FP32: its solves carry
+// rounding errors of up to 1e-5 after 200 iterations, which sums taken in
+// another order, or in double, would replace by other results.
 bool ApprBatch::live_candidate(const ApprSpec& s, double eps) const {
     const size_t x = s.x, y = s.y, z = s.z;
-    if (z > kFusedZ || x * y == 0 || x * y > 0xffffffffull) return false;
+    if (dtype_ != BNMF_F64 || z > kFusedZ || x * y == 0 || x * y > 0xffffffffull) return false;
     if (!(eps >= 1e-200 && eps <= 1.0)) return false;
     if (!within(s.alpha, x, 1e-6, 1e30) || !within(s.beta, z, 1e-6, 1e30)) return false;
-    auto tame = [&](const void* p, size_t n) {
-        return !p || (dtype_ == BNMF_F32 ? within(static_cast<const float*>(p), n, 0.0, 1e100)
-                                         : within(static_cast<const double*>(p), n, 0.0, 1e100));
-    };
-    return tame(s.nu0, x * z) && tame(s.mu0, z * y) && LivePlan::worth(dtype_, s.X, x * y, live_share(dtype_, x, y, s.z));
+    auto tame = [](const void* p, size_t n) { return !p || within(static_cast<const double*>(p), n, 0.0, 1e100); };
+    return tame(s.nu0, x * z) && tame(s.mu0, z * y) && LivePlan::worth(dtype_, s.X, x * y, live_share(x, y, s.z));
 }
 
 // The lists of the instances that are sparse enough, in one allocation; none
-// if it cannot be had. counts: (x + y) words per candidate, in order. al: the
-// descriptors ai as the lists' kernels read them.
-void ApprBatch::plan_live(uint32_t* counts, const std::vector<ApprInst>& ai, std::vector<ApprInst>& al,
-                          std::vector<BldInst>& bi) {
+// if it cannot be had. counts: (x + y) words per candidate, in order.
+void ApprBatch::plan_live(uint32_t* counts, std::vector<ApprInst>& ai, std::vector<BldInst>& bi) {
     char* const base = arena_.as<char>();
-    const int dt = dtype_ == BNMF_F32 ? 0 : 1;
-    al = ai;
     size_t total = 0;
     for (const L_& l : lay_)
         if (l.live) {
-            BNMF_HIP(launch_appr_count(dt, base + l.off_X, l.x, l.y, counts + total, nullptr));
+            BNMF_HIP(launch_appr_count(arena_.as<double>(l.off_X), l.x, l.y, counts + total, nullptr));
             total += (size_t)l.x + l.y;
         }
     if (total == 0) return;
@@ -145,15 +120,15 @@ void ApprBatch::plan_live(uint32_t* counts, const std::vector<ApprInst>& ai, std
         const uint32_t* const c = cnt.data() + at;
         at += (size_t)l.x + l.y;
         size_t entries = 0;
-        uint32_t longest[2] = {0, 0};
+        uint32_t longest = 0;
         bool bad = false;
         for (size_t i = 0; i < (size_t)l.x + l.y; ++i) {
             bad = bad || c[i] == ~0u;
-            longest[i >= l.x] = std::max(longest[i >= l.x], c[i]);
+            longest = std::max(longest, c[i]);
             if (i < l.x) entries += c[i];
         }
-        l.live = !bad && (double)entries <= live_share(dtype_, l.x, l.y, l.z) * (double)l.x * (double)l.y &&
-                 lists_fit(dtype_, longest, entries, l.x, l.y, l.z);
+        l.live = !bad && (double)entries <= live_share(l.x, l.y, l.z) * (double)l.x * (double)l.y &&
+                 (double)longest * zq_of(l.z) <= list_budget((double)l.x * l.y * l.z);
         if (!l.live) continue;
         l.entries = entries;
         off_ptr[n] = ptr.size();
@@ -171,9 +146,6 @@ void ApprBatch::plan_live(uint32_t* counts, const std::vector<ApprInst>& ai, std
         ptr.push_back(sum);
         off_ent[n] = ent_bytes;
         ent_bytes += 2 * (align_up(entries * 4 + 4) + align_up(entries * 8 + 8));
-        // an FP32 instance's factors, psi and block sums in double
-        if (dt == 0)
-            ent_bytes += 3 * align_up((size_t)l.x * l.z * 8) + 2 * align_up((size_t)l.y * l.z * 8) + align_up((size_t)l.z * 8);
     }
     if (ptr.empty()) return;
     const size_t ptr_bytes = align_up(ptr.size() * 4);
@@ -187,7 +159,7 @@ void ApprBatch::plan_live(uint32_t* counts, const std::vector<ApprInst>& ai, std
     lists_.bytes = ptr_bytes + ent_bytes;
     BNMF_HIP(hipMemcpy(p, ptr.data(), ptr.size() * 4, hipMemcpyHostToDevice));
     for (size_t n = 0; n < lay_.size(); ++n) {
-        L_& l = lay_[n];
+        const L_& l = lay_[n];
         if (!l.live) continue;
         const size_t oi = align_up(l.entries * 4 + 4), ox = align_up(l.entries * 8 + 8);
         const uint32_t* const rptr = lists_.as<uint32_t>(off_ptr[n] * 4);
@@ -197,34 +169,17 @@ void ApprBatch::plan_live(uint32_t* counts, const std::vector<ApprInst>& ai, std
         uint32_t* const cidx = reinterpret_cast<uint32_t*>(e + oi);
         double* const rxv = reinterpret_cast<double*>(e + 2 * oi);
         double* const cxv = reinterpret_cast<double*>(e + 2 * oi + ox);
-        BNMF_HIP(launch_appr_fill(dt, base + l.off_X, l.x, l.y, rptr, ridx, rxv, cptr, cidx, cxv, nullptr));
-        ApprInst& a = al[n];
+        BNMF_HIP(launch_appr_fill(arena_.as<double>(l.off_X), l.x, l.y, rptr, ridx, rxv, cptr, cidx, cxv, nullptr));
+        ApprInst& a = ai[n];
         a.rptr = rptr;
         a.ridx = ridx;
         a.rxv = rxv;
         a.cptr = cptr;
         a.cidx = cidx;
         a.cxv = cxv;
-        if (dt == 0) {
-            char* d = e + 2 * (oi + ox);
-            auto take = [&](size_t doubles) {
-                char* const at = d;
-                d += align_up(doubles * 8);
-                return at;
-            };
-            a.nu = take((size_t)l.x * l.z);
-            a.psia = take((size_t)l.x * l.z);
-            a.partA = take((size_t)l.x * l.z);
-            a.muT = take((size_t)l.y * l.z);
-            a.psib = take((size_t)l.y * l.z);
-            a.psiA = take(l.z);
-        } else {
-            // the dense passes' second partials are free: y*z and x*z at least
-            a.muT = base + l.off_pjk2;
-            a.partA = base + l.off_ipk2;
-        }
-        l.nu_d = static_cast<double*>(a.nu);
-        l.muT_d = static_cast<double*>(a.muT);
+        // the dense passes' second partials are free: y*z and x*z at least
+        a.muT = base + l.off_pjk2;
+        a.partA = base + l.off_ipk2;
         a.nA = ceil_div(l.x, 4u / list_waves(l.entries, l.x, l.z));
         zmax_live_ = std::max(zmax_live_, l.z);
         // left out of the dense instances' psi(A)
@@ -379,8 +334,7 @@ ApprBatch::ApprBatch(int dtype, double eps, const std::vector<ApprSpec>& specs)
         d.zq_log2 = lg;
         bi.push_back(d);
     }
-    std::vector<ApprInst> al;
-    plan_live(arena_.as<uint32_t>(total), ai, al, bi);
+    plan_live(arena_.as<uint32_t>(total), ai, bi);
 
     // work lists: pass items by z bucket, prep items, factor items
     std::map<uint32_t, std::vector<PassItem>> by_zb;
@@ -423,7 +377,6 @@ ApprBatch::ApprBatch(int dtype, double eps, const std::vector<ApprSpec>& specs)
     off_lrow_ = mtake(lrow.size() * sizeof(PassItem));
     off_lcol_ = mtake(lcol.size() * sizeof(PassItem));
     off_ai_ = mtake(ai.size() * sizeof(ApprInst));
-    off_al_ = mtake(al.size() * sizeof(ApprInst));
     off_bi_ = mtake(bi.size() * sizeof(BldInst));
     for (auto& kv : by_zb) {
         Group g;
@@ -449,7 +402,6 @@ ApprBatch::ApprBatch(int dtype, double eps, const std::vector<ApprSpec>& specs)
         if (nbytes) BNMF_HIP(hipMemcpy(m + off, src, nbytes, hipMemcpyHostToDevice));
     };
     put(off_ai_, ai.data(), ai.size() * sizeof(ApprInst));
-    put(off_al_, al.data(), al.size() * sizeof(ApprInst));
     put(off_bi_, bi.data(), bi.size() * sizeof(BldInst));
     {
         size_t gi = 0;
@@ -505,11 +457,11 @@ void ApprBatch::enqueue_dense() {
 
 void ApprBatch::enqueue_live(hipStream_t st) {
     char* m = meta_.as<char>();
-    const ApprInst* al = reinterpret_cast<const ApprInst*>(m + off_al_);
+    const ApprInst* ai = reinterpret_cast<const ApprInst*>(m + off_ai_);
     for (int half = 0; half < 2; ++half) {
-        BNMF_HIP(launch_appr_live(0, n_live_, st, al, reinterpret_cast<const PassItem*>(m + off_live_)));
-        BNMF_HIP(launch_appr_psiA((uint32_t)lay_.size(), zmax_live_, st, al));
-        BNMF_HIP(launch_appr_live(1, half == 0 ? n_lrow_ : n_lcol_, st, al,
+        BNMF_HIP(launch_appr_live(0, n_live_, st, ai, reinterpret_cast<const PassItem*>(m + off_live_)));
+        BNMF_HIP(launch_appr_psiA((uint32_t)lay_.size(), zmax_live_, st, ai));
+        BNMF_HIP(launch_appr_live(1, half == 0 ? n_lrow_ : n_lcol_, st, ai,
                                   reinterpret_cast<const PassItem*>(m + (half == 0 ? off_lrow_ : off_lcol_))));
     }
 }
@@ -570,24 +522,17 @@ void ApprBatch::solve_async(size_t iters) {
     store_factors();
 }
 
-// The factors of the instances that run over lists: mu is transposed during a
-// solve, and both are double.
+// mu of the instances that run over lists is transposed during a solve.
 void ApprBatch::load_factors() {
-    char* b = arena_.as<char>();
-    for (const L_& l : lay_) {
-        if (!l.live) continue;
-        BNMF_HIP(launch_appr_load(dtype_ == BNMF_F32 ? 0 : 1, l.muT_d, b + l.off_mu, l.y, l.z, stream_));
-        if (dtype_ == BNMF_F32) BNMF_HIP(launch_appr_load(0, l.nu_d, b + l.off_nu, (size_t)l.x * l.z, 1, stream_));
-    }
+    for (const L_& l : lay_)
+        if (l.live)
+            BNMF_HIP(launch_appr_transpose(arena_.as<double>(l.off_pjk2), arena_.as<double>(l.off_mu), l.y, l.z, stream_));
 }
 
 void ApprBatch::store_factors() {
-    char* b = arena_.as<char>();
-    for (const L_& l : lay_) {
-        if (!l.live) continue;
-        BNMF_HIP(launch_appr_store(dtype_ == BNMF_F32 ? 0 : 1, b + l.off_mu, l.muT_d, l.z, l.y, stream_));
-        if (dtype_ == BNMF_F32) BNMF_HIP(launch_appr_store(0, b + l.off_nu, l.nu_d, (size_t)l.x * l.z, 1, stream_));
-    }
+    for (const L_& l : lay_)
+        if (l.live)
+            BNMF_HIP(launch_appr_transpose(arena_.as<double>(l.off_mu), arena_.as<double>(l.off_pjk2), l.z, l.y, stream_));
 }
 
 void ApprBatch::synchronize() { BNMF_HIP(hipStreamSynchronize(stream_)); }

@@ -1,7 +1,5 @@
-// bld_appr_live.hip — the approximate solver's iteration
-// (bld_appr.hpp:320-348) over the nonempty entries of X, for z <= 64, in double.
-// An FP32 instance's X and factors are widened when its solve starts and its
-// factors rounded once when it ends.
+// bld_appr_live.hip — the approximate solver's FP64 iteration
+// (bld_appr.hpp:320-348) over the nonempty entries of X, for z <= 64.
 //
 // In factored form an entry with X_ij = 0 contributes nothing to any sum of an
 // iteration (S_ijk, orig_over_appr and orig_over_appr_squared are all
@@ -30,9 +28,6 @@
 // dense passes before, lists now: 1024 x 1024 x 32, 975 -> 73 us at 2 % nonempty
 // entries, 131 at 10 %, 307 at 30 %; 384 x 384 x 32, 492 -> 51 us at 10 %; 16
 // instances of up to 384 x 384 x 32 (100 iterations with S fetched), 96 -> 16 ms.
-// FP32 instances, against the FP32 dense passes: 1024 x 1024 x 32, 312 -> 69 us at 2 %
-// and 102 at 8 %; 2048 x 2048 x 64, 3830 -> 175 us at 2 %; sixteen of 384 x 384 x 32,
-// 574 -> 89 us at 2 %.
 
 #include <hip/hip_runtime.h>
 
@@ -240,9 +235,8 @@ __global__ void __launch_bounds__(256) bld_appr_psiA_kernel(const ApprInst* __re
 // The lists, a wavefront per row, then per column (whose reads four
 // neighbours share). Counts: rows, then columns; ~0u marks a list that
 // holds a negative X_ij or one near the type's range.
-template <typename T>
 __global__ void __launch_bounds__(256)
-    bld_appr_count_kernel(const T* __restrict__ X, uint32_t x, uint32_t y, double most, uint32_t* __restrict__ counts) {
+    bld_appr_count_kernel(const double* __restrict__ X, uint32_t x, uint32_t y, double most, uint32_t* __restrict__ counts) {
     const uint32_t lane = threadIdx.x & 63u, row_blocks = (x + 3u) / 4u;
     const bool rows = blockIdx.x < row_blocks;
     const uint32_t list = (rows ? blockIdx.x : blockIdx.x - row_blocks) * 4u + (threadIdx.x >> 6);
@@ -253,7 +247,7 @@ __global__ void __launch_bounds__(256)
     bool bad = false;
 #pragma unroll 4
     for (uint32_t t = lane; t < len; t += 64u) {
-        const double v = (double)X[at + t * step];
+        const double v = X[at + t * step];
         n += v != 0.0;
         bad = bad || !(v >= 0.0 && v <= most);
     }
@@ -262,9 +256,8 @@ __global__ void __launch_bounds__(256)
     if (lane == 0) counts[rows ? list : x + list] = any ? ~0u : n;
 }
 
-template <typename T>
 __global__ void __launch_bounds__(256)
-    bld_appr_fill_kernel(const T* __restrict__ X, uint32_t x, uint32_t y, const uint32_t* __restrict__ rptr,
+    bld_appr_fill_kernel(const double* __restrict__ X, uint32_t x, uint32_t y, const uint32_t* __restrict__ rptr,
                          uint32_t* __restrict__ ridx, double* __restrict__ rxv, const uint32_t* __restrict__ cptr,
                          uint32_t* __restrict__ cidx, double* __restrict__ cxv) {
     const uint32_t lane = threadIdx.x & 63u, row_blocks = (x + 3u) / 4u;
@@ -279,7 +272,7 @@ __global__ void __launch_bounds__(256)
 #pragma unroll 4
     for (uint32_t t0 = 0; t0 < len; t0 += 64u) {
         const uint32_t t = t0 + lane;
-        const double v = t < len ? (double)X[from + t * step] : 0.0;
+        const double v = t < len ? X[from + t * step] : 0.0;
         const unsigned long long m = __builtin_amdgcn_ballot_w64(v != 0.0);
         if (v != 0.0) {
             const uint32_t p = at + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
@@ -290,16 +283,13 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-// dst (n x m) = src (m x n) transposed; one thread per element of dst. m = 1
-// copies n values. The types differ where an FP32 instance's factors enter or
-// leave its solve.
-template <typename D, typename S>
+// dst (n x m) = src (m x n) transposed; one thread per element of dst
 __global__ void __launch_bounds__(256)
-    bld_appr_transpose_kernel(D* __restrict__ dst, const S* __restrict__ src, size_t n, uint32_t m) {
+    bld_appr_transpose_kernel(double* __restrict__ dst, const double* __restrict__ src, uint32_t n, uint32_t m) {
     const size_t e = (size_t)blockIdx.x * 256u + threadIdx.x;
-    if (e >= n * m) return;
+    if (e >= (size_t)n * m) return;
     const size_t r = e / m, c = e - r * m;
-    dst[e] = (D)src[c * n + r];
+    dst[e] = src[c * n + r];
 }
 
 // ----------------------------------------------------------- launchers
@@ -317,42 +307,23 @@ hipError_t launch_appr_psiA(uint32_t n_inst, uint32_t zmax, hipStream_t st, cons
     return hipGetLastError();
 }
 
-hipError_t launch_appr_count(int dtype, const void* X, uint32_t x, uint32_t y, uint32_t* counts, hipStream_t st) {
-    const dim3 grid((x + 3u) / 4u + (y + 3u) / 4u);
-    if (dtype == 0)
-        hipLaunchKernelGGL(bld_appr_count_kernel<float>, grid, dim3(256), 0, st, static_cast<const float*>(X), x, y, 1e200,
-                           counts);
-    else
-        hipLaunchKernelGGL(bld_appr_count_kernel<double>, grid, dim3(256), 0, st, static_cast<const double*>(X), x, y,
-                           1e200, counts);
+hipError_t launch_appr_count(const double* X, uint32_t x, uint32_t y, uint32_t* counts, hipStream_t st) {
+    hipLaunchKernelGGL(bld_appr_count_kernel, dim3((x + 3u) / 4u + (y + 3u) / 4u), dim3(256), 0, st, X, x, y, 1e200,
+                       counts);
     return hipGetLastError();
 }
 
-hipError_t launch_appr_fill(int dtype, const void* X, uint32_t x, uint32_t y, const uint32_t* rptr, uint32_t* ridx,
-                            double* rxv, const uint32_t* cptr, uint32_t* cidx, double* cxv, hipStream_t st) {
-    const dim3 grid((x + 3u) / 4u + (y + 3u) / 4u);
-    if (dtype == 0)
-        hipLaunchKernelGGL(bld_appr_fill_kernel<float>, grid, dim3(256), 0, st, static_cast<const float*>(X), x, y, rptr,
-                           ridx, rxv, cptr, cidx, cxv);
-    else
-        hipLaunchKernelGGL(bld_appr_fill_kernel<double>, grid, dim3(256), 0, st, static_cast<const double*>(X), x, y, rptr,
-                           ridx, rxv, cptr, cidx, cxv);
+hipError_t launch_appr_fill(const double* X, uint32_t x, uint32_t y, const uint32_t* rptr, uint32_t* ridx, double* rxv,
+                            const uint32_t* cptr, uint32_t* cidx, double* cxv, hipStream_t st) {
+    hipLaunchKernelGGL(bld_appr_fill_kernel, dim3((x + 3u) / 4u + (y + 3u) / 4u), dim3(256), 0, st, X, x, y, rptr, ridx,
+                       rxv, cptr, cidx, cxv);
     return hipGetLastError();
 }
 
-template <typename D, typename S>
-static hipError_t launch_transpose(void* dst, const void* src, size_t n, uint32_t m, hipStream_t st) {
-    hipLaunchKernelGGL((bld_appr_transpose_kernel<D, S>), dim3((unsigned)((n * m + 255) / 256)), dim3(256), 0, st,
-                       static_cast<D*>(dst), static_cast<const S*>(src), n, m);
+hipError_t launch_appr_transpose(double* dst, const double* src, uint32_t n, uint32_t m, hipStream_t st) {
+    hipLaunchKernelGGL(bld_appr_transpose_kernel, dim3((unsigned)(((size_t)n * m + 255) / 256)), dim3(256), 0, st, dst,
+                       src, n, m);
     return hipGetLastError();
-}
-
-hipError_t launch_appr_load(int dtype, double* dst, const void* src, size_t n, uint32_t m, hipStream_t st) {
-    return dtype == 0 ? launch_transpose<double, float>(dst, src, n, m, st) : launch_transpose<double, double>(dst, src, n, m, st);
-}
-
-hipError_t launch_appr_store(int dtype, void* dst, const double* src, size_t n, uint32_t m, hipStream_t st) {
-    return dtype == 0 ? launch_transpose<float, double>(dst, src, n, m, st) : launch_transpose<double, double>(dst, src, n, m, st);
 }
 
 }  // namespace bnmf

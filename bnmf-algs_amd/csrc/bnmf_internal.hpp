@@ -101,17 +101,15 @@ hipError_t launch_appr_pass(int dtype, int mode, int zb, dim3 grid, hipStream_t 
                             const PassItem* items, const uint32_t* n_items, uint32_t zmax);
 hipError_t launch_appr_factor(int dtype, int half, dim3 grid, hipStream_t st, const ApprInst* insts,
                               const PassItem* items, const uint32_t* n_items);
-// the iteration over the nonempty entries of X, in double (bld_appr_live.hip): step
+// the FP64 iteration over the nonempty entries of X (bld_appr_live.hip): step
 // 0 sums (row and column items), 1 step
 hipError_t launch_appr_live(int step, uint32_t n, hipStream_t st, const ApprInst* insts, const PassItem* items);
 hipError_t launch_appr_psiA(uint32_t n_inst, uint32_t zmax, hipStream_t st, const ApprInst* insts);
-// X of dtype 0 (float) or 1 (double)
-hipError_t launch_appr_count(int dtype, const void* X, uint32_t x, uint32_t y, uint32_t* counts, hipStream_t st);
-hipError_t launch_appr_fill(int dtype, const void* X, uint32_t x, uint32_t y, const uint32_t* rptr, uint32_t* ridx,
-                            double* rxv, const uint32_t* cptr, uint32_t* cidx, double* cxv, hipStream_t st);
-// dst (n x m) = src (m x n) transposed; a factor of dtype into a solve and back
-hipError_t launch_appr_load(int dtype, double* dst, const void* src, size_t n, uint32_t m, hipStream_t st);
-hipError_t launch_appr_store(int dtype, void* dst, const double* src, size_t n, uint32_t m, hipStream_t st);
+hipError_t launch_appr_count(const double* X, uint32_t x, uint32_t y, uint32_t* counts, hipStream_t st);
+hipError_t launch_appr_fill(const double* X, uint32_t x, uint32_t y, const uint32_t* rptr, uint32_t* ridx, double* rxv,
+                            const uint32_t* cptr, uint32_t* cidx, double* cxv, hipStream_t st);
+// dst (n x m) = src (m x n) transposed
+hipError_t launch_appr_transpose(double* dst, const double* src, uint32_t n, uint32_t m, hipStream_t st);
 hipError_t launch_appr_S(int dtype, const ApprInst* inst, size_t n_fibers, hipStream_t st);
 hipError_t init_appr_attributes();
 void ensure_runtime();  // per-process kernel attributes, once
@@ -436,7 +434,6 @@ class ApprBatch {
             off_psiA, off_pjk, off_pjk2, off_ipk, off_ipk2, off_S;
         bool live = false;  // over the nonempty entries of X
         size_t entries = 0;
-        double *nu_d = nullptr, *muT_d = nullptr;  // its factors during a solve
     };
     struct Group {
         uint32_t zb, zmax, n_items;
@@ -449,7 +446,7 @@ class ApprBatch {
     void load_factors();
     void store_factors();
     bool live_candidate(const ApprSpec& s, double eps) const;
-    void plan_live(uint32_t* counts, const std::vector<ApprInst>& ai, std::vector<ApprInst>& al, std::vector<BldInst>& bi);
+    void plan_live(uint32_t* counts, std::vector<ApprInst>& ai, std::vector<BldInst>& bi);
 
     int dtype_, psi_ = 0;
     size_t es_;
@@ -461,7 +458,7 @@ class ApprBatch {
     uint32_t n_prep_ = 0, n_fnu_ = 0, n_fmu_ = 0;
     // work lists over the nonempty entries: both sides (sums), rows, columns
     DeviceBuffer lists_;
-    size_t off_live_ = 0, off_lrow_ = 0, off_lcol_ = 0, off_al_ = 0;
+    size_t off_live_ = 0, off_lrow_ = 0, off_lcol_ = 0;
     uint32_t zmax_dense_ = 0, zmax_live_ = 0, n_live_ = 0, n_lrow_ = 0, n_lcol_ = 0;
     hipStream_t stream_ = nullptr;
     hipStream_t side_ = nullptr;  // the listed instances' branch of a graph

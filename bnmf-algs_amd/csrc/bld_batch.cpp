@@ -76,8 +76,8 @@ uint32_t tile_cols_of(int dtype, uint32_t z) {
 }
 
 uint32_t choose_ti_rows(int dtype, uint32_t x, uint32_t y, uint32_t z, bool tall) {
-    // an empty instance has no tiles (and x = 0 would divide by zero below)
-    if (x == 0 || y == 0) return 4;
+    // an empty instance has no tiles (and a 0 would divide by zero below)
+    if (x == 0 || y == 0 || z == 0) return 4;
     // deep fibers: the wide pass's fixed tiles
     if (z > kFusedZ) return kWideRows;
     // Row-tile height depends on the instance shape only (never on the rest

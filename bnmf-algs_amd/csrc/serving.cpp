@@ -566,8 +566,11 @@ class Server {
         for (size_t n = 0; n < all.size(); ++n)
             if (all[n]->fresh) all[n]->live.gather(desc + n, stream_);
         iterate(ws_all, k_iters);
+        // (a request of no iterations keeps the S0 it was given: no step has left a
+        // psi(A) for the scatter to read)
         for (size_t n = 0; n < all.size(); ++n)
-            if (all[n]->done_iter + k_iters >= all[n]->max_iter) all[n]->live.scatter(desc + n, stream_);
+            if (all[n]->max_iter > 0 && all[n]->done_iter + k_iters >= all[n]->max_iter)
+                all[n]->live.scatter(desc + n, stream_);
         // requests that finish in this step, scored if asked
         std::vector<Request*> fin, score;
         for (Request* r : all) {

@@ -189,14 +189,31 @@ void ApprBatch::plan_live(uint32_t* counts, std::vector<ApprInst>& ai, std::vect
 }
 
 ApprBatch::ApprBatch(int dtype, double eps, const std::vector<ApprSpec>& specs)
-    : dtype_(dtype), es_(dtype == BNMF_F32 ? 4 : 8) {
+    : dtype_(dtype), psi_(dtype == BNMF_F32 ? PSIM_F32 : PSIM_F64_APPR), es_(dtype == BNMF_F32 ? 4 : 8) {
     ensure_runtime();
-    const int psi = dtype == BNMF_F32 ? PSIM_F32 : PSIM_F64_APPR;
-    psi_ = psi;
+    for (const ApprSpec& s : specs) BNMF_REQUIRE(s.z >= 1, "bld_appr needs z >= 1");
+    // where memory runs out, without the lists: the dense passes, which sum
+    // in another order (last digits)
+    for (bool lists : {true, false}) {
+        try {
+            plan(specs, eps, lists);
+            return;
+        } catch (const Error& e) {
+            release();
+            if (e.status != BNMF_ERR_OUT_OF_MEMORY || !lists) throw;
+            (void)hipGetLastError();
+        } catch (...) {
+            release();
+            throw;
+        }
+    }
+}
+
+void ApprBatch::plan(const std::vector<ApprSpec>& specs, double eps, bool lists) {
+    const int dtype = dtype_;
     // layouts
     size_t total = 0, n_counts = 0;
     for (const ApprSpec& s : specs) {
-        BNMF_REQUIRE(s.z >= 1, "bld_appr needs z >= 1");
         L_ l{};
         l.x = s.x;
         l.y = s.y;
@@ -232,7 +249,7 @@ ApprBatch::ApprBatch(int dtype, double eps, const std::vector<ApprSpec>& specs)
         l.off_ipk = take((size_t)l.n_tj * x * z * es_);
         l.off_ipk2 = take((size_t)l.n_tj * x * z * es_);
         l.off_S = take(x * y * z * es_);
-        l.live = live_candidate(s, eps);
+        l.live = lists && live_candidate(s, eps);
         if (l.live) n_counts += x + y;
         total = off;
         lay_.push_back(l);
@@ -423,14 +440,26 @@ ApprBatch::ApprBatch(int dtype, double eps, const std::vector<ApprSpec>& specs)
     BNMF_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
 }
 
-ApprBatch::~ApprBatch() {
+ApprBatch::~ApprBatch() { release(); }
+
+void ApprBatch::release() {
     if (stream_) (void)hipStreamSynchronize(stream_);
-    for (hipGraphExec_t g : graphs_)
+    for (hipGraphExec_t& g : graphs_) {
         if (g) (void)hipGraphExecDestroy(g);
+        g = nullptr;
+    }
     if (stream_) (void)hipStreamDestroy(stream_);
     if (side_) (void)hipStreamDestroy(side_);
     if (fork_) (void)hipEventDestroy(fork_);
     if (join_) (void)hipEventDestroy(join_);
+    stream_ = side_ = nullptr;
+    fork_ = join_ = nullptr;
+    lists_ = DeviceBuffer();
+    meta_ = DeviceBuffer();
+    arena_ = DeviceBuffer();
+    lay_.clear();
+    groups_.clear();
+    zmax_dense_ = zmax_live_ = 0;
 }
 
 void ApprBatch::enqueue_dense() {

@@ -355,32 +355,42 @@ Batch::Batch(int dtype, int psi_mode, double eps, const std::vector<InstSpec>& s
     dev_ = dev;
     BNMF_HIP(hipDeviceGetAttribute(&cus_, hipDeviceAttributeMultiprocessorCount, dev));
 
-    // layouts and arena; tall tiles where the memory for short ones' partial
-    // sums cannot be had
-    std::vector<size_t> base_off(specs.size());
-    size_t off_scratch = 0;
     for (const InstSpec& s : specs)
         BNMF_REQUIRE(s.x < (1u << 31) && s.y < (1u << 31) && s.z < (1u << 31),
                      "x, y and z must be below 2^31");
-    auto plan = [&](bool tall) {
-        layouts_.clear();
-        size_t total = 0;
-        for (size_t n = 0; n < specs.size(); ++n) {
-            layouts_.push_back(plan_instance(dtype, specs[n].x, specs[n].y, specs[n].z, true, tall));
-            base_off[n] = total;
-            total += layouts_.back().bytes;
+    // Where memory runs out, what is there for speed is left out: first the
+    // packed fibers (the same results), then short tiles, whose partial sums
+    // take more room than tall ones' (sums in another order: last digits).
+    for (Extras extras : {Extras::kPacked, Extras::kShortTiles, Extras::kNone}) {
+        try {
+            plan(specs, extras);
+            return;
+        } catch (const Error& e) {
+            release();
+            if (e.status != BNMF_ERR_OUT_OF_MEMORY || extras == Extras::kNone) throw;
+            (void)hipGetLastError();
+        } catch (...) {
+            release();
+            throw;
         }
-        off_scratch = total;
-        return std::max<size_t>(total + LivePlan::scratch_bytes(layouts_), kAlign);
-    };
-    const size_t bytes = plan(false);
-    if (hipMalloc(&arena_.ptr, bytes) == hipSuccess) {
-        arena_.bytes = bytes;
-    } else {
-        (void)hipGetLastError();
-        arena_.ptr = nullptr;
-        arena_ = DeviceBuffer(plan(true));
     }
+}
+
+void Batch::plan(const std::vector<InstSpec>& specs, Extras extras) {
+    const int dtype = dtype_;
+    const double eps = eps_;
+    // layouts and arena
+    std::vector<size_t> base_off(specs.size());
+    size_t total = 0;
+    for (size_t n = 0; n < specs.size(); ++n) {
+        layouts_.push_back(
+            plan_instance(dtype, specs[n].x, specs[n].y, specs[n].z, true, extras == Extras::kNone));
+        base_off[n] = total;
+        total += layouts_.back().bytes;
+    }
+    const size_t off_scratch = total;
+    if (extras == Extras::kPacked) total += LivePlan::scratch_bytes(layouts_);
+    arena_ = DeviceBuffer(std::max<size_t>(total, kAlign));
     device_bytes_ = arena_.bytes;
 
     // uploads (X, alpha, beta, S0 or its device draw). nonneg[n]: S0 >= 0
@@ -403,7 +413,7 @@ Batch::Batch(int dtype, int psi_mode, double eps, const std::vector<InstSpec>& s
         bool nn = true, pk = true;
         classify(dtype, s, eps, &nn, &pk);
         nonneg[n] = nn;
-        packable[n] = pk;
+        packable[n] = pk && extras == Extras::kPacked;
         if (S0) {
             BNMF_HIP(hipMemcpy(b + L.off_S0, S0, xyz * es_, hipMemcpyHostToDevice));
         } else {
@@ -441,8 +451,10 @@ Batch::Batch(int dtype, int psi_mode, double eps, const std::vector<InstSpec>& s
         if (tiny_threads_) packable.assign(specs.size(), false);
     }
     // the instances whose nonempty fibers are kept packed
-    live_ = LivePlan(dtype, d_main, layouts_, packable, arena_.as<char>(off_scratch));
-    device_bytes_ += live_.bytes();
+    if (extras == Extras::kPacked) {
+        live_ = LivePlan(dtype, d_main, layouts_, packable, arena_.as<char>(off_scratch));
+        device_bytes_ += live_.bytes();
+    }
     std::vector<PrepItem> prep;
     for (size_t n = 0; n < specs.size(); ++n) {
         const InstLayout& L = layouts_[n];
@@ -637,14 +649,33 @@ Batch::Batch(int dtype, int psi_mode, double eps, const std::vector<InstSpec>& s
     }
 }
 
-Batch::~Batch() {
+Batch::~Batch() { release(); }
+
+void Batch::release() {
     if (stream_) (void)hipStreamSynchronize(stream_);
-    for (hipGraphExec_t g : graphs_)
+    for (hipGraphExec_t& g : graphs_) {
         if (g) (void)hipGraphExecDestroy(g);
-    for (size_t l = 1; l < side_.size(); ++l) (void)hipStreamDestroy(side_[l]);
-    for (hipEvent_t e : fork_ev_) (void)hipEventDestroy(e);
-    for (hipEvent_t e : join_ev_) (void)hipEventDestroy(e);
+        g = nullptr;
+    }
+    for (size_t l = 1; l < side_.size(); ++l)
+        if (side_[l]) (void)hipStreamDestroy(side_[l]);
+    for (std::vector<hipEvent_t>* v : {&fork_ev_, &join_ev_}) {
+        for (hipEvent_t e : *v)
+            if (e) (void)hipEventDestroy(e);
+        v->clear();
+    }
+    side_.clear();
     if (stream_) (void)hipStreamDestroy(stream_);
+    stream_ = nullptr;
+    live_ = LivePlan();
+    meta_ = DeviceBuffer();
+    arena_ = DeviceBuffer();
+    layouts_.clear();
+    lanes_.clear();
+    for (std::vector<Bucket>& g : groups_) g.clear();
+    tiny_threads_ = 0;
+    tiny_lds_ = 0;
+    zmax_ = 0;
 }
 
 void Batch::enqueue_pass(int mode, bool first) {

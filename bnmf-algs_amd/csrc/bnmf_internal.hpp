@@ -274,7 +274,7 @@ class LivePlan {
     // Uploads the tile table and builds the lists; insts: the descriptors on
     // the device
     void build(const std::vector<BldInst>& descs, const BldInst* insts, hipStream_t st);
-    const LiveTile* tiles() const { return tab_.as<LiveTile>(); }
+    const LiveTile* tiles() const { return tab_; }
     // packed S from S_src, and S from its packed form
     void gather(const BldInst* insts, hipStream_t st) const;
     void scatter(const BldInst* insts, hipStream_t st) const;
@@ -289,8 +289,9 @@ class LivePlan {
     }
     int dtype_ = 0;
     char* base_ = nullptr;
+    LiveTile* tab_ = nullptr;
     size_t bytes_ = 0;
-    DeviceBuffer buf_, tab_;
+    DeviceBuffer buf_;
     std::vector<Off> offs_;
     std::vector<size_t> fibers_;
     std::vector<uint32_t> lds_;  // 0: the instance runs the dense passes
@@ -334,6 +335,12 @@ class Batch {
         size_t off_count;
         uint32_t tile0 = 0, lds = 0;  // live groups: first tile, dynamic LDS
     };
+    // What a batch takes beyond what it cannot do without: short tiles and
+    // packed fibers, short tiles, nothing.
+    enum class Extras { kPacked, kShortTiles, kNone };
+    // Everything on the device for specs; release() undoes it.
+    void plan(const std::vector<InstSpec>& specs, Extras extras);
+    void release();
     // iterations of a batch of tiny instances; first: from S0
     void run_tiny(size_t iters, bool first);
     // S of the packed instances from their packed form, and back
@@ -439,6 +446,10 @@ class ApprBatch {
         uint32_t zb, zmax, n_items;
         size_t off_items, off_count;
     };
+    // everything on the device for specs, with the lists of nonempty entries
+    // or without; release() undoes it
+    void plan(const std::vector<ApprSpec>& specs, double eps, bool lists);
+    void release();
     void enqueue_dense();
     void enqueue_live(hipStream_t st);
     hipGraphExec_t graph_of(int level);

@@ -117,6 +117,7 @@ LivePlan::LivePlan(int dtype, const std::vector<BldInst>& descs, const std::vect
         at += nt;
     }
     if (slot_.empty()) return;
+    const size_t off_tab = take(slot_.size() * sizeof(LiveTile));
     // the packed form is extra memory: without room for it every instance
     // runs the dense passes, with the same results
     {
@@ -130,6 +131,7 @@ LivePlan::LivePlan(int dtype, const std::vector<BldInst>& descs, const std::vect
             return;
         }
         base_ = static_cast<char*>(p);
+        tab_ = at<LiveTile>(off_tab);
         bytes_ = off;
         if (!mem) {
             buf_.ptr = p;
@@ -191,9 +193,8 @@ uint32_t LivePlan::add_launch(std::vector<PassItem>& items, const std::vector<Bl
 void LivePlan::build(const std::vector<BldInst>& descs, const BldInst* insts, hipStream_t st) {
     if (!any()) return;
     for (LiveTile& t : tiles_) t.iter = descs[t.inst].iter;
-    tab_ = DeviceBuffer(tiles_.size() * sizeof(LiveTile));
-    BNMF_HIP(hipMemcpy(tab_.ptr, tiles_.data(), tab_.bytes, hipMemcpyHostToDevice));
-    BNMF_HIP(launch_live_build(dtype_, insts, tab_.as<LiveTile>(), (uint32_t)tiles_.size(), st));
+    BNMF_HIP(hipMemcpy(tab_, tiles_.data(), tiles_.size() * sizeof(LiveTile), hipMemcpyHostToDevice));
+    BNMF_HIP(launch_live_build(dtype_, insts, tab_, (uint32_t)tiles_.size(), st));
 }
 
 void LivePlan::gather(const BldInst* insts, hipStream_t st) const {

@@ -15,7 +15,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
-#include <system_error>
+#include <exception>
 #include <thread>
 #include <vector>
 
@@ -114,7 +114,7 @@ void HostStage::copy(void* dst, const void* src, size_t bytes, hipStream_t st) {
     th.reserve(n);
     try {
         for (unsigned w = 1; w < n; ++w) th.emplace_back([&c, w] { c.work(w); });
-    } catch (const std::system_error&) {
+    } catch (const std::exception&) {  // no thread, or no memory for one
     }
     c.work(0);
     for (std::thread& t : th) t.join();

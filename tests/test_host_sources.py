@@ -35,3 +35,7 @@ def _run(objects, tmp_path, name):
 
 def test_batches_at_the_limit_of_memory(objects, tmp_path):
     _run(objects, tmp_path, "test_batch_memory")
+
+
+def test_results_where_host_memory_runs_out(objects, tmp_path):
+    _run(objects, tmp_path, "test_host_copy_alloc")

@@ -175,11 +175,12 @@ struct DeviceBuffer {
     }
 };
 
-// Results to (pageable) host memory through a pinned buffer of its own
-// (hostcopy.cpp). Safe with several threads: one copy at a time.
+// Results to (pageable) host memory, large or many ones through a pinned buffer
+// of its own (hostcopy.cpp). Safe with several threads: one copy through the
+// buffer at a time.
 struct HostStage {
     void* pinned = nullptr;
-    size_t size = 0;
+    size_t fetched = 0;  // bytes of results large enough for the buffer
     std::mutex mu;
     HostStage() = default;
     HostStage(const HostStage&) = delete;

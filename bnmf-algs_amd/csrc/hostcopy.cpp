@@ -7,8 +7,15 @@
 // host copies of several chunks overlap each other and the link. Measured
 // (1 GiB into fresh huge pages, one MI355X, 16 host cores): 27 ms with 8
 // threads and 2 MiB chunks against 107 ms for hipMemcpy; 34 ms with 1 MiB
-// chunks, the same with 16 threads; into 4 KiB pages 48 ms. The pinned buffer
-// (at most 32 MiB) belongs to the batch or server whose results it carries.
+// chunks, the same with 16 threads; into 4 KiB pages 48 ms. The 60 results of a
+// batch, 5 MiB on average, take 3 ms longer where only those of 8 MiB and more
+// are staged.
+//
+// The pinned buffer (32 MiB) belongs to the batch or server whose results it
+// carries. Pinning it takes 1 to 2 ms, more than a small result does in all
+// (16 MiB: 0.95 ms by hipMemcpy, 2.0 ms with the pinning, 0.6 ms once pinned), so
+// an object's results go by hipMemcpy until they come to 40 MiB, and one that is
+// larger takes the buffer at once (48 MiB: 5.0 against 3.5 ms).
 
 #include <hip/hip_runtime.h>
 
@@ -26,8 +33,8 @@ namespace bnmf {
 namespace {
 constexpr size_t kChunk = 2u << 20, kChunkLeast = 256u << 10;
 constexpr unsigned kThreads = 8;
-// bytes a thread is worth starting for
-constexpr size_t kPerThread = 768u << 10;
+constexpr size_t kPerThread = 768u << 10;  // bytes a thread is worth starting for
+constexpr size_t kFirst = 40u << 20;       // bytes of results before a buffer is pinned
 
 struct Copy {
     char* dst;
@@ -80,25 +87,24 @@ void HostStage::copy(void* dst, const void* src, size_t bytes, hipStream_t st) {
     if (bytes == 0) return;
     const unsigned cores = std::max(1u, std::thread::hardware_concurrency());
     const unsigned n = (unsigned)std::min<size_t>(std::min(kThreads, cores), bytes / kPerThread);
-    const size_t chunk =
-        n ? std::min(kChunk, (bytes / (2 * n) + kChunkLeast - 1) / kChunkLeast * kChunkLeast) : kChunk;
-    std::unique_lock<std::mutex> lk(mu);
-    if (n >= 2 && size < 2 * n * chunk) {
-        if (pinned) (void)hipHostFree(pinned);
-        pinned = nullptr;
-        size = 2 * n * chunk;
-        if (hipHostMalloc(&pinned, size, 0) != hipSuccess) {
+    std::unique_lock<std::mutex> lk(mu, std::defer_lock);
+    bool staged = n >= 2;
+    if (staged) {
+        lk.lock();
+        fetched += bytes;
+        if (!pinned && fetched >= kFirst && hipHostMalloc(&pinned, 2 * kThreads * kChunk, 0) != hipSuccess) {
             (void)hipGetLastError();
             pinned = nullptr;
-            size = 0;
         }
+        staged = pinned != nullptr;
     }
-    if (n < 2 || pinned == nullptr) {
-        lk.unlock();
+    if (!staged) {
+        if (lk.owns_lock()) lk.unlock();
         BNMF_HIP(hipStreamSynchronize(st));
         BNMF_HIP(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost));
         return;
     }
+    const size_t chunk = std::min(kChunk, (bytes / (2 * n) + kChunkLeast - 1) / kChunkLeast * kChunkLeast);
     Copy c;
     c.dst = static_cast<char*>(dst);
     c.src = static_cast<const char*>(src);

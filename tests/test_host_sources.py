@@ -39,3 +39,7 @@ def test_batches_at_the_limit_of_memory(objects, tmp_path):
 
 def test_results_where_host_memory_runs_out(objects, tmp_path):
     _run(objects, tmp_path, "test_host_copy_alloc")
+
+
+def test_results_to_host_memory(objects, tmp_path):
+    _run(objects, tmp_path, "test_host_copy")

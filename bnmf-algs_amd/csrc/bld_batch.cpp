@@ -333,8 +333,9 @@ void classify(int dtype, const InstSpec& s, double eps, bool* nonneg, bool* pack
 }
 
 // ------------------------------------------------------------------ batch
-Batch::Batch(int dtype, int psi_mode, double eps, const std::vector<InstSpec>& specs, int algo)
-    : dtype_(dtype), psi_(psi_mode), algo_(algo), eps_(eps), es_(dtype == BNMF_F32 ? 4 : 8), specs_(specs) {
+Batch::Batch(int dtype, int psi_mode, double eps, const std::vector<InstSpec>& specs, int algo, size_t iters)
+    : dtype_(dtype), psi_(psi_mode), algo_(algo), eps_(eps), es_(dtype == BNMF_F32 ? 4 : 8), iters_known_(iters),
+      specs_(specs) {
     BNMF_REQUIRE(algo == BNMF_ALGO_MULT || algo == BNMF_ALGO_ADD, "algo must be BNMF_ALGO_MULT or BNMF_ALGO_ADD");
     // bld_add evaluates every digamma with psi_appr (src/bld/bld_add.hpp:137-146)
     if (algo == BNMF_ALGO_ADD) {
@@ -413,7 +414,7 @@ void Batch::plan(const std::vector<InstSpec>& specs, Extras extras) {
         bool nn = true, pk = true;
         classify(dtype, s, eps, &nn, &pk);
         nonneg[n] = nn;
-        packable[n] = pk && extras == Extras::kPacked;
+        packable[n] = pk && extras == Extras::kPacked && iters_known_ >= LivePlan::least_iterations(xyz);
         if (S0) {
             BNMF_HIP(hipMemcpy(b + L.off_S0, S0, xyz * es_, hipMemcpyHostToDevice));
         } else {

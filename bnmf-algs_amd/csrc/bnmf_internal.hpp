@@ -261,6 +261,8 @@ class LivePlan {
     // step's cost grows with the share, the dense step's does not; at 28 % (100 x
     // 100 x 17 in double) it takes half the dense step's time.
     static constexpr double kLiveMax = 0.5;
+    // Iterations from which packing an instance of so many elements pays.
+    static size_t least_iterations(size_t elements);
     // false where X (host, n entries) is plainly fuller than `most`
     static bool worth(int dtype, const void* X, size_t n, double most = kLiveMax);
     bool any() const { return !tiles_.empty(); }
@@ -304,9 +306,10 @@ class LivePlan {
 // captured per-iteration graphs.
 class Batch {
    public:
-    // algo: BNMF_ALGO_MULT (bld_mult) or BNMF_ALGO_ADD (bld_add)
-    Batch(int dtype, int psi_mode, double eps, const std::vector<InstSpec>& specs,
-          int algo = BNMF_ALGO_MULT);
+    // algo: BNMF_ALGO_MULT (bld_mult) or BNMF_ALGO_ADD (bld_add); iters: the
+    // iterations of the batch's only solve, where that is known
+    Batch(int dtype, int psi_mode, double eps, const std::vector<InstSpec>& specs, int algo = BNMF_ALGO_MULT,
+          size_t iters = SIZE_MAX);
     ~Batch();
     void solve_async(size_t iters);
     // Restarts from S0 and runs at most max_iter iterations; every
@@ -370,6 +373,7 @@ class Batch {
     int dev_ = 0;
     double eps_;
     size_t es_;
+    size_t iters_known_;  // iterations of the only solve, or SIZE_MAX
     std::vector<InstLayout> layouts_;
     std::vector<InstSpec> specs_;
     DeviceBuffer arena_;

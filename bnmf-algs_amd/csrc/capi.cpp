@@ -89,7 +89,7 @@ void solve_one(int dtype, const T* X, size_t x, size_t y, size_t z, const double
     s.beta = beta;
     s.S0 = S0;
     s.seed = seed;
-    bnmf::Batch b(dtype, psi_mode(dtype, use_psi_appr), eps, {s}, algo);
+    bnmf::Batch b(dtype, psi_mode(dtype, use_psi_appr), eps, {s}, algo, max_iter);
     b.solve_async(max_iter);
     b.synchronize();
     b.get_S(0, S_out);
@@ -287,7 +287,7 @@ bnmf_status bnmf_log_marginal_S(int dtype, const void* S, size_t x, size_t y, si
         s.a = a;
         s.b = b;
         s.S0 = S;
-        bnmf::Batch bt(dtype, psi_mode(dtype, 0), 1e-50, {s});
+        bnmf::Batch bt(dtype, psi_mode(dtype, 0), 1e-50, {s}, BNMF_ALGO_MULT, 0);
         bt.log_marginal(out);
     });
 }
@@ -309,7 +309,7 @@ bnmf_status bnmf_tensor_sums(int dtype, const void* S, size_t x, size_t y, size_
         s.alpha = ones_x.data();
         s.beta = ones_z.data();
         s.S0 = S;
-        bnmf::Batch bt(dtype, psi_mode(dtype, 0), 1e-50, {s});
+        bnmf::Batch bt(dtype, psi_mode(dtype, 0), 1e-50, {s}, BNMF_ALGO_MULT, 0);
         bt.tensor_sums(S_pjk, S_ipk, S_ijp);
     });
 }
@@ -427,7 +427,8 @@ bnmf_status bnmf_bld_fact(int dtype, const void* S, size_t x, size_t y, size_t z
         s.a = a;
         s.b = b;
         s.S0 = S;
-        bnmf::Batch bt(dtype, dtype == BNMF_F32 ? bnmf::PSIM_F32 : bnmf::PSIM_F64_EXACT, 1e-50, {s});
+        bnmf::Batch bt(dtype, dtype == BNMF_F32 ? bnmf::PSIM_F32 : bnmf::PSIM_F64_EXACT, 1e-50, {s}, BNMF_ALGO_MULT,
+                       0);
         bt.fact(0, eps, W, H, L);
     });
 }

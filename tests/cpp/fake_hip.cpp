@@ -16,14 +16,14 @@ namespace fake {
 std::mutex mu;
 std::map<void*, size_t> blocks;
 size_t used = 0, capacity = ~(size_t)0, fail_at = 0, mallocs = 0, pins = 0;
-std::atomic<size_t> copies{0}, launches{0};
+std::atomic<size_t> copies{0}, launches{0}, packs{0};
 
 void reset(size_t cap, size_t fail) {
     std::lock_guard<std::mutex> lk(mu);
     capacity = cap;
     fail_at = fail;
     mallocs = pins = 0;
-    copies = launches = 0;
+    copies = launches = packs = 0;
 }
 size_t in_use() {
     std::lock_guard<std::mutex> lk(mu);
@@ -47,6 +47,11 @@ hipError_t hipGetDevice(int* d) {
     return hipSuccess;
 }
 hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetDeviceCount(int* n) {
+    *n = 1;
+    return hipSuccess;
+}
+hipError_t hipDeviceSynchronize() { return hipSuccess; }
 hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) {
     *v = 256;
     return hipSuccess;
@@ -135,9 +140,6 @@ hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) {
 
 namespace bnmf {
 
-void set_last_error(const std::string&) {}
-void clear_last_error() {}
-
 static hipError_t launched() {
     ++fake::launches;
     return hipSuccess;
@@ -172,7 +174,13 @@ hipError_t launch_prep(int, int, bool, dim3, hipStream_t, const BldInst*, const 
 hipError_t launch_score(dim3, hipStream_t, const BldInst*, const PrepItem*, const uint32_t*, uint32_t) { return launched(); }
 hipError_t launch_fact(int, const BldInst*, uint32_t, uint32_t, double, double*, double*, double*, hipStream_t) { return launched(); }
 hipError_t launch_tiny(int, uint32_t, uint32_t, size_t, hipStream_t, const BldInst*, uint32_t) { return launched(); }
-hipError_t launch_live_build(int, const BldInst*, LiveTile*, uint32_t, hipStream_t) { return launched(); }
+hipError_t launch_live_build(int, const BldInst*, LiveTile*, uint32_t, hipStream_t) {
+    ++fake::packs;
+    return launched();
+}
+hipError_t launch_psi_eval(int, const double*, double*, size_t, hipStream_t) { return launched(); }
+hipError_t launch_sample(double*, const double*, const double*, const double*, size_t, uint32_t, uint64_t, int, size_t, hipStream_t) { return launched(); }
+void bld_mult_f32_noalloc(const float*, uint32_t, uint32_t, uint32_t, const double*, const double*, size_t, double, const float*, uint64_t, float*, hipStream_t) {}
 hipError_t launch_live_gather(int, const BldInst*, const LiveTile*, uint32_t, hipStream_t) { return launched(); }
 hipError_t launch_live_scatter(int, const BldInst*, const LiveTile*, uint32_t, hipStream_t) { return launched(); }
 hipError_t launch_appr_pass(int, int, int, dim3, hipStream_t, const ApprInst*, const PassItem*, const uint32_t*, uint32_t) { return launched(); }

@@ -11,5 +11,5 @@ void reset(size_t capacity = ~(size_t)0, size_t fail_at = 0);
 size_t in_use();     // bytes of device memory
 size_t n_mallocs();  // since reset
 size_t n_pins();     // hipHostMalloc since reset
-extern std::atomic<size_t> copies, launches;
+extern std::atomic<size_t> copies, launches, packs;  // packs: launches that pack fibers
 }  // namespace fake

@@ -12,7 +12,7 @@ SRC = os.path.join(ROOT, "bnmf-algs_amd", "csrc")
 CPP = os.path.join(ROOT, "tests", "cpp")
 FLAGS = ["-std=c++17", "-O1", "-Wall", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I", os.path.join(ROOT, "include"),
          "-fsanitize=address,undefined"]
-SOURCES = ["bld_batch", "live", "hostcopy", "bld_appr_host", "tune", "sampler", "serving"]
+SOURCES = ["bld_batch", "live", "hostcopy", "bld_appr_host", "tune", "sampler", "serving", "capi"]
 
 
 @pytest.fixture(scope="module")
@@ -43,3 +43,7 @@ def test_results_where_host_memory_runs_out(objects, tmp_path):
 
 def test_results_to_host_memory(objects, tmp_path):
     _run(objects, tmp_path, "test_host_copy")
+
+
+def test_calls_of_few_iterations(objects, tmp_path):
+    _run(objects, tmp_path, "test_few_iterations")

@@ -94,7 +94,7 @@ bool ApprBatch::live_candidate(const ApprSpec& s, double eps) const {
     if (!(eps >= 1e-200 && eps <= 1.0)) return false;
     if (!within(s.alpha, x, 1e-6, 1e30) || !within(s.beta, z, 1e-6, 1e30)) return false;
     auto tame = [](const void* p, size_t n) { return !p || within(static_cast<const double*>(p), n, 0.0, 1e100); };
-    return tame(s.nu0, x * z) && tame(s.mu0, z * y) && LivePlan::worth(dtype_, s.X, x * y, live_share(x, y, s.z));
+    return tame(s.nu0, x * z) && tame(s.mu0, z * y) && LivePlan::worth(dtype_, s.X, x, y, live_share(x, y, s.z));
 }
 
 // The lists of the instances that are sparse enough, in one allocation; none

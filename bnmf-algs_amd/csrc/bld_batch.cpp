@@ -319,7 +319,7 @@ void classify(int dtype, const InstSpec& s, double eps, bool* nonneg, bool* pack
     bool nn = true;
     for (uint32_t k = 0; k < s.z; ++k) nn = nn && s.beta[k] >= 1.0;
     bool pk = nn && xy > 0 && s.z <= kFusedZ && !(dtype == BNMF_F32 && generic_steps()) && eps >= 1e-200 && eps <= 1.0 &&
-              LivePlan::worth(dtype, s.X, xy);
+              LivePlan::worth(dtype, s.X, s.x, s.y);
     for (uint32_t i = 0; i < s.x; ++i) pk = pk && s.alpha[i] >= 1e-6 && s.alpha[i] <= 1e30;
     for (uint32_t k = 0; k < s.z; ++k) pk = pk && s.beta[k] <= 1e30;
     if (nn && s.S0) {

@@ -263,8 +263,8 @@ class LivePlan {
     static constexpr double kLiveMax = 0.5;
     // Iterations from which packing an instance of so many elements pays.
     static size_t least_iterations(size_t elements);
-    // false where X (host, n entries) is plainly fuller than `most`
-    static bool worth(int dtype, const void* X, size_t n, double most = kLiveMax);
+    // false where X (host, x*y entries) is plainly fuller than `most`
+    static bool worth(int dtype, const void* X, size_t x, size_t y, double most = kLiveMax);
     bool any() const { return !tiles_.empty(); }
     bool live(size_t n) const { return n < lds_.size() && lds_[n] > 0; }
     uint32_t lds(size_t n) const { return lds_[n]; }

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <numeric>
 #include <vector>
 
 #include "bnmf_internal.hpp"
@@ -27,11 +28,14 @@ size_t LivePlan::scratch_bytes(const std::vector<InstLayout>& lay) {
     return align_up(lay.size() * sizeof(BldInst)) + align_up(tiles * sizeof(PassItem)) + align_up(tiles * 4);
 }
 
-// A matrix whose sampled entries (4096 at most, evenly spaced) are mostly
-// nonzero is not worth the count on the device.
+// A matrix (rows of y entries) whose sampled entries (some 4096, evenly spaced)
+// are mostly nonzero is not worth the count on the device. The spacing has no
+// factor in common with y, so that the samples go through all columns: a busy
+// column, or a few, must not stand for the matrix.
 template <typename T>
-static bool mostly_full(const T* X, size_t n, double most) {
-    const size_t step = std::max<size_t>(1, n / 4096);
+static bool mostly_full(const T* X, size_t n, size_t y, double most) {
+    size_t step = std::max<size_t>(1, n / 4096);
+    while (std::gcd(step, y) != 1) ++step;
     size_t seen = 0, full = 0;
     for (size_t t = 0; t < n; t += step) {
         ++seen;
@@ -50,9 +54,9 @@ size_t LivePlan::least_iterations(size_t elements) {
     return elements < (1u << 22) ? 24 : elements < (1u << 24) ? 40 : 80;
 }
 
-bool LivePlan::worth(int dtype, const void* X, size_t n, double most) {
-    return !(dtype == BNMF_F32 ? mostly_full(static_cast<const float*>(X), n, most)
-                               : mostly_full(static_cast<const double*>(X), n, most));
+bool LivePlan::worth(int dtype, const void* X, size_t x, size_t y, double most) {
+    return !(dtype == BNMF_F32 ? mostly_full(static_cast<const float*>(X), x * y, y, most)
+                               : mostly_full(static_cast<const double*>(X), x * y, y, most));
 }
 
 LivePlan::LivePlan(int dtype, const std::vector<BldInst>& descs, const std::vector<InstLayout>& lay,

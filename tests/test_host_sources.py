@@ -47,3 +47,7 @@ def test_results_to_host_memory(objects, tmp_path):
 
 def test_calls_of_few_iterations(objects, tmp_path):
     _run(objects, tmp_path, "test_few_iterations")
+
+
+def test_share_from_a_sample(objects, tmp_path):
+    _run(objects, tmp_path, "test_worth")

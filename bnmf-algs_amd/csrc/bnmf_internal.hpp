@@ -241,8 +241,8 @@ hipError_t launch_pass_key(const PassKey& k, int dtype, int psi, int mode, dim3 
 
 // nonneg: S stays >= 0 (S0 >= 0 and beta >= 1). packable: additionally every
 // gradient of its solve is finite, so that a fiber with X_ij = 0 stays exactly
-// zero, and X looks sparse enough (LivePlan).
-void classify(int dtype, const InstSpec& s, double eps, bool* nonneg, bool* packable);
+// zero, and X looks sparse enough (LivePlan). add: for the additive solver.
+void classify(int dtype, bool add, const InstSpec& s, double eps, bool* nonneg, bool* packable);
 
 // Which instances of a batch keep their nonempty fibers packed, and where
 // (live.cpp). Results do not depend on it.
@@ -253,18 +253,17 @@ class LivePlan {
     // scratch: device memory of scratch_bytes, used until the call returns; it
     // starts with the descriptors. mem: where the packed buffers come from and
     // are given back to (null for none left); without it they are the plan's own.
-    LivePlan(int dtype, const std::vector<BldInst>& descs, const std::vector<InstLayout>& lay,
+    LivePlan(int dtype, bool add, const std::vector<BldInst>& descs, const std::vector<InstLayout>& lay,
              const std::vector<bool>& candidate, char* scratch, const std::function<void*(size_t)>& mem = nullptr);
     LivePlan() = default;
     static size_t scratch_bytes(const std::vector<InstLayout>& lay);
-    // Largest share of nonempty fibers at which an instance is packed. The packed
-    // step's cost grows with the share, the dense step's does not; at 28 % (100 x
-    // 100 x 17 in double) it takes half the dense step's time.
-    static constexpr double kLiveMax = 0.5;
+    // Largest share of nonempty fibers at which an instance is packed; elements:
+    // those of its batch. add: the additive solver's step.
+    static double most_share(int dtype, bool add, size_t x, size_t y, uint32_t z, size_t elements);
     // Iterations from which packing an instance of so many elements pays.
     static size_t least_iterations(size_t elements);
     // false where X (host, x*y entries) is plainly fuller than `most`
-    static bool worth(int dtype, const void* X, size_t x, size_t y, double most = kLiveMax);
+    static bool worth(int dtype, const void* X, size_t x, size_t y, double most);
     bool any() const { return !tiles_.empty(); }
     bool live(size_t n) const { return n < lds_.size() && lds_[n] > 0; }
     uint32_t lds(size_t n) const { return lds_[n]; }

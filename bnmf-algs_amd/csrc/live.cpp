@@ -59,15 +59,55 @@ bool LivePlan::worth(int dtype, const void* X, size_t x, size_t y, double most) 
                                : mostly_full(static_cast<const double*>(X), x * y, y, most));
 }
 
-LivePlan::LivePlan(int dtype, const std::vector<BldInst>& descs, const std::vector<InstLayout>& lay,
+// The packed step's cost grows with the share, the dense step's does not. Where
+// they meet, from iterations (packed / dense, us) of one or n instances:
+//   FP32  z <= 4, where a dense step is as fast as its launches: 128x128x4
+//         16.5/15.9 at a share of 0.03, 64 of them 18/19; 8 of 512x512x4 18/30
+//         and 31/31 at 0.49
+//         z <= 24: 513x861x24 44/44 at 0.49, 64 of 100x100x17 41/39
+//         z <= 32: 64 of 40x40x32 24/30 at 0.45; 100x100x32 37/38 at 0.40;
+//         256x256x32 39/44 at 0.35, 44/44 at 0.40; 32 of them 107/116, 123/116;
+//         16 of 400x400x28 126/140 at 0.40; 1448x1448x32 173/176 at 0.45;
+//         2048x2048x32 267/263 at 0.45, 432/265 at 0.49
+//         z <= 64: 64 of 32x32x64 50/64 at 0.45; 16 of 128x128x64 115/129 at
+//         0.30, 141/130 at 0.35; 16 of 200x200x40 77/83 at 0.35; 512x512x48 59/63
+//         at 0.40; 8 of 512x512x64 259/282 at 0.45; 2048x2048x64 439/484 at 0.30,
+//         515/485 at 0.35, 911/484 at 0.49
+//   FP64  z <= 24: 100x100x17 26/31 at 0.49, 8 of 384x384x24 175/175
+//         z <= 32: 256x256x32 30/31 at 0.35, 33/31 at 0.40; 4 of 512x512x32
+//         178/186 at 0.45; 1024x1024x32 159/167 at 0.30, 173/171 at 0.35;
+//         2048x2048x32 339/529 at 0.20, 483/546 at 0.25, 565/533 at 0.30
+//         z <= 64: 8 of 200x200x64 129/138 at 0.49; 4 of 512x512x64 263/323 at
+//         0.35, 334/327 at 0.40; 1024x1024x64 280/305 at 0.30, 335/307 at 0.35
+//         additive step: 4 of 512x512x64 571/724 at 0.49, 256x256x32 41/51
+// Large deep instances lose soonest: their tiles have more fibers than the LDS
+// holds, and the partial sums read S again in parts.
+double LivePlan::most_share(int dtype, bool add, size_t x, size_t y, uint32_t z, size_t elements) {
+    const size_t xy = x * y;
+    if (dtype == BNMF_F32) {
+        if (z <= 4) return elements >= 6000000 ? 0.5 : 0.0;
+        if (z <= 24) return 0.5;
+        if (z <= 32) return xy < (1u << 11) ? 0.5 : xy >= (1u << 20) ? 0.45 : z <= 28 ? 0.42 : 0.37;
+        if (xy >= (1u << 17)) return xy < (1u << 21) ? 0.43 : 0.32;
+        return xy < (1u << 11) ? 0.5 : z <= 48 ? 0.38 : 0.34;
+    }
+    if (add || z <= 24) return 0.5;
+    if (xy >= (1u << 20)) return xy < (1u << 21) ? 0.32 : 0.26;
+    return z <= 32 ? 0.4 : xy < (1u << 17) ? 0.5 : 0.38;
+}
+
+LivePlan::LivePlan(int dtype, bool add, const std::vector<BldInst>& descs, const std::vector<InstLayout>& lay,
                    const std::vector<bool>& candidate, char* scratch, const std::function<void*(size_t)>& mem)
     : dtype_(dtype), offs_(descs.size()), fibers_(descs.size(), 0), lds_(descs.size(), 0) {
     const size_t es = dtype == BNMF_F32 ? 4 : 8;
+    size_t elements = 0;
+    for (const InstLayout& L : lay) elements += L.elements();
+    auto most_of = [&](const InstLayout& L) { return most_share(dtype, add, L.x, L.y, L.z, elements); };
     // nonempty fibers of every candidate's tiles
     std::vector<PassItem> items;
     for (size_t n = 0; n < descs.size(); ++n) {
         const InstLayout& L = lay[n];
-        if (!candidate[n] || L.elements() == 0 || L.z > kFusedZ || L.ti_rows > kLiveRows) continue;
+        if (!candidate[n] || L.elements() == 0 || L.z > kFusedZ || L.ti_rows > kLiveRows || most_of(L) == 0.0) continue;
         for (uint32_t ti = 0; ti < L.n_ti; ++ti)
             for (uint32_t tj = 0; tj < L.n_tj; ++tj) items.push_back(PassItem{(uint32_t)n, ti, tj, 0});
     }
@@ -107,7 +147,7 @@ LivePlan::LivePlan(int dtype, const std::vector<BldInst>& descs, const std::vect
             slots += (c + gf - 1) / gf * gf;
             most = std::max(most, c);
         }
-        ok = ok && total > 0 && (double)total <= kLiveMax * (double)L.x * (double)L.y && slots < (1ull << 31);
+        ok = ok && total > 0 && (double)total <= most_of(L) * (double)L.x * (double)L.y && slots < (1ull << 31);
         if (ok) {
             const size_t least = live_lds_need(dtype, L.z, L.tile_cols, L.ti_rows, most, 4);
             const size_t all = live_lds_need(dtype, L.z, L.tile_cols, L.ti_rows, most, (L.z + 3) / 4 * 4);

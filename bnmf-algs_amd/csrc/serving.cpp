@@ -145,7 +145,7 @@ class Server {
         s.S0 = d.S0 ? r->S0.data() : nullptr;
         s.alpha = d.alpha;
         s.beta = d.beta;
-        classify(dtype_, s, eps_, &r->nonneg, &r->packable);
+        classify(dtype_, false, s, eps_, &r->nonneg, &r->packable);
         r->want_lm = want_lm != 0;
         r->max_iter = max_iter;
         r->L = plan_instance(dtype_, r->x, r->y, r->z, false);
@@ -337,7 +337,7 @@ class Server {
         const std::vector<BldInst> desc{make_desc(r.L, dev_buf_.as<char>(r.off), eps_, r.a, r.b, false, r.nonneg)};
         const size_t need = LivePlan::scratch_bytes(lay);
         if (scratch_.bytes < need) scratch_ = DeviceBuffer(need);
-        r.live = LivePlan(dtype_, desc, lay, {true}, scratch_.as<char>(), [&](size_t n) -> void* {
+        r.live = LivePlan(dtype_, false, desc, lay, {true}, scratch_.as<char>(), [&](size_t n) -> void* {
             std::lock_guard<std::mutex> lk(mu_);
             size_t waiting = 0;
             for (const auto& q : queue_) waiting += align_up(q->L.bytes);

@@ -779,6 +779,12 @@ __global__ void __launch_bounds__(64)
     BNMF_GLOBAL uint16_t* fib = (BNMF_GLOBAL uint16_t*)t->fib;
     BNMF_GLOBAL T* xv = (BNMF_GLOBAL T*)t->xv;
     BNMF_GLOBAL uint16_t* map = (BNMF_GLOBAL uint16_t*)t->map;
+    // FP32: the lanes past the last fiber of its group of 64 read their place
+    // and X; whatever their S is stays theirs
+    if (sizeof(T) == 4 && n + lane < (n + 63u) / 64u * 64u) {
+        fib[n + lane] = 0;
+        xv[n + lane] = T(0);
+    }
     const uint32_t q0 = pos;
     uint32_t per[kClasses] = {0u, 0u, 0u, 0u};
     for (uint32_t cls = 0; cls < kClasses; ++cls) {

@@ -251,10 +251,11 @@ class LivePlan {
     // Counts the nonempty fibers of the candidates' tiles (X and the tile
     // plan from the descriptors) and lays the packed buffers out.
     // scratch: device memory of scratch_bytes, used until the call returns; it
-    // starts with the descriptors. mem: where the packed buffers come from and
-    // are given back to (null for none left); without it they are the plan's own.
+    // starts with the descriptors. mem(n, bytes): where the packed buffers of
+    // instance n come from and are given back to (null for none left); without it
+    // they are the plan's own.
     LivePlan(int dtype, bool add, const std::vector<BldInst>& descs, const std::vector<InstLayout>& lay,
-             const std::vector<bool>& candidate, char* scratch, const std::function<void*(size_t)>& mem = nullptr);
+             const std::vector<bool>& candidate, char* scratch, const std::function<void*(size_t, size_t)>& mem = nullptr);
     LivePlan() = default;
     static size_t scratch_bytes(const std::vector<InstLayout>& lay);
     // Largest share of nonempty fibers at which an instance is packed; elements:
@@ -269,28 +270,25 @@ class LivePlan {
     uint32_t lds(size_t n) const { return lds_[n]; }
     size_t fibers(size_t n) const { return fibers_[n]; }  // its nonempty fibers
     size_t bytes() const { return bytes_; }
-    uint32_t n_tiles() const { return (uint32_t)tiles_.size(); }
     // Appends the tiles of one launch (items: batch instance numbers) to the
     // tile table and returns the first one's index.
     uint32_t add_launch(std::vector<PassItem>& items, const std::vector<BldInst>& descs);
     // Uploads the tile table and builds the lists; insts: the descriptors on
-    // the device
-    void build(const std::vector<BldInst>& descs, const BldInst* insts, hipStream_t st);
+    // the device. A plan whose buffers are not its own keeps its table on the
+    // host (host_tiles, complete once st is done) and only builds in tab.
+    void build(const std::vector<BldInst>& descs, const BldInst* insts, hipStream_t st, LiveTile* tab = nullptr);
     const LiveTile* tiles() const { return tab_; }
+    const std::vector<LiveTile>& host_tiles() const { return tiles_; }
     // packed S from S_src, and S from its packed form
     void gather(const BldInst* insts, hipStream_t st) const;
     void scatter(const BldInst* insts, hipStream_t st) const;
 
    private:
     struct Off {
+        char* base;  // of the instance's buffers
         size_t Sc, fib, xv, rdesc, cdesc, map, smap, tile0;
     };
-    template <typename T>
-    T* at(size_t off) const {
-        return reinterpret_cast<T*>(base_ + off);
-    }
     int dtype_ = 0;
-    char* base_ = nullptr;
     LiveTile* tab_ = nullptr;
     size_t bytes_ = 0;
     DeviceBuffer buf_;

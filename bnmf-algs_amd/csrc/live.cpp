@@ -97,7 +97,7 @@ double LivePlan::most_share(int dtype, bool add, size_t x, size_t y, uint32_t z,
 }
 
 LivePlan::LivePlan(int dtype, bool add, const std::vector<BldInst>& descs, const std::vector<InstLayout>& lay,
-                   const std::vector<bool>& candidate, char* scratch, const std::function<void*(size_t)>& mem)
+                   const std::vector<bool>& candidate, char* scratch, const std::function<void*(size_t, size_t)>& mem)
     : dtype_(dtype), offs_(descs.size()), fibers_(descs.size(), 0), lds_(descs.size(), 0) {
     const size_t es = dtype == BNMF_F32 ? 4 : 8;
     size_t elements = 0;
@@ -123,12 +123,9 @@ LivePlan::LivePlan(int dtype, bool add, const std::vector<BldInst>& descs, const
         BNMF_HIP(hipMemcpy(counts.data(), ct, items.size() * 4, hipMemcpyDeviceToHost));
     }
 
-    size_t off = 0;
-    auto take = [&](size_t n) {
-        const size_t o = off;
-        off = align_up(off + n);
-        return o;
-    };
+    // the packed form is extra memory: an instance without room for it runs the
+    // dense passes, with the same results
+    size_t all = 0;
     for (size_t at = 0; at < items.size();) {
         const size_t n = items[at].inst;
         const InstLayout& L = lay[n];
@@ -155,6 +152,12 @@ LivePlan::LivePlan(int dtype, bool add, const std::vector<BldInst>& descs, const
             if (ok) lds_[n] = (uint32_t)std::max(least, std::min(all, kLdsWant));
         }
         if (ok) {
+            size_t off = 0;
+            auto take = [&](size_t bytes) {
+                const size_t o = off;
+                off = align_up(off + bytes);
+                return o;
+            };
             fibers_[n] = (size_t)total;
             Off& o = offs_[n];
             o.Sc = take((size_t)(slots / gf) * ge * es);
@@ -164,36 +167,35 @@ LivePlan::LivePlan(int dtype, bool add, const std::vector<BldInst>& descs, const
             o.cdesc = take(nt * L.tile_cols * sizeof(LiveCol));
             o.map = take(nt * L.ti_rows * L.tile_cols * 2);
             o.smap = take(nt * L.ti_rows * L.tile_cols * 2);
+            o.base = reinterpret_cast<char*>(all);  // without mem: an offset so far
+            if (mem)
+                o.base = static_cast<char*>(mem(n, off));
+            else
+                all += off;
+            if (mem && !o.base) {
+                lds_[n] = 0;
+                at += nt;
+                continue;
+            }
             o.tile0 = slot_.size();
             slot_.insert(slot_.end(), slot.begin(), slot.end());
             count_.insert(count_.end(), counts.begin() + at, counts.begin() + at + nt);
         }
         at += nt;
     }
-    if (slot_.empty()) return;
-    const size_t off_tab = take(slot_.size() * sizeof(LiveTile));
-    // the packed form is extra memory: without room for it every instance
-    // runs the dense passes, with the same results
-    {
-        void* p = mem ? mem(off) : nullptr;
-        if (!mem && hipMalloc(&p, off) != hipSuccess) {
-            (void)hipGetLastError();
-            p = nullptr;
-        }
-        if (!p) {
-            std::fill(lds_.begin(), lds_.end(), 0u);
-            return;
-        }
-        base_ = static_cast<char*>(p);
-        tab_ = at<LiveTile>(off_tab);
-        bytes_ = off;
-        if (!mem) {
-            buf_.ptr = p;
-            buf_.bytes = off;
-        }
+    if (mem || slot_.empty()) return;
+    const size_t off_tab = all;
+    all = align_up(all + slot_.size() * sizeof(LiveTile));
+    void* p = nullptr;
+    if (hipMalloc(&p, all) != hipSuccess) {
+        (void)hipGetLastError();
+        std::fill(lds_.begin(), lds_.end(), 0u);
+        return;
     }
-    // slots past a tile's fibers are read as zeros
-    BNMF_HIP(hipMemset(base_, 0, off));
+    buf_.ptr = p;
+    buf_.bytes = bytes_ = all;
+    for (Off& o : offs_) o.base = buf_.as<char>((size_t)o.base);
+    tab_ = buf_.as<LiveTile>(off_tab);
 }
 
 uint32_t LivePlan::add_launch(std::vector<PassItem>& items, const std::vector<BldInst>& descs) {
@@ -215,13 +217,13 @@ uint32_t LivePlan::add_launch(std::vector<PassItem>& items, const std::vector<Bl
         uint32_t ge = 0, gf = 0;
         live_group(dtype_, d.z, &ge, &gf);
         LiveTile t{};
-        t.Sc = at<char>(o.Sc + slot / gf * ge * es);
-        t.fib = at<uint16_t>(o.fib) + slot;
-        t.xv = at<char>(o.xv + slot * es);
-        t.rdesc = at<LiveRow>(o.rdesc) + tile * d.ti_rows;
-        t.cdesc = at<LiveCol>(o.cdesc) + tile * d.tile_cols;
-        t.map = at<uint16_t>(o.map) + tile * d.ti_rows * d.tile_cols;
-        t.smap = at<uint16_t>(o.smap) + tile * d.ti_rows * d.tile_cols;
+        t.Sc = o.base + o.Sc + slot / gf * ge * es;
+        t.fib = reinterpret_cast<uint16_t*>(o.base + o.fib) + slot;
+        t.xv = o.base + o.xv + slot * es;
+        t.rdesc = reinterpret_cast<LiveRow*>(o.base + o.rdesc) + tile * d.ti_rows;
+        t.cdesc = reinterpret_cast<LiveCol*>(o.base + o.cdesc) + tile * d.tile_cols;
+        t.map = reinterpret_cast<uint16_t*>(o.base + o.map) + tile * d.ti_rows * d.tile_cols;
+        t.smap = reinterpret_cast<uint16_t*>(o.base + o.smap) + tile * d.ti_rows * d.tile_cols;
         t.psib = static_cast<const char*>(d.psib) + j0 * z * es;
         t.psia = static_cast<const char*>(d.psia) + i0 * z * es;
         t.psiA = d.psiA;
@@ -244,11 +246,14 @@ uint32_t LivePlan::add_launch(std::vector<PassItem>& items, const std::vector<Bl
     return first;
 }
 
-void LivePlan::build(const std::vector<BldInst>& descs, const BldInst* insts, hipStream_t st) {
+void LivePlan::build(const std::vector<BldInst>& descs, const BldInst* insts, hipStream_t st, LiveTile* tab) {
     if (!any()) return;
+    const size_t bytes = tiles_.size() * sizeof(LiveTile);
     for (LiveTile& t : tiles_) t.iter = descs[t.inst].iter;
-    BNMF_HIP(hipMemcpy(tab_, tiles_.data(), tiles_.size() * sizeof(LiveTile), hipMemcpyHostToDevice));
-    BNMF_HIP(launch_live_build(dtype_, insts, tab_, (uint32_t)tiles_.size(), st));
+    LiveTile* const dev = tab ? tab : tab_;
+    BNMF_HIP(hipMemcpy(dev, tiles_.data(), bytes, hipMemcpyHostToDevice));
+    BNMF_HIP(launch_live_build(dtype_, insts, dev, (uint32_t)tiles_.size(), st));
+    if (tab) BNMF_HIP(hipMemcpyAsync(tiles_.data(), dev, bytes, hipMemcpyDeviceToHost, st));
 }
 
 void LivePlan::gather(const BldInst* insts, hipStream_t st) const {

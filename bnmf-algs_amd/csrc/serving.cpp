@@ -56,9 +56,12 @@ struct Request {
     uint64_t seed = 0;
     bool has_S0 = false, want_lm = false;
     bool nonneg = false, packable = false;  // classify
-    // its packed nonempty fibers while it is active, in arena bytes of their own
-    LivePlan live;
-    size_t live_off = 0, live_bytes = 0;
+    // its packed nonempty fibers while it is active (their tiles; none: dense), in
+    // arena bytes of their own
+    std::vector<LiveTile> tiles;
+    uint32_t live_lds = 0;
+    size_t fibers = 0, live_off = 0, live_bytes = 0;
+    bool packed() const { return !tiles.empty(); }
     size_t max_iter = 0, done_iter = 0;
     InstLayout L{};
     size_t off = 0;
@@ -258,8 +261,9 @@ class Server {
         size_t off_desc = 0, off_prep = 0, off_prep_count = 0;
         uint32_t n_prep = 0, n_inst = 0;
         LaneWS lanes[4];
-        // the packed requests' tiles within the work lists
-        std::vector<std::pair<size_t, const Request*>> tiles;
+        // tiles of the packed requests that start, and that end, with this step
+        size_t off_gather = 0, off_scatter = 0;
+        uint32_t n_gather = 0, n_scatter = 0;
     };
 
     void loop() {
@@ -284,7 +288,7 @@ class Server {
                 peak_bytes_ = std::max(peak_bytes_, arena_.used());
             }
             try {
-                for (auto& r : admitted) upload(*r);
+                upload(admitted);
                 std::vector<std::shared_ptr<Request>> act;
                 {
                     std::lock_guard<std::mutex> lk(mu_);
@@ -306,56 +310,87 @@ class Server {
         return !queue_.empty() && active_.size() < max_active_ && arena_.fits(queue_.front()->L.bytes);
     }
 
-    void upload(Request& r) {
-        char* base = dev_buf_.as<char>(r.off);
-        const InstLayout& L = r.L;
-        const size_t xy = (size_t)r.x * r.y;
-        if (L.elements() == 0) return;
-        BNMF_HIP(hipMemcpyAsync(base + L.off_X, r.X.data(), xy * es_, hipMemcpyHostToDevice, stream_));
-        BNMF_HIP(hipMemcpyAsync(base + L.off_alpha, r.alpha.data(), r.x * 8, hipMemcpyHostToDevice, stream_));
-        BNMF_HIP(hipMemcpyAsync(base + L.off_beta, r.beta.data(), r.z * 8, hipMemcpyHostToDevice, stream_));
-        if (r.has_S0) {
-            BNMF_HIP(hipMemcpyAsync(base + L.off_S, r.S0.data(), L.elements() * es_, hipMemcpyHostToDevice,
-                                    stream_));
-        } else {
-            BNMF_HIP(launch_init_s(dtype_, base + L.off_S, base + L.off_X, xy, r.z, r.seed, stream_));
+    void upload(const std::vector<std::shared_ptr<Request>>& admitted) {
+        if (admitted.empty()) return;
+        for (const auto& p : admitted) {
+            Request& r = *p;
+            char* base = dev_buf_.as<char>(r.off);
+            const InstLayout& L = r.L;
+            const size_t xy = (size_t)r.x * r.y;
+            if (L.elements() == 0) continue;
+            BNMF_HIP(hipMemcpyAsync(base + L.off_X, r.X.data(), xy * es_, hipMemcpyHostToDevice, stream_));
+            BNMF_HIP(hipMemcpyAsync(base + L.off_alpha, r.alpha.data(), r.x * 8, hipMemcpyHostToDevice, stream_));
+            BNMF_HIP(hipMemcpyAsync(base + L.off_beta, r.beta.data(), r.z * 8, hipMemcpyHostToDevice, stream_));
+            if (r.has_S0) {
+                BNMF_HIP(hipMemcpyAsync(base + L.off_S, r.S0.data(), L.elements() * es_, hipMemcpyHostToDevice,
+                                        stream_));
+            } else {
+                BNMF_HIP(launch_init_s(dtype_, base + L.off_S, base + L.off_X, xy, r.z, r.seed, stream_));
+            }
         }
         // the host copies are dropped once the stream has consumed them
         BNMF_HIP(hipStreamSynchronize(stream_));
-        r.X.clear();
-        r.X.shrink_to_fit();
-        r.S0.clear();
-        r.S0.shrink_to_fit();
-        if (r.packable) pack(r);
+        for (const auto& p : admitted) {
+            p->X.clear();
+            p->X.shrink_to_fit();
+            p->S0.clear();
+            p->S0.shrink_to_fit();
+        }
+        pack(admitted);
     }
 
-    // The nonempty fibers' lists, in arena memory that no queued request waits for
-    // (only the tile table, some 150 bytes a tile, lies outside);
-    // without it the request runs the dense passes, with the same results.
-    void pack(Request& r) {
-        const std::vector<InstLayout> lay{r.L};
-        const std::vector<BldInst> desc{make_desc(r.L, dev_buf_.as<char>(r.off), eps_, r.a, r.b, false, r.nonneg)};
-        const size_t need = LivePlan::scratch_bytes(lay);
-        if (scratch_.bytes < need) scratch_ = DeviceBuffer(need);
-        r.live = LivePlan(dtype_, false, desc, lay, {true}, scratch_.as<char>(), [&](size_t n) -> void* {
-            std::lock_guard<std::mutex> lk(mu_);
-            size_t waiting = 0;
-            for (const auto& q : queue_) waiting += align_up(q->L.bytes);
-            if (arena_.used() + waiting + align_up(n) > arena_.capacity() || !arena_.alloc(align_up(n), &r.live_off))
-                return nullptr;
-            r.live_bytes = align_up(n);
-            peak_bytes_ = std::max(peak_bytes_, arena_.used());
-            return dev_buf_.as<char>(r.live_off);
-        });
-        if (!r.live.live(0)) return;
-        std::vector<PassItem> items;
-        for (uint32_t ti = 0; ti < r.L.n_ti; ++ti)
-            for (uint32_t tj = 0; tj < r.L.n_tj; ++tj) items.push_back(PassItem{0, ti, tj, 0});
-        r.live.add_launch(items, desc);
-        r.live.build(desc, scratch_.as<BldInst>(), stream_);
+    // The nonempty fibers' lists of the requests admitted together, each in arena
+    // memory that no queued request waits for; without it a request runs the
+    // dense passes, with the same results. The tile tables stay on the host and
+    // go to the device with each step's work lists.
+    void pack(const std::vector<std::shared_ptr<Request>>& admitted) {
+        std::vector<Request*> set;
+        std::vector<InstLayout> lay;
+        std::vector<BldInst> desc;
+        size_t tiles = 0;
+        for (const auto& p : admitted) {
+            Request& r = *p;
+            if (!r.packable || r.L.elements() == 0) continue;
+            set.push_back(&r);
+            lay.push_back(r.L);
+            desc.push_back(make_desc(r.L, dev_buf_.as<char>(r.off), eps_, r.a, r.b, false, r.nonneg));
+            tiles += (size_t)r.L.n_ti * r.L.n_tj;
+        }
+        if (set.empty()) return;
+        const size_t off_tab = align_up(LivePlan::scratch_bytes(lay)), need = off_tab + tiles * sizeof(LiveTile);
+        if (scratch_.bytes < need) scratch_ = DeviceBuffer(std::max(need, 2 * scratch_.bytes));
+        LivePlan plan(dtype_, false, desc, lay, std::vector<bool>(set.size(), true), scratch_.as<char>(),
+                      [&](size_t n, size_t bytes) -> void* {
+                          Request& r = *set[n];
+                          bytes = align_up(bytes);
+                          std::lock_guard<std::mutex> lk(mu_);
+                          size_t waiting = 0;
+                          for (const auto& q : queue_) waiting += align_up(q->L.bytes);
+                          if (arena_.used() + waiting + bytes > arena_.capacity() || !arena_.alloc(bytes, &r.live_off))
+                              return nullptr;
+                          r.live_bytes = bytes;
+                          peak_bytes_ = std::max(peak_bytes_, arena_.used());
+                          return dev_buf_.as<char>(r.live_off);
+                      });
+        std::vector<size_t> first(set.size(), 0);
+        for (size_t n = 0; n < set.size(); ++n) {
+            if (!plan.live(n)) continue;
+            std::vector<PassItem> items;
+            for (uint32_t ti = 0; ti < lay[n].n_ti; ++ti)
+                for (uint32_t tj = 0; tj < lay[n].n_tj; ++tj) items.push_back(PassItem{(uint32_t)n, ti, tj, 0});
+            first[n] = plan.add_launch(items, desc);
+        }
+        if (!plan.any()) return;
+        plan.build(desc, scratch_.as<BldInst>(), stream_, scratch_.as<LiveTile>(off_tab));
         BNMF_HIP(hipStreamSynchronize(stream_));
+        for (size_t n = 0; n < set.size(); ++n) {
+            if (!plan.live(n)) continue;
+            const LiveTile* const t = plan.host_tiles().data() + first[n];
+            set[n]->tiles.assign(t, t + (size_t)lay[n].n_ti * lay[n].n_tj);
+            set[n]->live_lds = plan.lds(n);
+            set[n]->fibers = plan.fibers(n);
+        }
     }
-
 
     // Builds descriptors and the work lists of `mode` passes for `set` in the
     // meta buffer region starting at `moff`; returns the end offset.
@@ -378,11 +413,11 @@ class Server {
             BldInst d = make_desc(L, dev_buf_.as<char>(r.off), eps_, r.a, r.b, false, r.nonneg);
             desc.push_back(d);
             if (L.elements() == 0) continue;
-            const PassKey key = pass_key(dtype_, mode, L, r.nonneg, r.live.live(0));
+            const PassKey key = pass_key(dtype_, mode, L, r.nonneg, r.packed());
             zmax[key] = std::max(zmax[key], L.z);
             members[key].push_back((uint32_t)n);
             // a packed element costs about three streamed ones
-            work[key] += key.live ? 3 * r.live.fibers(0) * L.z : L.elements();
+            work[key] += key.live ? 3 * r.fibers * L.z : L.elements();
             for (uint32_t c = 0; c < L.n_cj; ++c) prep.push_back(PrepItem{(uint32_t)n, 0, c, 0});
             for (uint32_t c = 0; c < L.nA; ++c) prep.push_back(PrepItem{(uint32_t)n, 1, c, 0});
         }
@@ -410,7 +445,7 @@ class Server {
             l.lane = (int)(std::min_element(load.begin(), load.end()) - load.begin());
             load[l.lane] += l.work;
             std::vector<PassItem> items;
-            uint32_t tiles = 0;
+            std::vector<LiveTile> tiles;
             for (uint32_t n : members[o.second]) {
                 uint32_t idx = n;
                 if (per_lane) {
@@ -419,23 +454,18 @@ class Server {
                 }
                 const InstLayout& L = set[n]->L;
                 if (l.key.live) {
-                    tiles += set[n]->live.n_tiles();
-                    l.lds = std::max(l.lds, set[n]->live.lds(0));
+                    tiles.insert(tiles.end(), set[n]->tiles.begin(), set[n]->tiles.end());
+                    l.lds = std::max(l.lds, set[n]->live_lds);
                     continue;
                 }
                 for (uint32_t ti = 0; ti < L.n_ti; ++ti)
                     for (uint32_t tj = 0; tj < L.n_tj; ++tj) items.push_back(PassItem{idx, ti, tj, 0});
             }
             if (l.key.live) {
-                // one launch for the packed requests, whose tiles are gathered
-                // on the device
-                l.n = tiles;
-                l.off_items = take(tiles * sizeof(LiveTile));
-                size_t at = l.off_items;
-                for (uint32_t n : members[o.second]) {
-                    ws.tiles.push_back({at, set[n]});
-                    at += set[n]->live.n_tiles() * sizeof(LiveTile);
-                }
+                // one launch for the packed requests
+                l.n = (uint32_t)tiles.size();
+                l.off_items = take(tiles.size() * sizeof(LiveTile));
+                std::memcpy(host.data() + l.off_items, tiles.data(), tiles.size() * sizeof(LiveTile));
                 ws.launches.push_back(l);
                 continue;
             }
@@ -554,23 +584,39 @@ class Server {
         std::vector<char> host;
         WorkSet ws_all, ws_fresh;
         size_t end = build(all, ws_all, host, 0, MODE_UPDATE);
+        // tiles of the requests whose S goes to its packed form before this step's
+        // iterations, or back after them (a request of no iterations keeps the S0 it
+        // was given: no step has left a psi(A) for the scatter to read)
+        auto list_tiles = [&](size_t* off, uint32_t* count, auto&& pick) {
+            std::vector<LiveTile> tiles;
+            for (size_t n = 0; n < all.size(); ++n) {
+                if (!pick(*all[n])) continue;
+                const size_t from = tiles.size();
+                tiles.insert(tiles.end(), all[n]->tiles.begin(), all[n]->tiles.end());
+                for (size_t t = from; t < tiles.size(); ++t) tiles[t].inst = (uint32_t)n;
+            }
+            *off = end;
+            *count = (uint32_t)tiles.size();
+            end = align_up(end + tiles.size() * sizeof(LiveTile));
+            host.resize(std::max(host.size(), end));
+            if (!tiles.empty()) std::memcpy(host.data() + *off, tiles.data(), tiles.size() * sizeof(LiveTile));
+        };
+        list_tiles(&ws_all.off_gather, &ws_all.n_gather, [](const Request& r) { return r.fresh && r.max_iter > 0; });
+        list_tiles(&ws_all.off_scatter, &ws_all.n_scatter,
+                   [&](const Request& r) { return r.max_iter > 0 && r.done_iter + k_iters >= r.max_iter; });
         if (!fresh.empty()) end = build(fresh, ws_fresh, host, end, MODE_SUMS);
         ensure_meta(end);
         BNMF_HIP(hipMemcpyAsync(meta_.ptr, host.data(), end, hipMemcpyHostToDevice, stream_));
         char* m = meta_.as<char>();
-        for (const auto& t : ws_all.tiles)
-            BNMF_HIP(hipMemcpyAsync(m + t.first, t.second->live.tiles(), t.second->live.n_tiles() * sizeof(LiveTile),
-                                    hipMemcpyDeviceToDevice, stream_));
         const BldInst* desc = reinterpret_cast<const BldInst*>(m + ws_all.off_desc);
         if (!fresh.empty()) passes(ws_fresh, MODE_SUMS);
-        for (size_t n = 0; n < all.size(); ++n)
-            if (all[n]->fresh) all[n]->live.gather(desc + n, stream_);
+        if (ws_all.n_gather)
+            BNMF_HIP(launch_live_gather(dtype_, desc, reinterpret_cast<const LiveTile*>(m + ws_all.off_gather),
+                                        ws_all.n_gather, stream_));
         iterate(ws_all, k_iters);
-        // (a request of no iterations keeps the S0 it was given: no step has left a
-        // psi(A) for the scatter to read)
-        for (size_t n = 0; n < all.size(); ++n)
-            if (all[n]->max_iter > 0 && all[n]->done_iter + k_iters >= all[n]->max_iter)
-                all[n]->live.scatter(desc + n, stream_);
+        if (ws_all.n_scatter)
+            BNMF_HIP(launch_live_scatter(dtype_, desc, reinterpret_cast<const LiveTile*>(m + ws_all.off_scatter),
+                                         ws_all.n_scatter, stream_));
         // requests that finish in this step, scored if asked
         std::vector<Request*> fin, score;
         for (Request* r : all) {
@@ -608,7 +654,7 @@ class Server {
         }
         BNMF_HIP(hipStreamSynchronize(stream_));
         const double t1 = now_s();
-        for (Request* r : fin) r->live = LivePlan();
+        for (Request* r : fin) r->tiles = {};
         std::lock_guard<std::mutex> lk(mu_);
         busy_s_ += t1 - t0;
         ++steps_;

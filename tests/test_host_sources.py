@@ -24,11 +24,11 @@ def objects(tmp_path_factory):
     return [str(out / (os.path.basename(f) + ".o")) for f in files]
 
 
-def _run(objects, tmp_path, name):
+def _run(objects, tmp_path, name, *args):
     exe = str(tmp_path / name)
     subprocess.run(["g++", *FLAGS, os.path.join(CPP, name + ".cpp"), *objects, "-o", exe, "-lpthread", "-ldl"], check=True)
     env = {**os.environ, "ASAN_OPTIONS": "verify_asan_link_order=0"}
-    r = subprocess.run([exe], capture_output=True, text=True, timeout=300, env=env)
+    r = subprocess.run([exe, *args], capture_output=True, text=True, timeout=300, env=env)
     assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-3000:]
     assert " ok" in r.stdout
 
@@ -51,3 +51,8 @@ def test_calls_of_few_iterations(objects, tmp_path):
 
 def test_share_from_a_sample(objects, tmp_path):
     _run(objects, tmp_path, "test_worth")
+
+
+@pytest.mark.parametrize("what", ["small"])
+def test_server_memory(objects, tmp_path, what):
+    _run(objects, tmp_path, "test_server_memory", what)

@@ -358,7 +358,16 @@ class Server {
         }
         if (set.empty()) return;
         const size_t off_tab = align_up(LivePlan::scratch_bytes(lay)), need = off_tab + tiles * sizeof(LiveTile);
-        if (scratch_.bytes < need) scratch_ = DeviceBuffer(std::max(need, 2 * scratch_.bytes));
+        if (scratch_.bytes < need) {
+            void* p = nullptr;
+            if (hipMalloc(&p, need) != hipSuccess) {
+                (void)hipGetLastError();
+                return;
+            }
+            scratch_ = DeviceBuffer();
+            scratch_.ptr = p;
+            scratch_.bytes = need;
+        }
         LivePlan plan(dtype_, false, desc, lay, std::vector<bool>(set.size(), true), scratch_.as<char>(),
                       [&](size_t n, size_t bytes) -> void* {
                           Request& r = *set[n];
@@ -508,6 +517,40 @@ class Server {
         meta_ = DeviceBuffer(std::max(bytes, meta_.bytes * 2));
     }
 
+    // ensure_meta, false where device memory runs out
+    bool try_meta(size_t bytes) {
+        try {
+            ensure_meta(bytes);
+        } catch (const Error& e) {
+            if (e.status != BNMF_ERR_OUT_OF_MEMORY) throw;
+            (void)hipGetLastError();
+            return false;
+        }
+        return true;
+    }
+
+    // A packed request goes on over the dense passes, with the same results: S
+    // back from its packed form (where an iteration has changed it) and the arena
+    // bytes given back. Its tiles were in the last step's work lists, so they fit
+    // the meta buffer.
+    void unpack(Request& r) {
+        if (!r.packed()) return;
+        if (r.done_iter > 0) {
+            const BldInst desc = make_desc(r.L, dev_buf_.as<char>(r.off), eps_, r.a, r.b, false, r.nonneg);
+            const size_t off = align_up(sizeof(BldInst)), n = r.tiles.size();
+            for (LiveTile& t : r.tiles) t.inst = 0;
+            BNMF_HIP(hipMemcpyAsync(meta_.ptr, &desc, sizeof(BldInst), hipMemcpyHostToDevice, stream_));
+            BNMF_HIP(hipMemcpyAsync(meta_.as<char>(off), r.tiles.data(), n * sizeof(LiveTile), hipMemcpyHostToDevice,
+                                    stream_));
+            BNMF_HIP(launch_live_scatter(dtype_, meta_.as<BldInst>(), meta_.as<LiveTile>(off), (uint32_t)n, stream_));
+            BNMF_HIP(hipStreamSynchronize(stream_));
+        }
+        r.tiles = {};
+        std::lock_guard<std::mutex> lk(mu_);
+        if (r.live_bytes) arena_.release(r.live_off, r.live_bytes);
+        r.live_bytes = 0;
+    }
+
     void passes(const WorkSet& ws, int mode) {
         char* m = meta_.as<char>();
         const BldInst* d = reinterpret_cast<const BldInst*>(m + ws.off_desc);
@@ -583,7 +626,7 @@ class Server {
         }
         std::vector<char> host;
         WorkSet ws_all, ws_fresh;
-        size_t end = build(all, ws_all, host, 0, MODE_UPDATE);
+        size_t end = 0;
         // tiles of the requests whose S goes to its packed form before this step's
         // iterations, or back after them (a request of no iterations keeps the S0 it
         // was given: no step has left a psi(A) for the scatter to read)
@@ -601,11 +644,23 @@ class Server {
             host.resize(std::max(host.size(), end));
             if (!tiles.empty()) std::memcpy(host.data() + *off, tiles.data(), tiles.size() * sizeof(LiveTile));
         };
-        list_tiles(&ws_all.off_gather, &ws_all.n_gather, [](const Request& r) { return r.fresh && r.max_iter > 0; });
-        list_tiles(&ws_all.off_scatter, &ws_all.n_scatter,
-                   [&](const Request& r) { return r.max_iter > 0 && r.done_iter + k_iters >= r.max_iter; });
-        if (!fresh.empty()) end = build(fresh, ws_fresh, host, end, MODE_SUMS);
-        ensure_meta(end);
+        auto lists = [&] {
+            host.clear();
+            ws_all = WorkSet();
+            ws_fresh = WorkSet();
+            end = build(all, ws_all, host, 0, MODE_UPDATE);
+            list_tiles(&ws_all.off_gather, &ws_all.n_gather, [](const Request& r) { return r.fresh && r.max_iter > 0; });
+            list_tiles(&ws_all.off_scatter, &ws_all.n_scatter,
+                       [&](const Request& r) { return r.max_iter > 0 && r.done_iter + k_iters >= r.max_iter; });
+            if (!fresh.empty()) end = build(fresh, ws_fresh, host, end, MODE_SUMS);
+        };
+        lists();
+        if (!try_meta(end)) {
+            // the dense passes' lists are a tenth of the packed fibers'
+            for (Request* r : all) unpack(*r);
+            lists();
+            ensure_meta(end);
+        }
         BNMF_HIP(hipMemcpyAsync(meta_.ptr, host.data(), end, hipMemcpyHostToDevice, stream_));
         char* m = meta_.as<char>();
         const BldInst* desc = reinterpret_cast<const BldInst*>(m + ws_all.off_desc);
@@ -632,9 +687,14 @@ class Server {
             WorkSet ws_sc;
             std::vector<char> h2;
             const size_t e2 = build(score, ws_sc, h2, 0, MODE_SCORE);
-            // a second region after the step's lists, so they stay valid
-            const size_t base = align_up(end);
-            ensure_meta(base + e2);
+            // a second region after the step's lists, which are still in use; or
+            // in their place, once they are not
+            size_t base = align_up(end);
+            if (!try_meta(base + e2)) {
+                BNMF_HIP(hipStreamSynchronize(stream_));
+                base = 0;
+                ensure_meta(e2);
+            }
             m = meta_.as<char>();
             for (auto& l : ws_sc.launches) {
                 l.off_items += base;

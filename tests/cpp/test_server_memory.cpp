@@ -53,6 +53,14 @@ static void full_device() {
     CHECK(bnmf_server_wait(s, t1, 30.0) == BNMF_OK, "a packable request on a full device");
     const uint64_t t2 = submit(s, dense, 100);
     CHECK(bnmf_server_wait(s, t2, 30.0) == BNMF_OK, "the next one");
+    // room for the packing's own scratch, not for longer work lists; several at once
+    fake::reset(fake::in_use() + 16384);
+    std::vector<uint64_t> t;
+    for (int k = 0; k < 6; ++k) {
+        t.push_back(submit(s, k % 3 ? sparse : dense, 30 + 10 * k));
+        if (k == 2) CHECK(bnmf_server_wait(s, t[0], 30.0) == BNMF_OK, "the first of several");
+    }
+    for (uint64_t k : t) CHECK(bnmf_server_wait(s, k, 30.0) == BNMF_OK, "one of several");
     bnmf_server_destroy(s);
     fake::reset();
     CHECK(fake::in_use() == 0, "%zu bytes left", fake::in_use());

@@ -270,24 +270,24 @@ class Server {
         (void)hipSetDevice(dev_);
         std::vector<std::shared_ptr<Request>> admitted;
         for (;;) {
-            {
-                std::unique_lock<std::mutex> lk(mu_);
-                cv_.wait(lk, [&] { return stop_ || !active_.empty() || can_admit_locked(); });
-                if (stop_) return;
-                admitted.clear();
-                while (!queue_.empty() && active_.size() + admitted.size() < max_active_) {
-                    auto& r = queue_.front();
-                    size_t off;
-                    if (!arena_.alloc(r->L.bytes, &off)) break;
-                    r->off = off;
-                    r->state = RS_ACTIVE;
-                    r->t_admit = now_s();
-                    admitted.push_back(r);
-                    queue_.pop_front();
-                }
-                peak_bytes_ = std::max(peak_bytes_, arena_.used());
-            }
             try {
+                {
+                    std::unique_lock<std::mutex> lk(mu_);
+                    cv_.wait(lk, [&] { return stop_ || !active_.empty() || can_admit_locked(); });
+                    if (stop_) return;
+                    admitted.clear();
+                    admit_locked(admitted);
+                    // packed fibers keep no request waiting
+                    for (;;) {
+                        const std::vector<Request*> give = in_the_way_locked(active_.size() + admitted.size());
+                        if (give.empty()) break;
+                        lk.unlock();
+                        for (Request* r : give) unpack(*r);
+                        lk.lock();
+                        admit_locked(admitted);
+                    }
+                    peak_bytes_ = std::max(peak_bytes_, arena_.used());
+                }
                 upload(admitted);
                 std::vector<std::shared_ptr<Request>> act;
                 {
@@ -303,6 +303,35 @@ class Server {
                 return;
             }
         }
+    }
+
+    // Requests from the head of the queue as far as slots and bytes go.
+    void admit_locked(std::vector<std::shared_ptr<Request>>& admitted) {
+        while (!queue_.empty() && active_.size() + admitted.size() < max_active_) {
+            auto& r = queue_.front();
+            size_t off;
+            if (!arena_.alloc(r->L.bytes, &off)) break;
+            r->off = off;
+            r->state = RS_ACTIVE;
+            r->t_admit = now_s();
+            admitted.push_back(r);
+            queue_.pop_front();
+        }
+    }
+
+    // The active requests, latest first, whose packed fibers have to go for the
+    // queue head to fit; none if it fits now or would not fit even so.
+    std::vector<Request*> in_the_way_locked(size_t n_active) const {
+        std::vector<Request*> out;
+        if (queue_.empty() || n_active >= max_active_ || arena_.fits(queue_.front()->L.bytes)) return out;
+        Arena then = arena_;
+        for (auto it = active_.rbegin(); it != active_.rend(); ++it) {
+            if ((*it)->live_bytes == 0) continue;
+            then.release((*it)->live_off, (*it)->live_bytes);
+            out.push_back(it->get());
+            if (then.fits(queue_.front()->L.bytes)) return out;
+        }
+        return {};
     }
 
     // The queue head can start now: a slot is free and its bytes fit.

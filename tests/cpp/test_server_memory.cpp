@@ -107,11 +107,26 @@ static void small_requests() {
     bnmf_server_destroy(s);
 }
 
+// requests of few iterations are not packed, others are
+static void few_iterations() {
+    bnmf_server* s = nullptr;
+    CHECK(bnmf_server_create(&s, BNMF_F32, (size_t)1 << 28, 0, 1, 1e-50) == BNMF_OK, "create");
+    Problem small(64, 64, 8, 0.05), large(512, 300, 32, 0.05);
+    for (Problem* p : {&small, &large})
+        for (size_t iters : {0, 1, 8, 64}) {
+            fake::reset();
+            CHECK(bnmf_server_wait(s, submit(s, *p, iters), 30.0) == BNMF_OK, "request");
+            CHECK((fake::packs > 0) == (iters == 64), "%zu iterations: packed %zu", iters, fake::packs.load());
+        }
+    bnmf_server_destroy(s);
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "full") full_device();
     if (what == "later") later_request();
     if (what == "small") small_requests();
+    if (what == "few") few_iterations();
     if (failures) return 1;
     std::printf("server memory ok\n");
     return 0;

@@ -440,14 +440,24 @@ void Batch::plan(const std::vector<InstSpec>& specs, Extras extras) {
     // theirs, and the tiny ones cost it next to nothing.
     if (dtype == BNMF_F64 && algo_ == BNMF_ALGO_MULT) {
         bool all = true;
+        size_t count = 0, elements = 0, shallow = 0;
         for (const InstLayout& L : layouts_) {
             if (L.elements() == 0) continue;
+            ++count;
+            elements += L.elements();
+            if (L.x < 12 && L.elements() > 1024) shallow += L.elements();
             all = all && L.n_ti == 1 && L.n_tj == 1 && L.z <= kFusedZ && L.x <= 64 && L.elements() <= kTinyElems &&
                   tiny_lds(L.x, L.y, L.z) <= kTinyLds;
             if (!all) break;
             tiny_threads_ = std::max(tiny_threads_, tiny_threads(L.x, L.y, L.z));
             tiny_lds_ = std::max(tiny_lds_, tiny_lds(L.x, L.y, L.z));
         }
+        // Four blocks to a CU or more, and what counts is their throughput: with
+        // few rows most of a block idles in the row and column sums. An
+        // iteration of 4096 instances, tiny and by the passes: 4x32x32 250 and 191
+        // us, 4x16x64 243 and 204, 8x32x16 198 and 191, 8x16x32 236 and 243, 16x32x8
+        // 150 and 185, 8x8x8 65 and 105.
+        if (count > 1024 && 2 * shallow > elements) all = false;
         if (!all) tiny_threads_ = 0;
         if (tiny_threads_) packable.assign(specs.size(), false);
     }

@@ -9,6 +9,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <vector>
 
 #include "../../bnmf-algs_amd/csrc/bnmf_internal.hpp"
 
@@ -16,6 +17,8 @@ namespace fake {
 std::mutex mu;
 std::map<void*, size_t> blocks;
 size_t used = 0, capacity = ~(size_t)0, fail_at = 0, mallocs = 0, pins = 0;
+bool tiny = false;
+std::vector<uint32_t> tiny_iters;
 std::atomic<size_t> copies{0}, launches{0}, packs{0};
 
 void reset(size_t cap, size_t fail) {
@@ -157,7 +160,7 @@ void read_layout(int, uint32_t z, uint32_t* rw, uint32_t* hs, uint32_t* hm) {
     *hs = *hm = 0;
 }
 int wide_regs_nk(uint32_t z) { return z <= 256 ? (int)((z + 63) / 64) : 0; }
-size_t tiny_lds(uint32_t, uint32_t, uint32_t) { return kTinyLds + 1; }
+size_t tiny_lds(uint32_t x, uint32_t y, uint32_t z) { return fake::tiny ? (size_t)2 * x * y * z * 8 : kTinyLds + 1; }
 uint32_t tiny_threads(uint32_t, uint32_t, uint32_t) { return 64; }
 size_t live_lds_need(int, uint32_t, uint32_t, uint32_t, uint32_t n, uint32_t) { return 4096 + n; }
 void live_group(int dtype, uint32_t z, uint32_t* elems, uint32_t* fibers) {
@@ -173,7 +176,10 @@ hipError_t launch_pass_live(int, int, int, bool, uint32_t, hipStream_t, const Li
 hipError_t launch_prep(int, int, bool, dim3, hipStream_t, const BldInst*, const PrepItem*, const uint32_t*, uint32_t, uint32_t) { return launched(); }
 hipError_t launch_score(dim3, hipStream_t, const BldInst*, const PrepItem*, const uint32_t*, uint32_t) { return launched(); }
 hipError_t launch_fact(int, const BldInst*, uint32_t, uint32_t, double, double*, double*, double*, hipStream_t) { return launched(); }
-hipError_t launch_tiny(int, uint32_t, uint32_t, size_t, hipStream_t, const BldInst*, uint32_t) { return launched(); }
+hipError_t launch_tiny(int, uint32_t, uint32_t, size_t, hipStream_t, const BldInst*, uint32_t iters) {
+    fake::tiny_iters.push_back(iters);
+    return launched();
+}
 hipError_t launch_live_build(int, const BldInst*, LiveTile*, uint32_t, hipStream_t) {
     ++fake::packs;
     return launched();

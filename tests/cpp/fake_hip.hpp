@@ -3,6 +3,8 @@
 
 #include <atomic>
 #include <cstddef>
+#include <cstdint>
+#include <vector>
 
 namespace fake {
 // bytes of device memory from here on, and the number of the hipMalloc call
@@ -11,5 +13,7 @@ void reset(size_t capacity = ~(size_t)0, size_t fail_at = 0);
 size_t in_use();     // bytes of device memory
 size_t n_mallocs();  // since reset
 size_t n_pins();     // hipHostMalloc since reset
+extern bool tiny;                         // whole solves in one launch where the planner wants them
+extern std::vector<uint32_t> tiny_iters;  // iterations of each such launch
 extern std::atomic<size_t> copies, launches, packs;  // packs: launches that pack fibers
 }  // namespace fake

@@ -56,3 +56,8 @@ def test_share_from_a_sample(objects, tmp_path):
 @pytest.mark.parametrize("what", ["few", "full", "later", "small"])
 def test_server_memory(objects, tmp_path, what):
     _run(objects, tmp_path, "test_server_memory", what)
+
+
+@pytest.mark.parametrize("what", ["route"])
+def test_tiny_batches(objects, tmp_path, what):
+    _run(objects, tmp_path, "test_tiny_batches", what)

@@ -440,11 +440,12 @@ void Batch::plan(const std::vector<InstSpec>& specs, Extras extras) {
     // theirs, and the tiny ones cost it next to nothing.
     if (dtype == BNMF_F64 && algo_ == BNMF_ALGO_MULT) {
         bool all = true;
-        size_t count = 0, elements = 0, shallow = 0;
+        size_t count = 0, elements = 0, shallow = 0, most = 0;
         for (const InstLayout& L : layouts_) {
             if (L.elements() == 0) continue;
             ++count;
             elements += L.elements();
+            most = std::max(most, L.elements());
             if (L.x < 12 && L.elements() > 1024) shallow += L.elements();
             all = all && L.n_ti == 1 && L.n_tj == 1 && L.z <= kFusedZ && L.x <= 64 && L.elements() <= kTinyElems &&
                   tiny_lds(L.x, L.y, L.z) <= kTinyLds;
@@ -459,6 +460,11 @@ void Batch::plan(const std::vector<InstSpec>& specs, Extras extras) {
         // 150 and 185, 8x8x8 65 and 105.
         if (count > 1024 && 2 * shallow > elements) all = false;
         if (!all) tiny_threads_ = 0;
+        // an iteration takes some 4 us and 3 ns an element of the largest instance
+        // (64x32x2 15.6 us), or 14 ps an element of a batch that fills the chip
+        // (4096 of 4x32x32 250 us)
+        tiny_iters_ = (uint32_t)std::min(std::max(20000.0 / (4.0 + 3e-3 * (double)most + 1.4e-5 * (double)elements), 1.0),
+                                         4096.0);
         if (tiny_threads_) packable.assign(specs.size(), false);
     }
     // the instances whose nonempty fibers are kept packed
@@ -810,10 +816,10 @@ void Batch::solve_async(size_t iters) {
     partials_valid_ = true;
 }
 
-// launches of 4096 iterations (some 20 ms) at most
+// launches of some 20 ms at most
 void Batch::run_tiny(size_t iters, bool first) {
     while (iters > 0) {
-        const uint32_t n = (uint32_t)std::min<size_t>(iters, 4096);
+        const uint32_t n = (uint32_t)std::min<size_t>(iters, tiny_iters_);
         BNMF_HIP(launch_tiny(psi_, (uint32_t)layouts_.size(), tiny_threads_, tiny_lds_, stream_,
                              reinterpret_cast<const BldInst*>(meta_.as<char>() + (first ? off_desc_first_ : off_desc_)), n));
         iters -= n;

@@ -376,8 +376,9 @@ class Batch {
     DeviceBuffer arena_;
     DeviceBuffer meta_;  // descriptors, work lists, counts
     LivePlan live_;
-    // every instance is tiny: threads and LDS of a block (0: run the passes)
-    uint32_t tiny_threads_ = 0;
+    // every instance is tiny: threads and LDS of a block (0: run the passes),
+    // iterations of a launch
+    uint32_t tiny_threads_ = 0, tiny_iters_ = 1;
     size_t tiny_lds_ = 0;
     mutable HostStage stage_;
     size_t off_desc_first_ = 0, off_desc_ = 0, off_prep_items_ = 0, off_prep_count_ = 0;

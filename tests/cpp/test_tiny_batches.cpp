@@ -52,6 +52,26 @@ int main(int argc, char** argv) {
         CHECK(launches(4, 16, 64, 2048, 10).empty(), "many of few rows");
         CHECK(launches(70, 10, 3, 1, 10).empty(), "not of one tile");
     }
+    if (what == "length") {
+        // at the rates measured on one MI355X: 3.8 us an iteration of 8x10x3, 15.6
+        // of 64x32x2, 250 of 4096 instances of 4096 elements
+        struct Case {
+            uint32_t x, y, z;
+            size_t n;
+            double us;
+        };
+        for (const Case& c : {Case{8, 10, 3, 1, 3.8}, Case{64, 32, 2, 1, 15.6}, Case{64, 32, 2, 4096, 256.0},
+                              Case{16, 32, 8, 40000, 1500.0}}) {
+            const std::vector<uint32_t> l = launches(c.x, c.y, c.z, c.n, 10000);
+            size_t sum = 0;
+            for (uint32_t n : l) {
+                sum += n;
+                CHECK(n * c.us < 50e3, "%zu of %u x %u x %u: a launch of %u iterations", c.n, c.x, c.y, c.z, n);
+            }
+            CHECK(sum == 10000, "%zu iterations", sum);
+            CHECK(l.size() < 10000 * c.us / 5e3 + 2, "%zu launches", l.size());
+        }
+    }
     if (failures) return 1;
     std::printf("tiny batches ok\n");
     return 0;

@@ -58,6 +58,6 @@ def test_server_memory(objects, tmp_path, what):
     _run(objects, tmp_path, "test_server_memory", what)
 
 
-@pytest.mark.parametrize("what", ["route"])
+@pytest.mark.parametrize("what", ["length", "route"])
 def test_tiny_batches(objects, tmp_path, what):
     _run(objects, tmp_path, "test_tiny_batches", what)

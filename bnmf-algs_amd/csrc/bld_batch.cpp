@@ -946,7 +946,10 @@ void Batch::time_pass(int reps, double* pass_ms, double* iter_ms) {
     // (every pass launch of an iteration, each group's on its stream), and
     // reps whole iterations (prep + pass). Each is replayed once to warm up,
     // then timed with events on the batch stream.
+    // A batch of tiny instances runs whole iterations in one launch and has no
+    // pass of its own: both graphs are replaced by such launches.
     auto capture = [&](bool with_prep, hipGraphExec_t* out) {
+        if (tiny_threads_) return;
         hipGraph_t g = nullptr;
         BNMF_HIP(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
         try {
@@ -976,14 +979,22 @@ void Batch::time_pass(int reps, double* pass_ms, double* iter_ms) {
         BNMF_HIP(hipEventCreate(&e0));
         BNMF_HIP(hipEventCreate(&e1));
         BNMF_HIP(hipEventCreate(&e2));
-        enqueue_pass(MODE_SUMS, false);
-        pack_S(false);
-        BNMF_HIP(hipGraphLaunch(gp, stream_));
-        BNMF_HIP(hipGraphLaunch(gi, stream_));
+        auto run = [&](hipGraphExec_t g) {
+            if (tiny_threads_)
+                run_tiny((size_t)reps, false);
+            else
+                BNMF_HIP(hipGraphLaunch(g, stream_));
+        };
+        if (!tiny_threads_) {
+            enqueue_pass(MODE_SUMS, false);
+            pack_S(false);
+        }
+        run(gp);
+        run(gi);
         BNMF_HIP(hipEventRecord(e0, stream_));
-        BNMF_HIP(hipGraphLaunch(gp, stream_));
+        run(gp);
         BNMF_HIP(hipEventRecord(e1, stream_));
-        BNMF_HIP(hipGraphLaunch(gi, stream_));
+        run(gi);
         BNMF_HIP(hipEventRecord(e2, stream_));
         unpack_S();
         BNMF_HIP(hipEventSynchronize(e2));

@@ -219,7 +219,9 @@ bnmf_status bnmf_batch_log_marginal(bnmf_batch* b, double* out);
  * launches) and of one whole iteration (prep + pass), each from a captured
  * graph of `reps` repetitions replayed as solves replay theirs and timed
  * with HIP events on the batch stream. Advances S by 4*reps passes; solve
- * again (from S0) to restore a result. */
+ * again (from S0) to restore a result. A batch whose solves run whole
+ * iterations in one launch (tiny FP64 instances) has no separate pass: both
+ * times are an iteration's. */
 bnmf_status bnmf_batch_time_pass(bnmf_batch* b, int reps, double* pass_ms, double* iter_ms);
 
 /* bld::bld_fact (src/bld/bld_fact.hpp:36-80) of instance idx's current S:

@@ -74,8 +74,8 @@ bool LivePlan::worth(int dtype, const void* X, size_t x, size_t y, double most) 
 //         at 0.40; 8 of 512x512x64 259/282 at 0.45; 2048x2048x64 439/484 at 0.30,
 //         515/485 at 0.35, 911/484 at 0.49
 //   FP64  z <= 24: 100x100x17 26/31 at 0.49, 8 of 384x384x24 175/175
-//         z <= 32: 256x256x32 30/31 at 0.35, 33/31 at 0.40; 4 of 512x512x32
-//         178/186 at 0.45; 1024x1024x32 159/167 at 0.30, 173/171 at 0.35;
+//         z <= 32: 256x256x32 30/31 at 0.35, 33/31 at 0.40; 16 of them 183/188,
+//         4 of 512x512x32 178/186 and 384x384x32 51/52 at 0.45; 1024x1024x32 159/167 at 0.30, 173/171 at 0.35;
 //         2048x2048x32 339/529 at 0.20, 483/546 at 0.25, 565/533 at 0.30
 //         z <= 64: 8 of 200x200x64 129/138 at 0.49; 4 of 512x512x64 263/323 at
 //         0.35, 334/327 at 0.40; 1024x1024x64 280/305 at 0.30, 335/307 at 0.35
@@ -93,7 +93,8 @@ double LivePlan::most_share(int dtype, bool add, size_t x, size_t y, uint32_t z,
     }
     if (add || z <= 24) return 0.5;
     if (xy >= (1u << 20)) return xy < (1u << 21) ? 0.32 : 0.26;
-    return z <= 32 ? 0.4 : xy < (1u << 17) ? 0.5 : 0.38;
+    if (z <= 32) return elements < (1u << 22) ? 0.38 : 0.45;
+    return xy < (1u << 17) ? 0.5 : 0.38;
 }
 
 LivePlan::LivePlan(int dtype, bool add, const std::vector<BldInst>& descs, const std::vector<InstLayout>& lay,

@@ -314,12 +314,12 @@ static void scan_S0(const T* S0, const T* X, size_t xy, size_t z, bool* nonneg, 
     *packable = nn && pk;
 }
 
-void classify(int dtype, bool add, const InstSpec& s, double eps, bool* nonneg, bool* packable) {
+void classify(int dtype, const InstSpec& s, double eps, bool* nonneg, bool* packable) {
     const size_t xy = (size_t)s.x * s.y;
     bool nn = true;
     for (uint32_t k = 0; k < s.z; ++k) nn = nn && s.beta[k] >= 1.0;
     bool pk = nn && xy > 0 && s.z <= kFusedZ && !(dtype == BNMF_F32 && generic_steps()) && eps >= 1e-200 && eps <= 1.0 &&
-              LivePlan::worth(dtype, s.X, s.x, s.y, LivePlan::most_share(dtype, add, s.x, s.y, s.z, SIZE_MAX));
+              LivePlan::worth(dtype, s.X, s.x, s.y, LivePlan::kMostShare);
     for (uint32_t i = 0; i < s.x; ++i) pk = pk && s.alpha[i] >= 1e-6 && s.alpha[i] <= 1e30;
     for (uint32_t k = 0; k < s.z; ++k) pk = pk && s.beta[k] <= 1e30;
     if (nn && s.S0) {
@@ -412,7 +412,7 @@ void Batch::plan(const std::vector<InstSpec>& specs, Extras extras) {
         BNMF_HIP(hipMemcpy(b + L.off_beta, s.beta, (size_t)s.z * 8, hipMemcpyHostToDevice));
         const void* S0 = s.S0;
         bool nn = true, pk = true;
-        classify(dtype, algo_ == BNMF_ALGO_ADD, s, eps, &nn, &pk);
+        classify(dtype, s, eps, &nn, &pk);
         nonneg[n] = nn;
         packable[n] = pk && extras == Extras::kPacked && iters_known_ >= LivePlan::least_iterations(xyz);
         if (S0) {

@@ -241,8 +241,8 @@ hipError_t launch_pass_key(const PassKey& k, int dtype, int psi, int mode, dim3 
 
 // nonneg: S stays >= 0 (S0 >= 0 and beta >= 1). packable: additionally every
 // gradient of its solve is finite, so that a fiber with X_ij = 0 stays exactly
-// zero, and X looks sparse enough (LivePlan). add: for the additive solver.
-void classify(int dtype, bool add, const InstSpec& s, double eps, bool* nonneg, bool* packable);
+// zero, and X looks sparse enough (LivePlan).
+void classify(int dtype, const InstSpec& s, double eps, bool* nonneg, bool* packable);
 
 // Which instances of a batch keep their nonempty fibers packed, and where
 // (live.cpp). Results do not depend on it.
@@ -258,8 +258,10 @@ class LivePlan {
              const std::vector<bool>& candidate, char* scratch, const std::function<void*(size_t, size_t)>& mem = nullptr);
     LivePlan() = default;
     static size_t scratch_bytes(const std::vector<InstLayout>& lay);
-    // Largest share of nonempty fibers at which an instance is packed; elements:
-    // those of its batch. add: the additive solver's step.
+    // Largest share of nonempty fibers at which packing an instance pays, alone or
+    // among its like; elements: those of its batch. add: the additive solver's
+    // step. None is packed above kMostShare.
+    static constexpr double kMostShare = 0.5;
     static double most_share(int dtype, bool add, size_t x, size_t y, uint32_t z, size_t elements);
     // Iterations from which packing an instance of so many elements pays.
     static size_t least_iterations(size_t elements);

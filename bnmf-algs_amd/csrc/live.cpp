@@ -103,12 +103,11 @@ LivePlan::LivePlan(int dtype, bool add, const std::vector<BldInst>& descs, const
     const size_t es = dtype == BNMF_F32 ? 4 : 8;
     size_t elements = 0;
     for (const InstLayout& L : lay) elements += L.elements();
-    auto most_of = [&](const InstLayout& L) { return most_share(dtype, add, L.x, L.y, L.z, elements); };
     // nonempty fibers of every candidate's tiles
     std::vector<PassItem> items;
     for (size_t n = 0; n < descs.size(); ++n) {
         const InstLayout& L = lay[n];
-        if (!candidate[n] || L.elements() == 0 || L.z > kFusedZ || L.ti_rows > kLiveRows || most_of(L) == 0.0) continue;
+        if (!candidate[n] || L.elements() == 0 || L.z > kFusedZ || L.ti_rows > kLiveRows) continue;
         for (uint32_t ti = 0; ti < L.n_ti; ++ti)
             for (uint32_t tj = 0; tj < L.n_tj; ++tj) items.push_back(PassItem{(uint32_t)n, ti, tj, 0});
     }
@@ -122,6 +121,28 @@ LivePlan::LivePlan(int dtype, bool add, const std::vector<BldInst>& descs, const
         BNMF_HIP(launch_live_count(dtype, reinterpret_cast<const BldInst*>(scratch), reinterpret_cast<const PassItem*>(it),
                                    (uint32_t)items.size(), reinterpret_cast<uint32_t*>(ct), nullptr));
         BNMF_HIP(hipMemcpy(counts.data(), ct, items.size() * 4, hipMemcpyDeviceToHost));
+    }
+
+    // Which instances pay, alone or among their like; work of those that do and
+    // those that do not, for each of the two launches (z <= 32, z <= 64). An
+    // instance past its own limit joins the others' launch all the same where
+    // they are the larger part of it: that costs an iteration less than a dense
+    // launch of its own (19 instances of up to 248x292x32, three of them past
+    // their limits: 133 iterations 9.0 against 12.1 ms).
+    std::vector<size_t> pays(descs.size(), 0);
+    size_t work[2][2] = {};
+    for (size_t at = 0; at < items.size();) {
+        const size_t n = items[at].inst;
+        const InstLayout& L = lay[n];
+        const size_t nt = (size_t)L.n_ti * L.n_tj;
+        size_t total = 0;
+        for (size_t t = 0; t < nt; ++t) total += counts[at + t];
+        const double xy = (double)L.x * (double)L.y;
+        if ((double)total <= kMostShare * xy) {
+            pays[n] = (double)total <= most_share(dtype, add, L.x, L.y, L.z, elements) * xy;
+            work[L.z > 32][pays[n]] += total * L.z;
+        }
+        at += nt;
     }
 
     // the packed form is extra memory: an instance without room for it runs the
@@ -145,7 +166,8 @@ LivePlan::LivePlan(int dtype, bool add, const std::vector<BldInst>& descs, const
             slots += (c + gf - 1) / gf * gf;
             most = std::max(most, c);
         }
-        ok = ok && total > 0 && (double)total <= most_of(L) * (double)L.x * (double)L.y && slots < (1ull << 31);
+        ok = ok && total > 0 && (double)total <= kMostShare * (double)L.x * (double)L.y && slots < (1ull << 31);
+        ok = ok && (pays[n] || work[L.z > 32][0] <= work[L.z > 32][1]);
         if (ok) {
             const size_t least = live_lds_need(dtype, L.z, L.tile_cols, L.ti_rows, most, 4);
             const size_t all = live_lds_need(dtype, L.z, L.tile_cols, L.ti_rows, most, (L.z + 3) / 4 * 4);

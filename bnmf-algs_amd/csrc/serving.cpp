@@ -148,7 +148,7 @@ class Server {
         s.S0 = d.S0 ? r->S0.data() : nullptr;
         s.alpha = d.alpha;
         s.beta = d.beta;
-        classify(dtype_, false, s, eps_, &r->nonneg, &r->packable);
+        classify(dtype_, s, eps_, &r->nonneg, &r->packable);
         // packing costs a request as much as some iterations save: sixteen of
         // 512x512x32 at 30 % nonempty 6.0 ms dense and 7.6 packed for 8 iterations,
         // four of 1024x1024x32 8.4 and 8.3 for 24; one of 64x64x8 0.17 and 0.26 ms

@@ -37,3 +37,26 @@ def test_limit(hip, case):
     # eps below 1e-200 is not for the packed form
     assert memory(loses, 1e-50) == memory(loses, 1e-250)
     assert pays is None or memory(pays, 1e-50) > memory(pays, 1e-250)
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_in_company(hip, dt):
+    """An instance past its own limit is packed where those within theirs are the
+    larger part of the launch, and not where it is."""
+    rng = np.random.default_rng(1)
+    lim, z = (0.45, 31) if dt == np.float32 else (0.47, 31)
+
+    def inst(x, y, share, seed):
+        return hip.Instance(X=(rng.random((x, y)) < share).astype(dt), z=z, params=hip.Params(1.0, 1.0, [1.0] * x, [1.0] * z),
+                            seed=seed)
+
+    def memory(insts, eps=1e-50):
+        with hip.Batch(insts, dtype=dt, eps=eps) as b:
+            return b.info()["device_bytes"]
+    past = inst(100, 90, lim, 0)
+    large, small = inst(400, 300, 0.1, 1), inst(60, 50, 0.1, 2)
+    extra = [memory(i) - memory(i, 1e-250) for i in ([past], [large], [small], [past, large], [past, small])]
+    assert extra[0] == 0 and extra[1] > 0 and extra[2] > 0
+    packed_S = 100 * 90 * lim * z * np.dtype(dt).itemsize  # (work lists differ by less)
+    assert extra[3] > extra[1] + packed_S
+    assert extra[4] < extra[2] + packed_S

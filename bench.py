@@ -22,10 +22,13 @@ Also measured (same JSON line):
     headline's 256 instances, with the roofline of its pass;
   * bld_appr_batched_fp32: the sibling approximate solver (bld::bld_appr) on
     the same instances;
-  * roofline of the fused pass kernel of the headline batch (HIP events on
-    the batch stream): algorithmic bytes 2*x*y*z*4 + x*y*4 per launch, beside
-    the rate plain streaming kernels reach on the same GPU (stream_ceiling:
-    bnmf-algs_amd/lib/stream_bw, non-temporal copy of 1 GiB);
+  * roofline of the step pass of the headline batch (HIP events on the batch
+    stream): what an iteration cannot do without, one read and one write of
+    the fibers with X > 0 and one read of those X (pass_bytes), beside the
+    rate plain streaming kernels reach on the same GPU (stream_ceiling:
+    bnmf-algs_amd/lib/stream_bw, non-temporal copy of 1 GiB). Nine tenths of
+    the fibers are empty, most instances keep the others packed, and latency,
+    not bandwidth, bounds the pass;
   * cpu_baseline: the FP64 C++/OpenMP oracle (a port of the reference CPU
     solver, which cannot be built here) on the reference's CPU config
     100x100x17, 1000 iterations, exact digamma.
@@ -83,6 +86,12 @@ def single(hip, x, y, z, a, seed):
 def as_dtype(inst, hip, dt):
     return hip.Instance(X=inst.X.astype(dt), z=inst.z, params=inst.params,
                         S0=inst.S0.astype(dt), seed=inst.seed)
+
+
+def pass_bytes(insts, es):
+    """Bytes one iteration's step pass cannot do without: S of the fibers with
+    X > 0 read and written, and their X read (an empty fiber stays zero)."""
+    return sum(int(np.count_nonzero(i.X)) * (2 * i.z + 1) * es for i in insts)
 
 
 def timed_solves(b, iters, steps, warmup):
@@ -234,23 +243,23 @@ def stream_ceiling():
         return None
 
 
-def measure_add(hip, c3f, elems3, fibers3, iters3):
+def measure_add(hip, c3f, elems3, iters3):
     """bld::bld_add batched FP32 on the headline's instances: solve rate and
-    the roofline of its pass (same algorithmic bytes as bld_mult's)."""
+    the roofline of its pass (same bytes as bld_mult's)."""
     log("[bench] batched FP32 bld_add on the same instances")
     ba = hip.Batch(c3f, dtype=np.float32, algo=hip.ALGO_ADD)
     ta = timed_solves(ba, iters3, 1, 1)
     pa, ia = ba.time_pass(20)
-    alg_bytes = 2 * elems3 * 4 + fibers3 * 4
-    ach_a = alg_bytes / (pa * 1e-3) / 1e9
+    ach_a = pass_bytes(c3f, 4) / (pa * 1e-3) / 1e9
     ba.close()
     log(f"[bench] bld_add FP32: {ta*1e3:.1f} ms/solve, pass {pa*1e3:.1f} us ({ach_a:.0f} GB/s)")
     return {
         "value": elems3 * iters3 / ta, "unit": "S-element updates/s",
         "ms_per_solve": ta * 1e3, "pass_us": pa * 1e3, "iter_us": ia * 1e3,
-        "roofline": {"bound": "hbm", "achieved": ach_a, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+        "roofline": {"bound": "latency", "achieved": ach_a, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": ach_a / HBM_PEAK_GBS,
-                     "kernel": "bld_pass_f32z_kernel additive step, all launches of one iteration"},
+                     "kernel": "additive step: bld_live_f32_kernel (packed fibers) and "
+                               "bld_pass_f32z_kernel (the fuller instances), all launches of one iteration"},
         "workload": "the headline's 256 instances, 200 iterations of bld::bld_add"}
 
 
@@ -276,8 +285,7 @@ def measure_appr(hip, c3f, elems3, iters3):
 
 def measure_c1(hip, iters=500, solves=1, reps=20):
     """One 1024x1024x32 instance in the plain FP64 form (exact digamma):
-    solve time and the graph-timed update pass (algorithmic bytes 2*x*y*z*8
-    + x*y*8 per pass)."""
+    solve time and the graph-timed update pass (packed fibers: pass_bytes)."""
     log(f"[bench] config 1: 1024x1024x32 FP64 exact, {iters} iterations")
     c1 = single(hip, 1024, 1024, 32, 40.0, 0xB1D1)
     b1 = hip.Batch([c1], dtype=np.float64, use_psi_appr=False)
@@ -285,7 +293,7 @@ def measure_c1(hip, iters=500, solves=1, reps=20):
     p1, it1 = b1.time_pass(reps)
     b1.close()
     e1 = 1024 * 1024 * 32
-    alg = 2 * e1 * 8 + 1024 * 1024 * 8
+    alg = pass_bytes([c1], 8)
     res = {"value": e1 * iters / t1, "unit": "S-element updates/s", "ms_per_solve": t1 * 1e3,
            "iterations": iters, "pass_us": p1 * 1e3, "iter_us": it1 * 1e3,
            "pass_GBps": alg / (p1 * 1e-3) / 1e9, "pass_frac_of_peak": alg / (p1 * 1e-3) / 1e9 / HBM_PEAK_GBS,
@@ -331,7 +339,7 @@ def measure_c2(hip, iters=300, reps=20, accuracy=True):
                                "mode": "bnmf_bld_mult_f32 on host X and S0, S returned to the host"}
         del c2f
     e2 = 2048 * 2048 * 64
-    alg = 2 * e2 * 4 + 2048 * 2048 * 4
+    alg = pass_bytes([c2], 4)
     res = {"value": e2 * iters / t2, "unit": "S-element updates/s", "ms_per_solve": t2 * 1e3,
            "iterations": iters, "pass_us": p2 * 1e3, "iter_us": it2 * 1e3,
            "pass_GBps": alg / (p2 * 1e-3) / 1e9, "pass_frac_of_peak": alg / (p2 * 1e-3) / 1e9 / HBM_PEAK_GBS,
@@ -455,7 +463,6 @@ def main():
     c3 = make_c3(hip)
     iters3 = 200
     elems3 = sum(i.X.shape[0] * i.X.shape[1] * i.z for i in c3)
-    fibers3 = sum(i.X.shape[0] * i.X.shape[1] for i in c3)
     c3f = [as_dtype(i, hip, np.float32) for i in c3]
     tuned = None
     if args.tune_file:
@@ -474,8 +481,7 @@ def main():
         if args.save_tune:
             hip.tune_save(args.save_tune)
     if args.add_only:
-        print(json.dumps({"bld_add_batched_fp32": measure_add(hip, c3f, elems3, fibers3, iters3)}),
-              flush=True)
+        print(json.dumps({"bld_add_batched_fp32": measure_add(hip, c3f, elems3, iters3)}), flush=True)
         return
     if args.appr_only:
         print(json.dumps({"bld_appr_batched_fp32": measure_appr(hip, c3f, elems3, iters3)}), flush=True)
@@ -488,7 +494,7 @@ def main():
     lm32 = b32.log_marginal()
     b32.solve(iters3)  # restore S (log_marginal reuses the partial buffers)
     pass_ms, iter_ms = b32.time_pass(50)
-    alg_bytes = 2 * elems3 * 4 + fibers3 * 4
+    alg_bytes = pass_bytes(c3f, 4)
     achieved = alg_bytes / (pass_ms * 1e-3) / 1e9
     info = b32.info()
     log(f"[bench] batched FP32: {t_step*1e3:.2f} ms/solve, {value:.3e} upd/s, "
@@ -534,14 +540,14 @@ def main():
         out["fp64_batched_same_workload"] = {
             "value": elems3 * iters3 / t64b, "unit": "S-element updates/s",
             "ms_per_solve": t64b * 1e3, "pass_us": p64 * 1e3, "iter_us": i64 * 1e3,
-            "pass_GBps": (2 * elems3 * 8 + fibers3 * 8) / (p64 * 1e-3) / 1e9,
+            "pass_GBps": pass_bytes(c3d, 8) / (p64 * 1e-3) / 1e9,
             "dtype": "f64", "digamma": "exact", "mode": "the 256 instances as one batch"}
         out["ratio_vs_fp64_batched"] = value / out["fp64_batched_same_workload"]["value"]
         log(f"[bench] FP64 batch: {t64b*1e3:.1f} ms/solve, pass {p64*1e3:.1f} us")
 
     # ------------------------ sibling solver: bld_add on the same 256 instances
     if not args.only_headline and not args.no_add:
-        out["bld_add_batched_fp32"] = measure_add(hip, c3f, elems3, fibers3, iters3)
+        out["bld_add_batched_fp32"] = measure_add(hip, c3f, elems3, iters3)
 
     # ----------------------- sibling solver: bld_appr on the same 256 instances
     if not args.only_headline and not args.no_appr:
@@ -580,10 +586,11 @@ def main():
                    "instances": len(c3), "elements": elems3, "iterations": iters3,
                    "pass_items": info["pass_items"], "pass_launches": info["n_buckets"],
                    "tile_autotune": tuned, "parallelism": "single GPU"},
-        "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+        "roofline": {"bound": "latency", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
                      "traffic_source": traffic_src,
-                     "kernel": "bld_pass_f32z_kernel (FP32 update), all launches of one iteration",
+                     "kernel": "FP32 update: bld_live_f32_kernel (packed fibers) and bld_pass_f32z_kernel "
+                               "(the fuller instances), all launches of one iteration",
                      "pass_us": pass_ms * 1e3, "iter_us": iter_ms * 1e3,
                      "algorithmic_bytes_per_launch": alg_bytes},
         "cpu_baseline": cpu,

@@ -81,7 +81,10 @@ uint32_t choose_ti_rows(int dtype, uint32_t x, uint32_t y, uint32_t z, bool tall
     // deep fibers: the wide pass's fixed tiles
     if (z > kFusedZ) return kWideRows;
     // Row-tile height depends on the instance shape only (never on the rest
-    // of a batch), so an instance sums in the same order alone or batched.
+    // of a batch), so an instance sums in the same order alone or batched;
+    // except where memory runs out: `tall` (a batch on a full device, a served
+    // request above the server's budget) has tiles with less room for partial
+    // sums and results that differ in the last digits.
     // Tall tiles (up to 128 rows) amortise the tile prologue/epilogue and
     // cut the S_+jk partial traffic to 1/TI of S; an instance with a million
     // fibers or more takes shorter tiles if that is what it needs to give
@@ -102,13 +105,17 @@ uint32_t choose_ti_rows(int dtype, uint32_t x, uint32_t y, uint32_t z, bool tall
                                      : tuned ? tuned : (large ? 128u : 64u);
     uint32_t nt = (x + cap - 1) / cap;
     // A small FP64 instance without a table entry takes tiles of about 5120
-    // elements, of 8 rows at least, up to 1024 tiles: its step is bound by the
-    // arithmetic of each tile's block, and 64-row tiles leave most CUs idle.
-    // Iteration of a lone dense instance at 64 rows and by this rule: 100x100x17
-    // 127 -> 74 us, 384x300x32 180 -> 54, 256x128x64 193 -> 167; with mostly zero
-    // counts 225 -> 49, 98 -> 34 and 136 -> 35. Sixteen at once: 128 -> 75,
-    // 200x200x17 187 -> 163, 256x128x64 279 -> 293 dense and 182 -> 43. FP32 keeps
-    // its heights: its sums in another order move results by up to 1e-5.
+    // elements, of 8 rows at least, up to 1024 tiles: alone, its step is bound by
+    // the arithmetic of each tile's block, and 64-row tiles leave most CUs idle.
+    // Iterations of solves at 64 rows and by this rule, alone and dense: 100x100x17
+    // 104 -> 31 us, 384x300x32 110 -> 38, 256x128x64 114 -> 33; at 5 % nonempty
+    // (packed at both heights) 23 -> 20, 33 -> 25 and 40 -> 25. Sixteen of
+    // 100x100x17 at once 98 -> 55. A dense batch that fills the chip pays for the
+    // short tiles' partial sums: 64 of 100x100x17 126 -> 154, 64 of 200x200x17 415
+    // -> 487, 32 of 384x300x32 519 -> 623, 16 of 256x128x64 159 -> 196; so does a
+    // packed one (29 -> 59, 67 -> 172, 105 -> 262, 52 -> 82), though less than the
+    // dense passes at 64 rows would take (122, 409, 488, 150). FP32 keeps its
+    // heights: its sums in another order move results by up to 1e-5.
     if (dtype == BNMF_F64 && !large && !tall && env_cap <= 0 && tuned == 0) {
         const uint64_t row = (uint64_t)std::min(y, tile_cols_of(dtype, z)) * z;
         const uint32_t rows = (uint32_t)std::max<uint64_t>(5120u / row / 4u * 4u, 8u);

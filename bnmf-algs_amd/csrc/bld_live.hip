@@ -31,8 +31,9 @@
 // step and the partial sums, not bytes; a launch has one block per tile, two
 // to four resident per CU. Measured on one MI355X (kernel trace), one pass of
 // the benchmark's counts: 2048 x 2048 x 64 FP32 32 us against 470 us for the
-// dense pass, 1024 x 1024 x 32 FP64 32 us against 151 us, 100 x 100 x 17 FP64
-// 46 us against 93 us.
+// dense pass, 1024 x 1024 x 32 FP64 29 us against 151 us, 100 x 100 x 17 FP64 with
+// a third of X nonempty (8-row tiles) 12 us against some 19 us. Up to which share
+// it pays: LivePlan::most_share.
 //
 // Reference operations: src/bld/bld_mult/bld_mult_funcs.hpp (X_reciprocal
 // :95, grad_plus :177-192, nom :242-259, denom :272-290, update_S :307-327),

@@ -23,7 +23,8 @@
 // against 19.1, 64x32x2 18.6 against 47.8, 4x16x64 12.8 against 20.9, and with
 // mostly zero counts 12.4 against 15.7 (packed fibers). 256 of 8x32x16 at once 12.1
 // against 23.1, 1024 of them 48 against 55: the line of kTinyElems lies where the
-// gain for full batches ends and the LDS for one block does.
+// gain for full batches ends and the LDS for one block does. Beyond 1024 instances,
+// those of few rows take the passes (Batch::plan).
 //
 // Reference operations: src/bld/bld_mult/bld_mult_funcs.hpp (X_reciprocal :95,
 // alpha_eph :130-141, beta_eph :152-163, grad_plus :177-192, grad_minus

@@ -219,8 +219,9 @@ BldInst make_desc(const InstLayout& L, void* base, double eps, double a, double 
 // Kernel of one pass launch: the exact-z FP32 step kernel (zexact > 0), the
 // FP64 step kernel (f64, z bucket zb, LDS read width rw), the generic
 // z-bucket kernel (zb, rw) or, for z > kFusedZ, the wide kernel (zb = 0).
-// Instances with equal keys share a launch. The key depends on the instance
-// shape only, so an instance runs the same kernel alone, batched or served.
+// Instances with equal keys share a launch. The key follows from the instance's
+// shape, S0 and parameters, so an instance runs the same kernel alone, batched or
+// served, and from whether its nonempty fibers are packed (the same bits).
 struct PassKey {
     int zexact = 0, zb = 0, rw = 0, f64 = 0;  // wide: rw as wide_regs_nk
     int live = 0;  // step over packed nonempty fibers: 1 for z <= 32, 2 for 33 <= z <= 64

@@ -13,7 +13,8 @@
 //    boundary, finished ones leave;
 //  * draws S0 on the device from the same Philox stream as the host init_S
 //    when the request carries none, so only X crosses PCIe.
-// Every instance's tiles and sums are fixed by its own shape, so a result is
+// Every instance's tiles and sums are fixed by its own shape (and, for a request
+// that fits the budget only with tall tiles, by the budget), so a result is
 // bitwise the same whichever requests share the GPU with it.
 
 #include <hip/hip_runtime.h>

@@ -476,7 +476,8 @@ void Batch::plan(const std::vector<InstSpec>& specs, Extras extras) {
     }
     // the instances whose nonempty fibers are kept packed
     if (extras == Extras::kPacked) {
-        live_ = LivePlan(dtype, algo_ == BNMF_ALGO_ADD, d_main, layouts_, packable, arena_.as<char>(off_scratch));
+        live_ = LivePlan(dtype, algo_ == BNMF_ALGO_ADD, d_main, layouts_, packable, arena_.as<char>(off_scratch),
+                         nullptr);
         device_bytes_ += live_.bytes();
     }
     std::vector<PrepItem> prep;

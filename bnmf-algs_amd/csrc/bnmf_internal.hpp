@@ -252,11 +252,13 @@ class LivePlan {
     // Counts the nonempty fibers of the candidates' tiles (X and the tile
     // plan from the descriptors) and lays the packed buffers out.
     // scratch: device memory of scratch_bytes, used until the call returns; it
-    // starts with the descriptors. mem(n, bytes): where the packed buffers of
-    // instance n come from and are given back to (null for none left); without it
-    // they are the plan's own.
+    // starts with the descriptors. st: where X is ready; the counts run there (a
+    // server's own stream, never the null stream, on which results are copied to
+    // callers). mem(n, bytes): where the packed buffers of instance n come from and
+    // are given back to (null for none left); without it they are the plan's own.
     LivePlan(int dtype, bool add, const std::vector<BldInst>& descs, const std::vector<InstLayout>& lay,
-             const std::vector<bool>& candidate, char* scratch, const std::function<void*(size_t, size_t)>& mem = nullptr);
+             const std::vector<bool>& candidate, char* scratch, hipStream_t st,
+             const std::function<void*(size_t, size_t)>& mem = nullptr);
     LivePlan() = default;
     static size_t scratch_bytes(const std::vector<InstLayout>& lay);
     // Largest share of nonempty fibers at which packing an instance pays, alone or

@@ -98,7 +98,8 @@ double LivePlan::most_share(int dtype, bool add, size_t x, size_t y, uint32_t z,
 }
 
 LivePlan::LivePlan(int dtype, bool add, const std::vector<BldInst>& descs, const std::vector<InstLayout>& lay,
-                   const std::vector<bool>& candidate, char* scratch, const std::function<void*(size_t, size_t)>& mem)
+                   const std::vector<bool>& candidate, char* scratch, hipStream_t st,
+                   const std::function<void*(size_t, size_t)>& mem)
     : dtype_(dtype), offs_(descs.size()), fibers_(descs.size(), 0), lds_(descs.size(), 0) {
     const size_t es = dtype == BNMF_F32 ? 4 : 8;
     size_t elements = 0;
@@ -116,11 +117,12 @@ LivePlan::LivePlan(int dtype, bool add, const std::vector<BldInst>& descs, const
     {
         char* const it = scratch + align_up(descs.size() * sizeof(BldInst));
         char* const ct = it + align_up(items.size() * sizeof(PassItem));
-        BNMF_HIP(hipMemcpy(scratch, descs.data(), descs.size() * sizeof(BldInst), hipMemcpyHostToDevice));
-        BNMF_HIP(hipMemcpy(it, items.data(), items.size() * sizeof(PassItem), hipMemcpyHostToDevice));
+        BNMF_HIP(hipMemcpyAsync(scratch, descs.data(), descs.size() * sizeof(BldInst), hipMemcpyHostToDevice, st));
+        BNMF_HIP(hipMemcpyAsync(it, items.data(), items.size() * sizeof(PassItem), hipMemcpyHostToDevice, st));
         BNMF_HIP(launch_live_count(dtype, reinterpret_cast<const BldInst*>(scratch), reinterpret_cast<const PassItem*>(it),
-                                   (uint32_t)items.size(), reinterpret_cast<uint32_t*>(ct), nullptr));
-        BNMF_HIP(hipMemcpy(counts.data(), ct, items.size() * 4, hipMemcpyDeviceToHost));
+                                   (uint32_t)items.size(), reinterpret_cast<uint32_t*>(ct), st));
+        BNMF_HIP(hipMemcpyAsync(counts.data(), ct, items.size() * 4, hipMemcpyDeviceToHost, st));
+        BNMF_HIP(hipStreamSynchronize(st));
     }
 
     // Which instances pay, alone or among their like; work of those that do and
@@ -274,7 +276,7 @@ void LivePlan::build(const std::vector<BldInst>& descs, const BldInst* insts, hi
     const size_t bytes = tiles_.size() * sizeof(LiveTile);
     for (LiveTile& t : tiles_) t.iter = descs[t.inst].iter;
     LiveTile* const dev = tab ? tab : tab_;
-    BNMF_HIP(hipMemcpy(dev, tiles_.data(), bytes, hipMemcpyHostToDevice));
+    BNMF_HIP(hipMemcpyAsync(dev, tiles_.data(), bytes, hipMemcpyHostToDevice, st));
     BNMF_HIP(launch_live_build(dtype_, insts, dev, (uint32_t)tiles_.size(), st));
     if (tab) BNMF_HIP(hipMemcpyAsync(tiles_.data(), dev, bytes, hipMemcpyDeviceToHost, st));
 }

@@ -403,7 +403,7 @@ class Server {
             scratch_.ptr = p;
             scratch_.bytes = need;
         }
-        LivePlan plan(dtype_, false, desc, lay, std::vector<bool>(set.size(), true), scratch_.as<char>(),
+        LivePlan plan(dtype_, false, desc, lay, std::vector<bool>(set.size(), true), scratch_.as<char>(), stream_,
                       [&](size_t n, size_t bytes) -> void* {
                           Request& r = *set[n];
                           bytes = align_up(bytes);

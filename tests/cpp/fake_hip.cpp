@@ -19,14 +19,14 @@ std::map<void*, size_t> blocks;
 size_t used = 0, capacity = ~(size_t)0, fail_at = 0, mallocs = 0, pins = 0;
 bool tiny = false;
 std::vector<uint32_t> tiny_iters;
-std::atomic<size_t> copies{0}, launches{0}, packs{0};
+std::atomic<size_t> copies{0}, launches{0}, packs{0}, on_null{0};
 
 void reset(size_t cap, size_t fail) {
     std::lock_guard<std::mutex> lk(mu);
     capacity = cap;
     fail_at = fail;
     mallocs = pins = 0;
-    copies = launches = packs = 0;
+    copies = launches = packs = on_null = 0;
 }
 size_t in_use() {
     std::lock_guard<std::mutex> lk(mu);
@@ -91,11 +91,13 @@ hipError_t hipHostFree(void* p) {
 }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) {
     ++fake::copies;
+    ++fake::on_null;
     std::memcpy(d, s, n);
     return hipSuccess;
 }
-hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t st) {
     ++fake::copies;
+    fake::on_null += st == nullptr;
     std::memcpy(d, s, n);
     return hipSuccess;
 }
@@ -212,7 +214,8 @@ static uint32_t count_tile(const BldInst& I, const PassItem& it) {
             n += static_cast<const T*>(I.X)[(size_t)i * I.y + j] != T(0);
     return n;
 }
-hipError_t launch_live_count(int dtype, const BldInst* insts, const PassItem* items, uint32_t n, uint32_t* counts, hipStream_t) {
+hipError_t launch_live_count(int dtype, const BldInst* insts, const PassItem* items, uint32_t n, uint32_t* counts, hipStream_t st) {
+    fake::on_null += st == nullptr;
     for (uint32_t t = 0; t < n; ++t) {
         const BldInst& I = insts[items[t].inst];
         counts[t] = dtype == 0 ? count_tile<float>(I, items[t]) : count_tile<double>(I, items[t]);

@@ -15,5 +15,6 @@ size_t n_mallocs();  // since reset
 size_t n_pins();     // hipHostMalloc since reset
 extern bool tiny;                         // whole solves in one launch where the planner wants them
 extern std::vector<uint32_t> tiny_iters;  // iterations of each such launch
-extern std::atomic<size_t> copies, launches, packs;  // packs: launches that pack fibers
+// packs: launches that pack fibers; on_null: copies and counts on the null stream
+extern std::atomic<size_t> copies, launches, packs, on_null;
 }  // namespace fake

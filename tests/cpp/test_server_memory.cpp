@@ -107,6 +107,19 @@ static void small_requests() {
     bnmf_server_destroy(s);
 }
 
+// the scheduler keeps to its own streams: copies of results to callers run on the
+// null stream, and it would wait for them there
+static void own_streams() {
+    Problem p(300, 250, 24, 0.08);
+    bnmf_server* s = nullptr;
+    CHECK(bnmf_server_create(&s, BNMF_F32, 4 * p.bytes(), 0, 1, 1e-50) == BNMF_OK, "create");
+    fake::reset();
+    CHECK(bnmf_server_wait(s, submit(s, p, 100), 30.0) == BNMF_OK, "request");
+    CHECK(fake::packs > 0, "nothing packed");
+    CHECK(fake::on_null == 0, "%zu operations on the null stream", fake::on_null.load());
+    bnmf_server_destroy(s);
+}
+
 // requests of few iterations are not packed, others are
 static void few_iterations() {
     bnmf_server* s = nullptr;
@@ -127,6 +140,7 @@ int main(int argc, char** argv) {
     if (what == "later") later_request();
     if (what == "small") small_requests();
     if (what == "few") few_iterations();
+    if (what == "streams") own_streams();
     if (failures) return 1;
     std::printf("server memory ok\n");
     return 0;

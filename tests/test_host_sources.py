@@ -53,7 +53,7 @@ def test_share_from_a_sample(objects, tmp_path):
     _run(objects, tmp_path, "test_worth")
 
 
-@pytest.mark.parametrize("what", ["few", "full", "later", "small"])
+@pytest.mark.parametrize("what", ["few", "full", "later", "small", "streams"])
 def test_server_memory(objects, tmp_path, what):
     _run(objects, tmp_path, "test_server_memory", what)
 
